@@ -320,10 +320,9 @@ int smoe_hip_set_decode_engine(SmoeMetalCtx* ctx, int engine);
 /* Prefill MoE block (prefill.cpp:308-453) over n_tokens rows [n_tokens x
  * d_model]: per token RMSNorm + router + top-k, then the layer-major expert
  * grouping (token-by-expert permute, grouped expert GEMMs on MFMA, weighted
- * combine into the residual).  Tokens are processed in passes of as many as
- * one permute workgroup holds (736 at 128 experts x top-8); results do not
- * depend on the pass size.  ids_out / weights_out [n_tokens x top_k] are
- * optional.  Optional device outputs of the permute (these require all tokens
+ * combine into the residual).  Tokens are processed in passes of up to 4096
+ * (32768 / top_k if that is less); results do not depend on the pass size.
+ * ids_out / weights_out [n_tokens x top_k] are optional.  Optional device outputs of the permute (these require all tokens
  * in one pass, else SMOE_ERR_SHAPE):
  *   expert_offsets [n_experts+1], sorted_tokens [n_tokens*top_k],
  *   union_ids [n_experts] (first-appearance order, prefill.cpp:55-68),

@@ -14,12 +14,17 @@
 //   k_split_rows   per row: power-of-two scale 2^e with |x| < 2^e and the
 //                  f16 hi/lo planes of x * 2^-e (hi + lo carries 22 bits),
 //                  columns of every 8 in the order 0 2 4 6 1 3 5 7.
-//   k_permute      stable counting sort of the T*k (token, rank) pairs by
-//                  expert (one workgroup), union order by first appearance.
-//   k_grouped_mm   per expert: [pairs x K] x [K x rows] tiles (128 gate +
-//                  128 up rows, or 256 down rows, per block) on MFMA
-//                  v_mfma_f32_16x16x32_f16, weights and activation rows
-//                  streamed through LDS rings.  Weights enter exactly as
+//   k_perm_count, k_perm_scatter  stable counting sort of the T*k (token,
+//                  rank) pairs by expert, one workgroup per segment of pairs,
+//                  and the GEMMs' work list (k_permute: one workgroup, with the
+//                  union order by first appearance, for callers that ask for
+//                  the permute's outputs).
+//   k_grouped_reg  per unit of up to 64 pairs of an expert: [pairs x K] x [K x
+//                  rows] tiles (128 gate + 128 up rows, or 256 down rows, per
+//                  block) on MFMA v_mfma_f32_16x16x32_f16, weights streamed into
+//                  registers, activation rows through LDS (k_grouped_mm, with
+//                  the weights through LDS too, where a row has an odd number
+//                  of groups).  Weights enter exactly as
 //                  (2c - 15)/8 (f16), activations as hi and lo planes (two
 //                  MFMAs into one fp32 accumulator); each 64-column group adds
 //                  s_g * sum, the row scale 8 * 2^e / 15 closes the dot
@@ -28,7 +33,7 @@
 //   k_combine_pairs hidden[t] += sum_r w[t][r] * y[t*k + r] in rank order.
 //
 // Blocks of one expert are mapped to one XCD (block id mod 8), so its token
-// rows stay in that XCD's L2 while the expert's weights stream once.
+// rows stay in that XCD's L2 and its weights are shared there by its passes.
 #include <algorithm>
 #include <type_traits>
 
@@ -468,24 +473,88 @@ void k_split_rows(const float* __restrict__ src, uint32_t rows, uint32_t cols, u
 // table put them all in one: 14.2 -> 11.6 us at 512 tokens of the 30B shape).
 // Union order (first appearance, token-major, prefill.cpp:55-68) ranks the
 // touched experts by their first pair.  ids >= E are skipped and flagged in
-// err (bit 1).  sched (optional, [E + 1]) receives the grouped GEMMs' work
-// order: sched[0] = number of touched experts, then the touched experts by
-// decreasing cost (gm_cost of their pair count), ties by expert id, ranked by
-// one key per expert computed with its total.
+// err (bit 1).  units (optional) receives the grouped GEMMs' work list.
 // ---------------------------------------------------------------------------
 constexpr int PERM_THREADS = 1024;
 
-// relative cost of one (expert, row tile) block of the grouped GEMMs with M
-// pairs: a fixed share per pass of up to 64 pairs plus one per 16-pair m-tile
-__device__ __forceinline__ uint32_t gm_cost(uint32_t M) { return 2u * ((M + 63u) >> 6) + ((M + 15u) >> 4); }
+// The grouped GEMMs' work list: units[0] = the number U of units, units[1] = the
+// most rows of a unit (cap: 64 or 32), units[2 + u] = expert | pass << 16,
+// experts ascending, passes ascending.  An expert's M pairs take as few passes
+// as cap allows, of equal numbers of 16-row tiles.
+__device__ __forceinline__ uint32_t unit_count(uint32_t M, uint32_t cap) { return (M + cap - 1u) / cap; }
+__device__ __forceinline__ uint32_t unit_rows(uint32_t M, uint32_t cap)
+{
+    const uint32_t tiles = (M + 15u) >> 4, n = unit_count(M, cap);
+    return n ? 16u * ((tiles + n - 1u) / n) : 16u;
+}
+
+// One wave: exclusive scans of the E experts' totals s_tot into s_off [E + 1]
+// (pairs) and s_unit [E + 1] (units), eight experts a lane, and the cap.  Units
+// of 32 rows where 64 would leave the list shorter than few_units: the GEMMs'
+// blocks (units x row tiles) would not fill the chip, and a long expert's
+// passes then run side by side.
+__device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, uint32_t few_units, uint32_t* s_off,
+                                           uint32_t* s_unit, uint32_t* s_cap)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t tot[8], u64 = 0, u32 = 0, sum = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t e = 8 * lane + i;
+        tot[i] = e < E ? s_tot[e] : 0u;
+        sum += tot[i];
+        u64 += unit_count(tot[i], 64u);
+        u32 += unit_count(tot[i], 32u);
+    }
+    auto inclusive = [&](uint32_t v) {
+        for (uint32_t dlt = 1; dlt < WAVE; dlt <<= 1) {
+            const uint32_t o = __shfl_up(v, dlt);
+            if (lane >= dlt) v += o;
+        }
+        return v;
+    };
+    const uint32_t i_tot = inclusive(sum), i64 = inclusive(u64), i32 = inclusive(u32);
+    const uint32_t cap = readlane_u32(i64, WAVE - 1) < few_units ? 32u : 64u;
+    uint32_t run = i_tot - sum, urun = cap == 32u ? i32 - u32 : i64 - u64;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t e = 8 * lane + i;
+        if (e <= E) {
+            s_off[e] = run;
+            s_unit[e] = urun;
+        }
+        run += tot[i];
+        urun += unit_count(tot[i], cap);
+    }
+    if (lane == WAVE - 1) {   // (E = 512 is past the last lane's eight)
+        s_off[E] = run;
+        s_unit[E] = urun;
+        *s_cap = cap;
+    }
+}
+
+// a workgroup writes the work list (s_unit, cap: scan_units)
+__device__ __forceinline__ void write_units(const uint32_t* s_unit, uint32_t E, uint32_t cap, uint32_t* units)
+{
+    for (uint32_t e = threadIdx.x; e < E; e += blockDim.x) {
+        const uint32_t u0 = s_unit[e], n = s_unit[e + 1] - u0;
+        for (uint32_t i = 0; i < n; ++i) units[2 + u0 + i] = e | (i << 16);
+    }
+    if (threadIdx.x == 0) {
+        units[0] = s_unit[E];
+        units[1] = cap;
+    }
+}
 
 __global__ __launch_bounds__(PERM_THREADS)
 void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, uint32_t P, uint32_t K, uint32_t E,
                uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs,
                uint32_t* __restrict__ sorted_tokens, float* __restrict__ sorted_w, uint32_t* __restrict__ union_ids,
-               uint32_t* __restrict__ union_size, uint32_t* __restrict__ sched, uint32_t* __restrict__ err)
+               uint32_t* __restrict__ union_size, uint32_t* __restrict__ units, uint32_t few_units,
+               uint32_t* __restrict__ err)
 {
     extern __shared__ uint32_t s_mem[];
+    __shared__ uint32_t s_cap;
     // the count table is [E][C | 1]: the odd row stride puts a chunk's experts,
     // and the chunks one expert's threads read, in different banks
     const uint32_t C = (P + 63) / 64, CS = C | 1u;
@@ -493,7 +562,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
     uint32_t* s_first = s_cnt + CS * E;    // [E]
     uint32_t* s_tot = s_first + E;         // [E]
     uint32_t* s_off = s_tot + E;           // [E + 1]
-    uint32_t* s_key = s_off + E + 1;       // [E] work-order keys
+    uint32_t* s_unit = s_off + E + 1;      // [E + 1]
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     constexpr int NW = PERM_THREADS / WAVE;
 
@@ -554,39 +623,12 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
                 s_cnt[e * CS + c] = run;
                 run += t;
             }
-            if (sg == S - 1) {
-                s_tot[e] = inc;
-                // work-order key: cost, then the lower id first (0: untouched);
-                // the cost of P pairs is at most 6 C, so it fits while C * E
-                // fits the LDS
-                s_key[e] = inc ? gm_cost(inc) * E + (E - 1 - e) : 0u;
-            }
+            if (sg == S - 1) s_tot[e] = inc;
         }
     }
     __syncthreads();
-    // expert offsets: exclusive scan of the totals by wave 0, eight experts a lane
-    if (wv == 0) {
-        uint32_t loc[8], sum = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t e = 8 * lane + i;
-            loc[i] = e < E ? s_tot[e] : 0u;
-            sum += loc[i];
-        }
-        uint32_t inc = sum;
-        for (int dlt = 1; dlt < WAVE; dlt <<= 1) {
-            const uint32_t o = __shfl_up(inc, dlt);
-            if (lane >= dlt) inc += o;
-        }
-        uint32_t run = inc - sum;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t e = 8 * lane + i;
-            if (e <= E) s_off[e] = run;
-            run += loc[i];
-        }
-        if (lane == WAVE - 1) s_off[E] = inc;   // (E = 512 is past the last lane's eight)
-    }
+    // expert offsets and units
+    if (wv == 0) scan_units(s_tot, E, few_units, s_off, s_unit, &s_cap);
     __syncthreads();
     for (uint32_t e = threadIdx.x; e <= E; e += PERM_THREADS) offsets[e] = s_off[e];
     // scatter: rank among equal ids of lower lanes of the same chunk; the
@@ -632,45 +674,133 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
         for (uint32_t e = 0; e < E; ++e) n += s_tot[e] != 0;
         *union_size = n;
     }
-    // GEMM work order: rank of each touched expert by (cost descending, id).  S
-    // threads (a power of two, in one wave) share an expert's comparisons, as in
-    // the prefix above, and sum their counts with shuffles.
-    if (sched) {
-        uint32_t S = 64;
+    if (units) write_units(s_unit, E, s_cap, units);
+}
+
+// ---------------------------------------------------------------------------
+// The permute of long batches, in segments of PERM_SEG_CHUNKS(E) chunks of 64
+// pairs, one workgroup each (k_permute's tables of a whole long batch do not
+// fit one workgroup's LDS, and one CU would take the scatter alone):
+//   k_perm_count    per segment and expert: the number of its pairs;
+//   k_perm_scatter  every workgroup adds up the counts of the segments before
+//                   its own and of all of them, scans the totals into the
+//                   expert offsets, and places its segment's pairs as
+//                   k_permute does.  Workgroup 0 also writes the offsets and
+//                   the grouped GEMMs' work list.
+// ---------------------------------------------------------------------------
+constexpr uint32_t perm_seg_chunks(uint32_t E) { return E <= 256 ? 32u : 16u; }
+
+__global__ __launch_bounds__(PERM_THREADS)
+void k_perm_count(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, uint32_t* __restrict__ seg_cnt,
+                  uint32_t* __restrict__ err)
+{
+    __shared__ uint32_t s_cnt[SMOE_TOPK_MAX_N];
+    for (uint32_t e = threadIdx.x; e < E; e += PERM_THREADS) s_cnt[e] = 0;
+    __syncthreads();
+    const uint32_t len = 64u * perm_seg_chunks(E), p0 = blockIdx.x * len, p1 = min(P, p0 + len);
+    for (uint32_t p = p0 + threadIdx.x; p < p1; p += PERM_THREADS) {
+        const uint32_t e = ids[p];
+        if (e < E) atomicAdd(&s_cnt[e], 1u);
+        else atomicOr(err, 2u);
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < E; e += PERM_THREADS)
+        seg_cnt[static_cast<size_t>(blockIdx.x) * E + e] = s_cnt[e];
+}
+
+__global__ __launch_bounds__(PERM_THREADS)
+void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, const uint32_t* __restrict__ seg_cnt,
+                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs, uint32_t* __restrict__ units,
+                    uint32_t few_units)
+{
+    extern __shared__ uint32_t s_mem[];
+    __shared__ uint32_t s_cap;
+    const uint32_t CH = perm_seg_chunks(E), CS = CH | 1u;
+    uint32_t* s_cnt = s_mem;               // [E x CS]
+    uint32_t* s_base = s_cnt + E * CS;     // [E] pairs of the expert in earlier segments
+    uint32_t* s_tot = s_base + E;          // [E]
+    uint32_t* s_off = s_tot + E;           // [E + 1]
+    uint32_t* s_unit = s_off + E + 1;      // [E + 1]
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    constexpr uint32_t NW = PERM_THREADS / WAVE;
+    const uint32_t seg = blockIdx.x, nseg = gridDim.x;
+    for (uint32_t i = threadIdx.x; i < E * CS; i += PERM_THREADS) s_cnt[i] = 0;
+    uint32_t eid[2];                       // this wave's chunks wv and wv + NW of the segment
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        const uint32_t c = wv + k * NW, p = (seg * CH + c) * 64 + lane;
+        eid[k] = c < CH && p < P ? ids[p] : 0xFFFFFFFFu;
+    }
+    for (uint32_t e = threadIdx.x; e < E; e += PERM_THREADS) {
+        uint32_t before = 0, tot = 0;
+#pragma unroll 8
+        for (uint32_t s = 0; s < nseg; ++s) {
+            const uint32_t n = seg_cnt[static_cast<size_t>(s) * E + e];
+            tot += n;
+            before += s < seg ? n : 0u;
+        }
+        s_base[e] = before;
+        s_tot[e] = tot;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k)
+        if (eid[k] < E) atomicAdd(&s_cnt[eid[k] * CS + wv + k * NW], 1u);
+    if (wv == 0) scan_units(s_tot, E, few_units, s_off, s_unit, &s_cap);
+    __syncthreads();
+    // counts -> exclusive prefix over the segment's chunks; S threads (a power
+    // of two, in one wave) share an expert's chunks
+    {
+        uint32_t S = CH;
         while (S > 1 && E * S > PERM_THREADS) S >>= 1;
         const uint32_t e = threadIdx.x / S, sg = threadIdx.x % S;
-        uint32_t r = 0, n = 0, ke = 0;
+        const uint32_t Lc = CH / S, c0 = sg * Lc;
+        uint32_t sum = 0;
+        if (e < E)
+            for (uint32_t c = c0; c < c0 + Lc; ++c) sum += s_cnt[e * CS + c];
+        uint32_t inc = sum;
+        for (uint32_t dlt = 1; dlt < S; dlt <<= 1) {
+            const uint32_t o = __shfl_up(inc, dlt, S);
+            if (sg >= dlt) inc += o;
+        }
         if (e < E) {
-            ke = s_key[e];
-            for (uint32_t e2 = sg; e2 < E; e2 += S) {
-                const uint32_t k2 = s_key[e2];
-                n += k2 != 0;
-                r += k2 > ke;
+            uint32_t run = s_off[e] + s_base[e] + inc - sum;
+            for (uint32_t c = c0; c < c0 + Lc; ++c) {
+                const uint32_t t = s_cnt[e * CS + c];
+                s_cnt[e * CS + c] = run;
+                run += t;
             }
         }
-        for (uint32_t dlt = 1; dlt < S; dlt <<= 1) {
-            r += __shfl_xor(r, dlt, S);
-            n += __shfl_xor(n, dlt, S);
+    }
+    __syncthreads();
+    uint32_t nbits = 1;
+    while ((1u << nbits) < E) ++nbits;
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        const uint32_t c = wv + k * NW, e = eid[k];
+        const bool ok = e < E;
+        uint64_t same = __ballot(ok);
+        for (uint32_t b = 0; b < nbits; ++b) {
+            const bool bit = (e >> b) & 1u;
+            const uint64_t set = __ballot(ok && bit);
+            same &= bit ? set : ~set;
         }
-        if (e < E && sg == 0) {
-            if (ke != 0) sched[1 + r] = e;
-            if (e == 0) sched[0] = n;
-        }
+        const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
+        if (ok) sorted_pairs[s_cnt[e * CS + c] + rank] = (seg * CH + c) * 64 + lane;
+    }
+    if (seg == 0) {
+        for (uint32_t e = threadIdx.x; e <= E; e += PERM_THREADS) offsets[e] = s_off[e];
+        write_units(s_unit, E, s_cap, units);
     }
 }
 
 // ---------------------------------------------------------------------------
-// k_grouped_mm: for each expert e with M = offsets[e+1] - offsets[e] pairs,
+// k_grouped_mm: for each unit (a pass of up to 64 pairs of an expert),
 // out[pair][n] for one tile of its weight matrix: 128 rows of gate and of up
 // (gate+up, SiLU fused) or 256 rows of down.  Block = 8 waves; wave w owns two
 // 16-row MFMA subtiles (gate and up rows 16w.., or down rows 32w.. and
-// 32w + 16..) and all m-tiles of the pass (up to 64 pairs, so each weight is
-// read once per expert for M <= 64).  Block b works on the schedule's rank
-// r = 8 s + x (s even) or 8 s + 7 - x (s odd) for x = b mod 8 (its XCD under
-// the round-robin deal) and slot s = (b / 8) / n_tiles, tile (b / 8) mod
-// n_tiles: every tile of an expert runs on one XCD (the activation rows stay
-// in its L2), and the experts, dealt in decreasing cost down and up the XCDs,
-// leave every XCD about the same work whatever the routing.
+// 32w + 16..) and all m-tiles of the pass.  Serves rows with an odd number of
+// groups and weights that are not 16-byte aligned; others take k_grouped_reg.
 //
 // The k dimension streams through two rings in LDS, filled by direct
 // global->LDS loads (global_load_lds_dwordx4) so that nothing in flight holds
@@ -760,7 +890,7 @@ __device__ __forceinline__ void gm_barrier()
 
 template <bool GATE_UP, int MS>
 __device__ __forceinline__ void grouped_mm_expert(
-    const MoeDims& d, const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t M,
+    const MoeDims& d, const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t mb, uint32_t M,
     const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi, const uint16_t* __restrict__ a_lo,
     const float* __restrict__ a_scale, uint32_t a_row_div, float* __restrict__ out, uint32_t n_dim, uint32_t k_dim,
     GmW& w0, GmW& w1, GmW& w2, GmW& w3, GmA& a0, GmA& a1, GmA& a2, GmA& a3, uint32_t (&s_row)[GM_PASS],
@@ -814,7 +944,7 @@ __device__ __forceinline__ void grouped_mm_expert(
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl) aoff[stp][pl] = m16 * 256 + 16 * ((8 * pl + 2 * q + stp) ^ m16);
 
-    for (uint32_t m0 = 0; m0 < M; m0 += PASS) {
+    for (uint32_t m0 = mb; m0 < M; m0 += PASS) {
         __syncthreads();
         if (threadIdx.x < PASS) {
             const uint32_t p = sorted_pairs[base + min(m0 + threadIdx.x, M - 1)];
@@ -935,10 +1065,33 @@ __device__ __forceinline__ void grouped_mm_expert(
     }
 }
 
+// block b of a grid over units x n_tiles -> unit and tile: XCD b mod 8 (the
+// round-robin deal) takes a contiguous eighth of the list, tile by tile of a
+// unit, so an expert's blocks run together on one XCD, sharing its activation
+// rows and, between its passes, its weights in the L2.
+__device__ __forceinline__ bool unit_of_block(const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ units,
+                                              uint32_t n_tiles, uint32_t& e, uint32_t& tile, uint32_t& base,
+                                              uint32_t& mb, uint32_t& me, uint32_t& rows)
+{
+    const uint32_t U = units[0], cap = units[1], per = (U + 7u) >> 3;
+    const uint32_t b = blockIdx.x, xcd = b & 7u, jb = b >> 3;
+    const uint32_t j = jb / n_tiles, u = xcd * per + j;
+    tile = jb % n_tiles;
+    if (j >= per || u >= U) return false;
+    const uint32_t word = units[2 + u], pass = word >> 16;
+    e = word & 0xFFFFu;
+    base = offsets[e];
+    const uint32_t M = offsets[e + 1] - base;
+    rows = unit_rows(M, cap);
+    mb = pass * rows;
+    me = min(M, mb + rows);
+    return true;
+}
+
 template <bool GATE_UP>
 __global__ __launch_bounds__(GM_WAVES * WAVE, 1)
 void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
-                  const uint32_t* __restrict__ sched, const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
+                  const uint32_t* __restrict__ units, const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
                   const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale, uint32_t a_row_div,
                   float* __restrict__ out, uint32_t n_dim, uint32_t k_dim, uint32_t n_tiles)
 {
@@ -946,124 +1099,162 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
     __shared__ __align__(16) GmA a0, a1, a2, a3;
     __shared__ uint32_t s_row[GM_PASS];
     __shared__ uint32_t s_pair[GM_PASS];
-    const uint32_t b = blockIdx.x, xcd = b & 7u, jb = b >> 3;
-    const uint32_t slot = jb / n_tiles, tile = jb % n_tiles;
-    const uint32_t r = 8u * slot + ((slot & 1u) ? 7u - xcd : xcd);
-    if (r >= sched[0]) return;
-    const uint32_t e = sched[1 + r];
-    if (e >= d.E) return;
-    const uint32_t base = offsets[e], M = offsets[e + 1] - base;
-    if (M == 0) return;
-    if (M <= 16)
-        grouped_mm_expert<GATE_UP, 1>(d, L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, a_row_div, out,
-                                      n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3, s_row, s_pair);
-    else if (M <= 32)
-        grouped_mm_expert<GATE_UP, 2>(d, L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, a_row_div, out,
-                                      n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3, s_row, s_pair);
-    else if (M <= 48)
-        grouped_mm_expert<GATE_UP, 3>(d, L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, a_row_div, out,
-                                      n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3, s_row, s_pair);
-    else
-        grouped_mm_expert<GATE_UP, 4>(d, L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, a_row_div, out,
-                                      n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3, s_row, s_pair);
+    uint32_t e, tile, base, mb, me, rows;
+    if (!unit_of_block(offsets, units, n_tiles, e, tile, base, mb, me, rows)) return;
+    auto go = [&](auto ms) {
+        grouped_mm_expert<GATE_UP, decltype(ms)::value>(d, L, e, tile, base, mb, me, sorted_pairs, a_hi, a_lo, a_scale,
+                                                        a_row_div, out, n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3,
+                                                        s_row, s_pair);
+    };
+    if (rows == 16) go(std::integral_constant<int, 1>{});
+    else if (rows == 32) go(std::integral_constant<int, 2>{});
+    else if (rows == 48) go(std::integral_constant<int, 3>{});
+    else go(std::integral_constant<int, 4>{});
 }
 
 // ---------------------------------------------------------------------------
-// k_grouped_down: the down products of k_grouped_mm<false> (same pairs, same
-// sums per 64-column group, same epilogue) with the weights streamed into
-// registers: each weight row belongs to one wave, so plain loads need neither
-// LDS nor a barrier for them.  Blocks of 4 waves x 64 rows (four 16-row
-// subtiles a wave), two blocks per CU: every activation fragment read from LDS
-// feeds four subtiles (half the LDS reads per weight of the 8 x 32-row block),
-// and the two blocks of a CU pass their barriers independently, so one block's
-// MFMAs overlap the other's conversion.  Needs an even number of groups (a
-// stage's two scales are one dword).  30B layer, 512 tokens: 58.9 us against
-// 72 for k_grouped_mm<false> (bench.py --workload prefill).
-//   weights  per wave and stage (two groups: 64 bytes of every row), subtile
-//            j: lane l loads row l & 15, bytes 16 (l >> 4) .. + 15; one
-//            v_permlane32_swap per two dwords then leaves every lane one dword
-//            of each (group, MFMA step): quad q, step s of either group holds
-//            its 8-column unit 4 (q & 1) + 2 (q >> 1) + s, and the activation
-//            fragments are read from those units;
-//   acts     the ring of k_grouped_mm (f16 hi/lo planes, XOR-swizzled 16-byte
-//            slots), filled by direct loads issued from inline asm: the
-//            compiler does not track them, so it adds no waits of its own for
-//            the ring (it would drain every load in flight once per unrolled
-//            iteration); the explicit vmcnt waits cover them.
+// grouped_reg: the grouped products with the weights streamed into registers:
+// each weight row belongs to one wave, so plain loads need neither LDS nor a
+// barrier for them.  Blocks of 4 waves x 64 weight rows (four 16-row subtiles
+// a wave; gate/up: 32 gate rows and the same 32 up rows), two blocks per CU:
+// every activation fragment read from LDS feeds four subtiles, and the two
+// blocks of a CU pass their barriers independently, so one block's MFMAs
+// overlap the other's conversion.  Needs an even number of groups (a stage's
+// two scales are one dword).
+//   stage    two 64-column groups; while one is computed the next one's
+//            weights are on their way into registers and its activation rows
+//            into the other LDS buffer, one wait and one barrier per stage;
+//   weights  subtile j: lane l loads row l & 15, bytes 16 (l >> 4) .. + 15 of
+//            the stage's 64; v_permlane16_swap and v_permlane32_swap then
+//            leave quad q = l >> 4, MFMA step s the 8-column unit 2 q + s of
+//            either group, as in k_grouped_mm;
+//   acts     [plane][row][16 units of 8 columns], unit x of row r in slot
+//            x ^ (r & 15): conflict-free for the fragment reads (units 2 q + s
+//            of rows 0 .. 15), filled by direct loads (4 rows x 256 bytes each)
+//            issued from inline asm: the compiler does not track them, so it
+//            adds no waits of its own;
+//   scales   one load of eight groups of the wave's rows instead of a load per
+//            row and stage, passed across the wave (ds_bpermute).
+//   MFMA     the four products of a group (hi and lo of two steps) accumulate
+//            in one register set per subtile; the four subtiles' chains run
+//            interleaved, the next m-tile's fragments are read during them, and
+//            the sums are scaled into the accumulators during the next
+//            m-tile's chains.
+// Up to two m-tiles a pass (HBM-bound: few pairs per weight byte) a stage is
+// two such steps, so a CU has 64 KB of weights in flight; with more m-tiles
+// LDS and registers hold one.  Measured against the kernels before it (weights
+// of gate/up through LDS, 8 waves and one block per CU; passes of at most 736
+// tokens): 4096 tokens of the 30B shape gate/up 700 -> 407 us (1.05 PFLOP/s
+// of f16 products; a library f16 GEMM reaches 1.19 on the same card), down 407
+// -> 243; 512 tokens gate/up 97 -> 88, down 54 -> 51; 64 tokens of the 235B
+// shape gate/up 248 -> 195 (4.4 TB/s), down 125 -> 113.  Three blocks per CU with 168
+// registers: no faster (spills).
 // ---------------------------------------------------------------------------
 constexpr int GD_WAVES = 4;
 constexpr int GD_SUB = 4;                                  // 16-row subtiles a wave
-constexpr uint32_t GD_ROWS = 16 * GD_SUB * GD_WAVES;       // down rows per block
+constexpr uint32_t GD_ROWS = 16 * GD_SUB * GD_WAVES;       // weight rows per block
+constexpr uint32_t GD_STAGE = GM_PASS * 512;               // bytes of an activation stage of 64 rows
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p)
 {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
 }
-// lane l's 16 bytes land at LDS byte address lds + 16 l
-__device__ __forceinline__ void dma16(const void* g, uint32_t lds)
+// a resource over `bytes` of weights at p (wave-uniform): loads past it return 0
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const void* p, uint32_t bytes)
 {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds) : "memory", "m0");
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
+}
+// lane l's 16 bytes at base + off (off per lane) land at LDS byte address lds + 16 l
+__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
 }
 
-template <int MS>
-__device__ __forceinline__ void grouped_down_expert(
-    const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t M, const uint32_t* __restrict__ sorted_pairs,
-    const uint16_t* __restrict__ a_hi, const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale,
-    float* __restrict__ out, uint32_t n_dim, uint32_t k_dim, GmA& a0, GmA& a1, GmA& a2, GmA& a3,
-    uint32_t (&s_row)[GM_PASS], uint32_t (&s_pair)[GM_PASS])
+// Pairs [mb, me) of expert e (passes of 16 MS), one tile of GD_ROWS weight rows.
+template <bool GATE_UP, int MS>
+__device__ __forceinline__ void grouped_reg_expert(
+    const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t mb, uint32_t me,
+    const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi, const uint16_t* __restrict__ a_lo,
+    const float* __restrict__ a_scale, uint32_t a_row_div, float* __restrict__ out, uint32_t n_dim, uint32_t k_dim,
+    uint8_t* abuf, uint32_t (&s_row)[GM_PASS], uint32_t (&s_pair)[GM_PASS])
 {
-    constexpr int AN = MS;                       // activation loads per wave and stage (4 rows each)
     constexpr int PASS = 16 * MS;
-    constexpr int WS = 2 * GD_SUB;               // loads per weight stage (codes, scales)
+    constexpr int NH = MS <= 2 ? 2 : 1;          // pairs of groups in a stage
+    constexpr uint32_t PLANE = PASS * 256, HALF = 2 * PLANE, STAGE = NH * HALF;
+    static_assert(STAGE <= GD_STAGE, "a stage fits its buffer");
     const int lane = threadIdx.x & 63;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t G = k_dim >> 6, NWS = G / 2;
+    const uint32_t G = k_dim >> 6, NHS = G / 2, NST = (NHS + NH - 1) / NH;
     const uint32_t m16 = lane & 15, q = lane >> 4;
 
+    // codes and scales through buffer resources: a scalar base and one offset
+    // register a subtile (64-bit addresses took 16 registers more and spilled)
     const uint8_t* blob = L.experts + static_cast<size_t>(e) * L.stride;
-    const size_t row_bytes = k_dim >> 1;
-    const uint8_t* w_src[GD_SUB];
-    const uint32_t* s_src[GD_SUB];
+    constexpr int NM = GATE_UP ? 2 : 1, SM = GD_SUB / NM;   // matrices, subtiles of each
+    __amdgpu_buffer_rsrc_t w_mat[NM], s_mat[NM];
 #pragma unroll
-    for (int j = 0; j < GD_SUB; ++j) {
-        const uint32_t r = min(tile * GD_ROWS + 16 * GD_SUB * wv + 16 * j + m16, n_dim - 1);
-        w_src[j] = blob + L.off[4] + static_cast<size_t>(r) * row_bytes + 16 * q;
-        s_src[j] = reinterpret_cast<const uint32_t*>(blob + L.off[5] + static_cast<size_t>(r) * G * 2);
+    for (int i = 0; i < NM; ++i) {
+        const int o = GATE_UP ? 2 * i : 4;
+        w_mat[i] = weight_rsrc(blob + L.off[o], n_dim * (k_dim >> 1));
+        s_mat[i] = weight_rsrc(blob + L.off[o + 1], n_dim * G * 2);
     }
-    uint4 wr[4][GD_SUB];                         // weight ring: [stage slot][subtile]
-    uint32_t sr[4][GD_SUB];                      // the stage's two fp16 scales per subtile
-    auto issue_w = [&](int slot, uint32_t st) {
+    // gate/up: subtiles 0, 1 are 32 gate rows, 2, 3 the same rows of up
+    const uint32_t row_w = tile * (GD_ROWS / NM) + 16 * SM * wv;
+    uint32_t w_off[SM];
 #pragma unroll
-        for (int j = 0; j < GD_SUB; ++j) wr[slot][j] = *reinterpret_cast<const uint4*>(w_src[j] + 64 * st);
+    for (int j = 0; j < SM; ++j) w_off[j] = min(row_w + 16 * j + m16, n_dim - 1) * (k_dim >> 1) + 16 * q;
+    // scales: lane l loads eight groups of the wave's row l (% 32) at once
+    // (every load instruction costs the CU a request slot whatever its width:
+    // one load per four pairs of groups instead of four per pair); the lanes
+    // that use them fetch them across the wave
+    const uint32_t s_off = min(row_w + (lane & (16 * SM - 1)), n_dim - 1) * G * 2;
+    u32x4_t wr[NH][GD_SUB];                      // the next stage's codes
+    u32x4_t sc_next[NM], sc_cur[NM];             // scales of eight groups: the next ones, the current ones
+    auto issue_w = [&](uint32_t st) {
 #pragma unroll
-        for (int j = 0; j < GD_SUB; ++j) sr[slot][j] = s_src[j][st];
+        for (int j = 0; j < GD_SUB; ++j)
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+                wr[h][j] = __builtin_amdgcn_raw_buffer_load_b128(w_mat[j / SM], w_off[j % SM],
+                                                                 64 * min(NH * st + h, NHS - 1), 0);
     };
+    auto issue_s = [&](uint32_t piece) {
+#pragma unroll
+        for (int i = 0; i < NM; ++i) sc_next[i] = __builtin_amdgcn_raw_buffer_load_b128(s_mat[i], s_off, 16 * piece, 0);
+    };
+    // fragment of group g, step s of this lane: 16 bytes at aoff[g][s] (m-tile ms: + 4096 ms; lo plane: + PLANE)
     uint32_t aoff[2][2];
-    const uint32_t u8 = 4 * (q & 1) + 2 * (q >> 1);
 #pragma unroll
-    for (int stp = 0; stp < 2; ++stp)
+    for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int pl = 0; pl < 2; ++pl) aoff[stp][pl] = m16 * 256 + 16 * ((8 * pl + u8 + stp) ^ m16);
+        for (int stp = 0; stp < 2; ++stp) aoff[g][stp] = m16 * 256 + 16 * ((8 * g + 2 * q + stp) ^ m16);
 
-    for (uint32_t m0 = 0; m0 < M; m0 += PASS) {
+    for (uint32_t m0 = mb; m0 < me; m0 += PASS) {
         __syncthreads();
         if (threadIdx.x < PASS) {
-            const uint32_t p = sorted_pairs[base + min(m0 + threadIdx.x, M - 1)];
+            const uint32_t p = sorted_pairs[base + min(m0 + threadIdx.x, me - 1)];
             s_pair[threadIdx.x] = p;
-            s_row[threadIdx.x] = p;
+            s_row[threadIdx.x] = GATE_UP ? p / a_row_div : p;
         }
         __syncthreads();
-        const uint16_t* a_src[AN];
+        // activation fill: waves 0, 1 the hi plane, 2, 3 the lo plane, 2 MS loads of 4 rows each
+        const uint16_t* plane = wv >= 2 ? a_lo : a_hi;
+        const uint32_t row0 = (wv & 1) * 8 * MS;
+        uint32_t a_off[2 * MS];
 #pragma unroll
-        for (int u = 0; u < AN; ++u) {
-            const uint32_t r = wv * 4 * AN + 4 * u + (lane >> 4);
-            const uint32_t x = (lane & 15) ^ (r & 15);
-            const uint32_t srow = s_row[min(r, static_cast<uint32_t>(PASS - 1))];
-            a_src[u] = ((x >> 3) ? a_lo : a_hi) + static_cast<size_t>(srow) * k_dim + 8 * (x & 7);
+        for (int u = 0; u < 2 * MS; ++u) {
+            const uint32_t r = row0 + 4 * u + q;
+            a_off[u] = (s_row[r] * k_dim + 8 * (m16 ^ (r & 15))) * 2;
         }
-        auto issue_a = [&](GmA& S, uint32_t c) {
+        const uint32_t a_dst = lds_addr(abuf) + (wv >> 1) * PLANE + row0 * 256;
+        auto issue_a = [&](uint32_t buf, uint32_t st) {
 #pragma unroll
-            for (int u = 0; u < AN; ++u) dma16(a_src[u] + c * 64, lds_addr(&S.a[(wv * 4 * AN + 4 * u) * 256]));
+            for (int h = 0; h < NH; ++h) {
+                const uint8_t* src = reinterpret_cast<const uint8_t*>(plane) + 256 * min(NH * st + h, NHS - 1);
+#pragma unroll
+                for (int u = 0; u < 2 * MS; ++u) dma16(src, a_off[u], a_dst + buf * STAGE + h * HALF + u * 1024);
+            }
         };
 
         f32x4_t acc[MS][GD_SUB];
@@ -1072,135 +1263,152 @@ __device__ __forceinline__ void grouped_down_expert(
 #pragma unroll
             for (int j = 0; j < GD_SUB; ++j) acc[ms][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-        // body c issues the activation stage c + 3 and then (even c) the weight
-        // stage c / 2 + 3; the prologue replays bodies -6 .. -1
-        if (0 < NWS) issue_w(0, 0);
-        if (1 < NWS) issue_w(1, 1);
-        issue_a(a0, 0);
-        if (1 < G) issue_a(a1, 1);
-        if (2 < NWS) issue_w(2, 2);
-        if (2 < G) issue_a(a2, 2);
+        issue_s(0);
+        issue_w(0);
+        issue_a(0, 0);
         mem_fence_compiler();
 
-        uint32_t gw[GD_SUB][2][2];               // [subtile][group of the stage][MFMA step]
-        auto body = [&](uint32_t c, int slot, int g, int nslot, GmA& A, GmA& AN_) {
-            // After A(c) (first load of body c - 3) came: the weight stage of body c - 3
-            // when c - 3 is even, A(c + 1), A(c + 2) and the weight stage of the even one
-            // of bodies c - 2, c - 1.  When all of those were issued, 2 AN + WS (even c)
-            // or 2 AN + 2 WS (odd c) loads may still be pending; near the end fewer
-            // were, and the wait covers everything.  A(c) done also means the weight
-            // stage c / 2 is: it was issued in body c - 6, before A(c).
-            if (c + 2 < G && (c + 4 + (c & 1)) / 2 < NWS) {
-                if (g) vm_wait<2 * AN + 2 * WS>();
-                else vm_wait<2 * AN + WS>();
-            } else {
-                vm_wait<0>();
-            }
+        for (uint32_t st = 0; st < NST; ++st) {
+            const uint32_t buf = st & 1;
+            vm_wait<0>();
             gm_barrier();
-            if (c + 3 < G) issue_a(AN_, c + 3);
-            if (g == 0 && c / 2 + 3 < NWS) issue_w(nslot, c / 2 + 3);
-            mem_fence_compiler();
-            if (g == 0) {
+            uint32_t gw[NH][GD_SUB][2][2];       // [pair of groups][subtile][group][MFMA step]
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
 #pragma unroll
                 for (int j = 0; j < GD_SUB; ++j)
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
-                        // lanes 0-31 hold the stage's group 0 (bytes 0-31 of the 64), lanes
-                        // 32-63 group 1: swap dwords 2 + s of the lower half with dwords s
-                        // of the upper half
-                        const uint32_t lo = s ? wr[slot][j].y : wr[slot][j].x;
-                        const uint32_t hi = s ? wr[slot][j].w : wr[slot][j].z;
-                        const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
-                        gw[j][0][s] = r[0];
-                        gw[j][1][s] = r[1];
+                        const auto x = __builtin_amdgcn_permlane16_swap(wr[h][j][s], wr[h][j][2 + s], false, false);
+                        const auto r = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
+                        gw[h][j][0][s] = r[0];
+                        gw[h][j][1][s] = r[1];
                     }
+            // (the last stage requests itself again, into the other buffer)
+            const uint32_t nx = min(st + 1, NST - 1);
+            if ((NH * st) % 4 == 0) {
+#pragma unroll
+                for (int i = 0; i < NM; ++i) sc_cur[i] = sc_next[i];
+                issue_s(min((NH * st) / 4 + 1, (NHS - 1) / 4));
             }
-            half8_t b[GD_SUB][2];
-            float sc[GD_SUB];
+            issue_w(nx);
+            issue_a(buf ^ 1u, nx);
+            mem_fence_compiler();
 #pragma unroll
-            for (int j = 0; j < GD_SUB; ++j) {
-                b[j][0] = q4_codes_to_f16(gw[j][g][0]);
-                b[j][1] = q4_codes_to_f16(gw[j][g][1]);
-                sc[j] = f16_bits_to_f32(static_cast<uint16_t>(g ? sr[slot][j] >> 16 : sr[slot][j]));
-            }
+            for (int h = 0; h < NH; ++h) {
+                if (NH > 1 && h > 0 && NH * st + h >= NHS) break;
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t sc2[GD_SUB];            // the two groups' fp16 scales
 #pragma unroll
-            for (int ms = 0; ms < MS; ++ms) {
-                half8_t xa[2][2];
+                for (int j = 0; j < GD_SUB; ++j)
+                    sc2[j] = __builtin_amdgcn_ds_bpermute(4 * (16 * (j % SM) + m16), sc_cur[j / SM][0]);
 #pragma unroll
-                for (int stp = 0; stp < 2; ++stp)
+                for (int i = 0; i < NM; ++i) {
+                    sc_cur[i][0] = sc_cur[i][1];
+                    sc_cur[i][1] = sc_cur[i][2];
+                    sc_cur[i][2] = sc_cur[i][3];
+                }
+                const uint8_t* A = abuf + buf * STAGE + h * HALF;
+                // fragment c (step c / 2, plane c & 1) of m-tile k % MS of group k / MS
+                half8_t xa[4];
+                auto load_a = [&](int k, int c) {
+                    xa[c] = lds_half8(A + (c & 1) * PLANE + (k % MS) * 4096 + aoff[k / MS][c >> 1]);
+                };
+                // The sched_barriers pin the order (left to itself the compiler reads
+                // each fragment right before its use and runs the chains one after
+                // the other, waiting out every latency).
 #pragma unroll
-                    for (int pl = 0; pl < 2; ++pl) xa[stp][pl] = lds_half8(A.a + ms * 4096 + aoff[stp][pl]);
+                for (int c = 0; c < 4; ++c) load_a(0, c);
 #pragma unroll
-                for (int j = 0; j < GD_SUB; ++j) {
-                    f32x4_t t = {0.f, 0.f, 0.f, 0.f};
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][0], b[j][0], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][1], b[j][0], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][0], b[j][1], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][1], b[j][1], t, 0, 0, 0);
+                for (int g = 0; g < 2; ++g) {
+                    f32x4_t t[GD_SUB];
+                    half8_t b[GD_SUB][2];
+                    float sc[GD_SUB];
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[i], acc[ms][j][i]);
+                    for (int j = 0; j < GD_SUB; ++j) {
+                        b[j][0] = q4_codes_to_f16(gw[h][j][g][0]);
+                        sc[j] = f16_bits_to_f32(static_cast<uint16_t>(g ? sc2[j] >> 16 : sc2[j]));
+                    }
+                    auto scale_in = [&](int ms, int j) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[j][i], acc[ms][j][i]);
+                    };
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms) {
+                        const int k = g * MS + ms;
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+                            for (int j = 0; j < GD_SUB; ++j) {
+                                const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+                                if (c == 0 && ms > 0) scale_in(ms - 1, j);
+                                t[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c], b[j][c >> 1], c ? t[j] : z, 0, 0,
+                                                                              0);
+                            }
+                            if (ms == 0 && c < 2) {
+                                b[2 * c][1] = q4_codes_to_f16(gw[h][2 * c][g][1]);
+                                b[2 * c + 1][1] = q4_codes_to_f16(gw[h][2 * c + 1][g][1]);
+                            }
+                            __builtin_amdgcn_sched_barrier(0);
+                            if (k + 1 < 2 * MS) load_a(k + 1, c);
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < GD_SUB; ++j) scale_in(MS - 1, j);
                 }
             }
             mem_fence_compiler();
-        };
-        for (uint32_t c = 0; c < G; c += 8) {
-            body(c, 0, 0, 3, a0, a3);
-            if (c + 1 < G) body(c + 1, 0, 1, 3, a1, a0);
-            if (c + 2 < G) body(c + 2, 1, 0, 0, a2, a1);
-            if (c + 3 < G) body(c + 3, 1, 1, 0, a3, a2);
-            if (c + 4 < G) body(c + 4, 2, 0, 1, a0, a3);
-            if (c + 5 < G) body(c + 5, 2, 1, 1, a1, a0);
-            if (c + 6 < G) body(c + 6, 3, 0, 2, a2, a1);
-            if (c + 7 < G) body(c + 7, 3, 1, 2, a3, a2);
         }
+        vm_wait<0>();
 #pragma unroll
         for (int ms = 0; ms < MS; ++ms) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t m = 16 * ms + 4 * q + i;
-                if (m0 + m >= M) continue;
+                if (m0 + m >= me) continue;
                 const float rs = a_scale[s_row[m]] * (8.0f / 15.0f);   // weights are (2c - 15) / 8
                 float* o = out + static_cast<size_t>(s_pair[m]) * n_dim;
+                if constexpr (GATE_UP) {
 #pragma unroll
-                for (int j = 0; j < GD_SUB; ++j) {
-                    const uint32_t n = tile * GD_ROWS + 16 * GD_SUB * wv + 16 * j + m16;
-                    if (n < n_dim) o[n] = acc[ms][j][i] * rs;
+                    for (int j = 0; j < GD_SUB / 2; ++j) {
+                        const uint32_t n = tile * (GD_ROWS / 2) + 8 * GD_SUB * wv + 16 * j + m16;
+                        const float v0 = acc[ms][j][i] * rs, v1 = acc[ms][j + GD_SUB / 2][i] * rs;
+                        if (n < n_dim) o[n] = (v0 * (1.0f / (1.0f + expf(-v0)))) * v1;
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < GD_SUB; ++j) {
+                        const uint32_t n = tile * GD_ROWS + 16 * GD_SUB * wv + 16 * j + m16;
+                        if (n < n_dim) o[n] = acc[ms][j][i] * rs;
+                    }
                 }
             }
         }
     }
 }
 
+template <bool GATE_UP>
 __global__ __launch_bounds__(GD_WAVES * WAVE, 2)
-void k_grouped_down(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ sched,
-                    const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
-                    const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale, float* __restrict__ out,
-                    uint32_t n_dim, uint32_t k_dim, uint32_t n_tiles)
+void k_grouped_reg(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ units,
+                   const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
+                   const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale, uint32_t a_row_div,
+                   float* __restrict__ out, uint32_t n_dim, uint32_t k_dim, uint32_t n_tiles)
 {
-    __shared__ __align__(16) GmA a0, a1, a2, a3;
+    __shared__ __align__(16) uint8_t abuf[2 * GD_STAGE];
     __shared__ uint32_t s_row[GM_PASS];
     __shared__ uint32_t s_pair[GM_PASS];
-    // the schedule order of k_grouped_mm
-    const uint32_t b = blockIdx.x, xcd = b & 7u, jb = b >> 3;
-    const uint32_t slot = jb / n_tiles, tile = jb % n_tiles;
-    const uint32_t r = 8u * slot + ((slot & 1u) ? 7u - xcd : xcd);
-    if (r >= sched[0]) return;
-    const uint32_t e = sched[1 + r];
-    if (e >= d.E) return;
-    const uint32_t base = offsets[e], M = offsets[e + 1] - base;
-    if (M == 0) return;
-    if (M <= 16)
-        grouped_down_expert<1>(L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, out, n_dim, k_dim, a0, a1, a2,
-                               a3, s_row, s_pair);
-    else if (M <= 32)
-        grouped_down_expert<2>(L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, out, n_dim, k_dim, a0, a1, a2,
-                               a3, s_row, s_pair);
-    else if (M <= 48)
-        grouped_down_expert<3>(L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, out, n_dim, k_dim, a0, a1, a2,
-                               a3, s_row, s_pair);
-    else
-        grouped_down_expert<4>(L, e, tile, base, M, sorted_pairs, a_hi, a_lo, a_scale, out, n_dim, k_dim, a0, a1, a2,
-                               a3, s_row, s_pair);
+    uint32_t e, tile, base, mb, me, rows;
+    if (!unit_of_block(offsets, units, n_tiles, e, tile, base, mb, me, rows)) return;
+    auto go = [&](auto ms) {
+        grouped_reg_expert<GATE_UP, decltype(ms)::value>(L, e, tile, base, mb, me, sorted_pairs, a_hi, a_lo, a_scale,
+                                                         a_row_div, out, n_dim, k_dim, abuf, s_row, s_pair);
+    };
+    if (rows == 16) go(std::integral_constant<int, 1>{});
+    else if (rows == 32) go(std::integral_constant<int, 2>{});
+    else if (rows == 48) go(std::integral_constant<int, 3>{});
+    else go(std::integral_constant<int, 4>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1292,52 +1500,84 @@ size_t permute_lds_bytes(uint32_t P, uint32_t E)
     return (C * E + 3 * size_t(E) + 1) * sizeof(uint32_t);
 }
 
-// what k_permute allocates: the count table's odd row stride and the keys add
-// at most 2 E words to permute_lds_bytes (which bounds the pass sizes)
+// what k_permute allocates: the count table's odd row stride and the unit
+// offsets add at most 2 E + 1 words to permute_lds_bytes (which bounds the batch)
 static size_t permute_lds_alloc(uint32_t P, uint32_t E)
 {
     const size_t CS = ((P + 63) / 64) | 1u;
-    return (CS * E + 4 * size_t(E) + 1) * sizeof(uint32_t);
+    return (CS * E + 4 * size_t(E) + 2) * sizeof(uint32_t);
 }
 
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
-                          uint32_t* union_size, uint32_t* sched, uint32_t* err, hipStream_t s)
+                          uint32_t* union_size, uint32_t* units, uint32_t few_units, uint32_t* err, hipStream_t s)
 {
     if (P == 0 || E == 0 || permute_lds_bytes(P, E) > PERMUTE_MAX_LDS) return hipErrorInvalidValue;
     const size_t lds = permute_lds_alloc(P, E);
     launch_kernel_lds(k_permute, dim3(1), dim3(PERM_THREADS), static_cast<uint32_t>(lds), s, ids, w, P, K, E,
-                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, sched, err);
+                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, units, few_units, err);
     return hipGetLastError();
 }
 
-hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, const uint32_t* offsets,
-                                  const uint32_t* sched, const uint32_t* sorted_pairs, const uint16_t* x_hi,
+uint32_t perm_segments(uint32_t P, uint32_t E)
+{
+    const uint32_t len = 64u * perm_seg_chunks(E);
+    return (P + len - 1) / len;
+}
+
+hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
+                              uint32_t* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
+{
+    if (P == 0 || E == 0 || E > SMOE_TOPK_MAX_N) return hipErrorInvalidValue;
+    const uint32_t nseg = perm_segments(P, E);
+    launch_kernel(k_perm_count, dim3(nseg), dim3(PERM_THREADS), s, ids, P, E, seg_cnt, err);
+    const uint32_t lds = (E * (perm_seg_chunks(E) | 1u) + 4 * E + 2) * static_cast<uint32_t>(sizeof(uint32_t));
+    launch_kernel_lds(k_perm_scatter, dim3(nseg), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt, offsets,
+                      sorted_pairs, units, few_units);
+    return hipGetLastError();
+}
+
+// k_grouped_reg needs an even number of 64-column groups and its 16-byte
+// weight loads; other layers take k_grouped_mm
+static bool reg_supported(const LayerDesc& L, uint32_t k_dim)
+{
+    bool ok = k_dim % 128 == 0 && reinterpret_cast<uintptr_t>(L.experts) % 16 == 0 && L.stride % 16 == 0;
+    for (int i = 0; i < 6; ++i) ok = ok && L.off[i] % 16 == 0;
+    return ok;
+}
+
+template <bool GATE_UP>
+static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
+                                 const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* a_hi,
+                                 const uint16_t* a_lo, const float* a_scale, float* out, hipStream_t s)
+{
+    if (d.group != 64 || d.I % 64 || d.D % 64 || P == 0 || !offsets || !units) return hipErrorInvalidValue;
+    const uint32_t n_dim = GATE_UP ? d.I : d.D, k_dim = GATE_UP ? d.D : d.I, div = GATE_UP ? d.K : 1u;
+    const uint32_t per = (max_units(P, d.E, few_units) + 7) / 8;
+    if (reg_supported(L, k_dim)) {
+        const uint32_t rows = GATE_UP ? GD_ROWS / 2 : GD_ROWS, nt = (n_dim + rows - 1) / rows;
+        launch_kernel(k_grouped_reg<GATE_UP>, dim3(8 * per * nt), dim3(GD_WAVES * WAVE), s, d, L, offsets, units,
+                      sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
+    } else {
+        const uint32_t rows = GATE_UP ? GM_ROWS_GU : GM_ROWS_DN, nt = (n_dim + rows - 1) / rows;
+        launch_kernel(k_grouped_mm<GATE_UP>, dim3(8 * per * nt), dim3(GM_WAVES * WAVE), s, d, L, offsets, units,
+                      sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
+                                  const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* x_hi,
                                   const uint16_t* x_lo, const float* x_scale, float* h, hipStream_t s)
 {
-    if (d.group != 64 || d.I % 64 || d.D % 64 || !offsets || !sched) return hipErrorInvalidValue;
-    const uint32_t n_tiles = (d.I + GM_ROWS_GU - 1) / GM_ROWS_GU, eg = (d.E + 7) / 8;
-    launch_kernel(k_grouped_mm<true>, dim3(8 * eg * n_tiles), dim3(GM_WAVES * WAVE), s, d, L, offsets, sched,
-                  sorted_pairs, x_hi, x_lo, x_scale, d.K, h, d.I, d.D, n_tiles);
-    return hipGetLastError();
+    return launch_grouped<true>(d, L, P, few_units, offsets, units, sorted_pairs, x_hi, x_lo, x_scale, h, s);
 }
 
-hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, const uint32_t* offsets,
-                               const uint32_t* sched, const uint32_t* sorted_pairs, const uint16_t* h_hi,
+hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
+                               const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* h_hi,
                                const uint16_t* h_lo, const float* h_scale, float* y, hipStream_t s)
 {
-    if (d.group != 64 || d.D % 64 || d.I % 64 || !offsets || !sched) return hipErrorInvalidValue;
-    const uint32_t eg = (d.E + 7) / 8;
-    if (d.I % 128 == 0) {                        // an even number of groups: the register-weight kernel
-        const uint32_t nt = (d.D + GD_ROWS - 1) / GD_ROWS;
-        launch_kernel(k_grouped_down, dim3(8 * eg * nt), dim3(GD_WAVES * WAVE), s, d, L, offsets, sched, sorted_pairs,
-                      h_hi, h_lo, h_scale, y, d.D, d.I, nt);
-        return hipGetLastError();
-    }
-    const uint32_t n_tiles = (d.D + GM_ROWS_DN - 1) / GM_ROWS_DN;
-    launch_kernel(k_grouped_mm<false>, dim3(8 * eg * n_tiles), dim3(GM_WAVES * WAVE), s, d, L, offsets, sched,
-                  sorted_pairs, h_hi, h_lo, h_scale, 1u, y, d.D, d.I, n_tiles);
-    return hipGetLastError();
+    return launch_grouped<false>(d, L, P, few_units, offsets, units, sorted_pairs, h_hi, h_lo, h_scale, y, s);
 }
 
 hipError_t launch_combine_pairs(const float* y, const float* w, uint32_t T, uint32_t K, uint32_t D, float* hidden,

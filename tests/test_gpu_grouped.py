@@ -1,0 +1,53 @@
+"""The grouped prefill GEMMs and the segmented permute at the edges of their
+passes: pair counts around every 16-row tile and 64-row pass, rows of one to
+several pairs of 64-column groups (with and without a remainder), an odd number of
+groups (the LDS-weight kernel), batches over several permute segments and over
+one pass.  Every result against fp64 (moe_delta_f64_batch) and bit for bit
+against the same tokens in calls of 16."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import Layer, hidden_states, moe_delta_f64_batch, rel_err
+
+pytestmark = pytest.mark.gpu
+TOL_F64 = 5e-4   # of test_gpu_prefill's comparison with fp64
+
+
+def prefill(ctx, layer, h, step):
+    out = h.clone()
+    T, K = h.shape[0], layer.K
+    ids = torch.zeros((T, K), dtype=torch.int32, device="cuda")
+    w = torch.zeros((T, K), dtype=torch.float32, device="cuda")
+    for t in range(0, T, step):
+        n = min(step, T - t)
+        ctx.moe_prefill(layer.shape, layer.layer, out[t].data_ptr(), n, ids[t].data_ptr(), w[t].data_ptr())
+    ctx.synchronize()
+    return out, ids, w
+
+
+@pytest.mark.parametrize("D,E,K,I,Ts", [
+    (384, 1, 1, 128, (1, 15, 16, 17, 32, 33, 48, 49, 63, 64, 65, 97, 129, 200)),   # every pair on one expert
+    (128, 1, 1, 640, (16, 33, 65)),      # one pair of groups in, five out
+    (1280, 4, 2, 704, (37, 150)),        # an odd number of groups in the down rows
+    (320, 8, 3, 192, (50,)),             # and in both
+    (256, 512, 8, 128, (300,)),          # segments of 16 chunks
+    (256, 128, 8, 128, (1000, 5000)),    # several segments, several passes
+])
+def test_passes_and_segments(ctx, D, E, K, I, Ts):
+    layer = Layer(ctx, D, E, K, I, layer_id=500 + D + I)
+    hs = hidden_states(ctx, min(max(Ts), 512), D, index0=77)
+    hs = hs.repeat((max(Ts) + len(hs) - 1) // len(hs), 1)
+    hs[:, 0] += torch.arange(len(hs), device="cuda") * 1e-3      # (repeated rows differ)
+    for T in Ts:
+        print(f"case D={D} E={E} K={K} I={I} T={T}", flush=True)
+        h = hs[:T].contiguous()
+        out, ids, w = prefill(ctx, layer, h, T)
+        out16, ids16, w16 = prefill(ctx, layer, h, 16)
+        assert torch.equal(ids, ids16) and torch.equal(w, w16) and torch.equal(out, out16)
+        rows = np.unique(np.linspace(0, T - 1, 200).astype(int))
+        x = h.cpu().numpy()[rows]
+        ref = moe_delta_f64_batch(layer, x, ids.cpu().numpy()[rows], w.cpu().numpy()[rows])
+        got = out.cpu().numpy()[rows]
+        err, _ = rel_err(got.astype(np.float64) - x, ref, slack=np.spacing(np.abs(got)))
+        assert err <= TOL_F64, f"T={T}: {err:.2e}"
