@@ -28,6 +28,7 @@ using smoe::shape_check;
 namespace {
 
 constexpr uint32_t kSlots = SMOE_MAX_ACTIVE;   // scratch regions (metal_bridge.mm:205-210)
+static_assert(smoe::ExpertTable::MAX == kSlots, "a dispatch fits the kernel argument");
 constexpr uint32_t kEvents = 256;              // handle ring
 
 struct DeviceScratch {
@@ -98,7 +99,6 @@ struct SmoeMetalCtx {
     float* d_batch_in = nullptr;     // [64 x 16384]
     float* d_batch_hidden = nullptr;
     float* d_batch_out = nullptr;
-    ExpertPtrs* d_tbl_ref = nullptr; // [kSlots]
 
     hipEvent_t ev[kEvents] = {};
     uint64_t seq = 0;
@@ -357,24 +357,20 @@ bool wait_handle(SmoeMetalCtx* ctx, void* handle)
 }
 
 // one group of same-shaped experts on ctx->d_input (reference surface)
-void* dispatch_group(SmoeMetalCtx* ctx, const ExpertPtrs* tbl_host, uint32_t n, const float* input_vec,
+void* dispatch_group(SmoeMetalCtx* ctx, const smoe::ExpertTable& tbl, uint32_t n, const float* input_vec,
                      uint32_t gate_rows, uint32_t gate_cols, uint32_t group_size)
 {
     const MoeDims d{gate_cols, 0, n, gate_rows, group_size, 0};
     if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_input, input_vec, gate_cols * sizeof(float), hipMemcpyHostToDevice,
                                     ctx->stream), "hipMemcpyAsync(input)"))
         return nullptr;
-    if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_tbl_ref, tbl_host, n * sizeof(ExpertPtrs), hipMemcpyHostToDevice,
-                                    ctx->stream), "hipMemcpyAsync(table)"))
-        return nullptr;
     if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up", [&] {
-            return smoe::launch_gate_up(d, ctx->d_tbl_ref, n, ctx->d_input, ctx->d_hidden, ctx->max_rows, 1, 0, 0, 0,
-                                        ctx->stream);
+            return smoe::launch_gate_up(d, tbl, n, ctx->d_input, ctx->d_hidden, ctx->max_rows, ctx->stream);
         }))
         return nullptr;
     if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down", [&] {
-            return smoe::launch_down_slots(d, ctx->d_tbl_ref, n, ctx->d_hidden, ctx->max_rows, ctx->d_output,
-                                           ctx->max_rows, 1, 0, 0, 0, ctx->stream);
+            return smoe::launch_down_slots(d, tbl, n, ctx->d_hidden, ctx->max_rows, ctx->d_output, ctx->max_rows,
+                                           ctx->stream);
         }))
         return nullptr;
     ctx->dispatches.fetch_add(n, std::memory_order_relaxed);
@@ -403,7 +399,7 @@ extern "C" SmoeMetalCtx* smoe_metal_init(size_t slot_bytes)
               dalloc(ctx, &ctx->d_input, SMOE_MAX_DIM) && dalloc(ctx, &ctx->d_hidden, size_t(kSlots) * ctx->max_rows) &&
               dalloc(ctx, &ctx->d_output, size_t(kSlots) * ctx->max_rows) && dalloc(ctx, &ctx->d_batch_in, plane) &&
               dalloc(ctx, &ctx->d_batch_hidden, plane) && dalloc(ctx, &ctx->d_batch_out, plane) &&
-              dalloc(ctx, &ctx->d_tbl_ref, kSlots) && dalloc(ctx, &ctx->d_err, 1) &&
+              dalloc(ctx, &ctx->d_err, 1) &&
               hip_ok(ctx, hipMemset(ctx->d_err, 0, sizeof(uint32_t)), "hipMemset");
     for (uint32_t i = 0; ok && i < kEvents; ++i)
         ok = hip_ok(ctx, hipEventCreateWithFlags(&ctx->ev[i], hipEventDisableTiming), "hipEventCreate");
@@ -444,7 +440,6 @@ extern "C" void smoe_metal_destroy(SmoeMetalCtx* ctx)
     dfree(ctx->d_batch_in);
     dfree(ctx->d_batch_hidden);
     dfree(ctx->d_batch_out);
-    dfree(ctx->d_tbl_ref);
     for (uint32_t i = 0; i < kEvents; ++i)
         if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
     for (auto& p : ctx->prof) {
@@ -469,8 +464,9 @@ extern "C" void* smoe_metal_fused_ffn(SmoeMetalCtx* ctx, const uint8_t* packed_g
         !scales_down || expert_index >= kSlots)
         return nullptr;
     if (!ref_shape_ok(ctx, gate_rows, gate_cols, down_rows, down_cols, group_size, bits)) return nullptr;
-    ExpertPtrs e{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, expert_index, 0};
-    return dispatch_group(ctx, &e, 1, input_vec, gate_rows, gate_cols, group_size);
+    smoe::ExpertTable tbl{};
+    tbl.e[0] = ExpertPtrs{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, expert_index, 0};
+    return dispatch_group(ctx, tbl, 1, input_vec, gate_rows, gate_cols, group_size);
 }
 
 extern "C" void smoe_metal_wait(SmoeMetalCtx* ctx, void* handle, float* output_vec, uint32_t expert_index,
@@ -489,14 +485,14 @@ extern "C" void* smoe_metal_fused_ffn_group(SmoeMetalCtx* ctx, const SmoeExpertB
 {
     if (!ctx || !experts || !input_vec || n_experts == 0 || n_experts > kSlots) return nullptr;
     if (!ref_shape_ok(ctx, gate_rows, gate_cols, down_rows, down_cols, group_size, bits)) return nullptr;
-    ExpertPtrs tbl[kSlots];
+    smoe::ExpertTable tbl{};
     for (uint32_t i = 0; i < n_experts; ++i) {
         const SmoeExpertBlob& b = experts[i];
         if (!b.packed_gate || !b.scales_gate || !b.packed_up || !b.scales_up || !b.packed_down || !b.scales_down ||
             b.slot >= kSlots)
             return nullptr;
-        tbl[i] = ExpertPtrs{b.packed_gate, b.scales_gate, b.packed_up, b.scales_up, b.packed_down, b.scales_down,
-                            b.slot, 0};
+        tbl.e[i] = ExpertPtrs{b.packed_gate, b.scales_gate, b.packed_up, b.scales_up, b.packed_down, b.scales_down,
+                              b.slot, 0};
     }
     return dispatch_group(ctx, tbl, n_experts, input_vec, gate_rows, gate_cols, group_size);
 }
@@ -515,21 +511,16 @@ extern "C" void* smoe_metal_fused_ffn_batch(SmoeMetalCtx* ctx, const uint8_t* pa
     if (!packed_gate || !scales_gate || !packed_up || !scales_up || !packed_down || !scales_down) return nullptr;
     if (!ref_shape_ok(nullptr, gate_rows, gate_cols, down_rows, down_cols, group_size, bits)) return nullptr;
     const MoeDims d{gate_cols, 0, 1, gate_rows, group_size, 0};
-    ExpertPtrs e{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, 0, 0};
+    const ExpertPtrs e{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, 0, 0};
     if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_batch_in, input_mat, size_t(batch) * gate_cols * sizeof(float),
                                     hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync(batch)"))
         return nullptr;
-    if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_tbl_ref, &e, sizeof(e), hipMemcpyHostToDevice, ctx->stream),
-                "hipMemcpyAsync(table)"))
-        return nullptr;
     if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up(batch)", [&] {
-            return smoe::launch_gate_up(d, ctx->d_tbl_ref, 1, ctx->d_batch_in, ctx->d_batch_hidden, 0, batch,
-                                        gate_cols, 0, gate_rows, ctx->stream);
+            return smoe::launch_gate_up_tokens(d, e, ctx->d_batch_in, ctx->d_batch_hidden, batch, ctx->stream);
         }))
         return nullptr;
     if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down(batch)", [&] {
-            return smoe::launch_down_slots(d, ctx->d_tbl_ref, 1, ctx->d_batch_hidden, 0, ctx->d_batch_out, 0, batch,
-                                           0, gate_rows, down_rows, ctx->stream);
+            return smoe::launch_down_tokens(d, e, ctx->d_batch_hidden, ctx->d_batch_out, batch, ctx->stream);
         }))
         return nullptr;
     ctx->dispatches.fetch_add(1, std::memory_order_relaxed);

@@ -340,6 +340,18 @@ __device__ __forceinline__ float q4_chunk_dot(uint4 v, const float* __restrict__
     return (a0 + a1) + (a2 + a3);
 }
 
+// The eight codes of a word as floats c - 7.5 (exact).
+__device__ __forceinline__ void q4_word_floats(uint32_t w, float (&f)[8])
+{
+    const uint32_t lo = w & 0x0F0F0F0Fu;          // codes 0,2,4,6
+    const uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;   // codes 1,3,5,7
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        f[2 * b] = static_cast<float>((lo >> (8 * b)) & 0xFFu) - 7.5f;
+        f[2 * b + 1] = static_cast<float>((hi >> (8 * b)) & 0xFFu) - 7.5f;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Integer form of a 32-value activation chunk for 4-bit dot products.
 // The chunk is scaled by 2^sh (sh = 22 - exponent of its absmax) and rounded

@@ -58,6 +58,12 @@ struct ExpertPtrs {
     uint32_t        pad_;
 };
 
+// The experts of one reference-surface dispatch (SMOE_MAX_ACTIVE), a kernel argument.
+struct ExpertTable {
+    static constexpr uint32_t MAX = 16;
+    ExpertPtrs e[MAX];
+};
+
 struct MoeDims {
     uint32_t D, E, K, I, group, norm_topk;
     uint32_t quant = 0;   // SMOE_QUANT_*: 0 fp16 absmax (SMOE-Q4), 1 bf16 scale + bf16 min
@@ -78,12 +84,18 @@ struct LayerDesc {
 // err receives 1 if the routing exchange timed out.
 hipError_t launch_moe_up(const MoeDims& d, const LayerDesc& L, const float* hidden, uint32_t n_tok, uint64_t* ll,
                          float* h, uint32_t* ids, float* w, ExpertPtrs* tbl, uint32_t* err, hipStream_t s);
-// h[slot * h_stride + row] = silu(gate.x) * (up.x) for n_exp table entries;
-// x_tok_stride / tbl_tok_stride / h_tok_stride step blockIdx.y over tokens.
-hipError_t launch_gate_up(const MoeDims& d, const ExpertPtrs* tbl, uint32_t n_exp,
-                          const float* x, float* h, uint32_t h_stride, uint32_t n_tok,
-                          uint32_t x_tok_stride, uint32_t tbl_tok_stride,
-                          uint32_t h_tok_stride, hipStream_t s);
+// reference surface, one vector: h[slot * h_stride + row] = silu(gate.x) * (up.x)
+// for n_exp table entries, and out[slot * out_stride + row] = down_slot . h_slot
+hipError_t launch_gate_up(const MoeDims& d, const ExpertTable& tbl, uint32_t n_exp, const float* x, float* h,
+                          uint32_t h_stride, hipStream_t s);
+hipError_t launch_down_slots(const MoeDims& d, const ExpertTable& tbl, uint32_t n_exp, const float* h,
+                             uint32_t h_stride, float* out, uint32_t out_stride, hipStream_t s);
+// reference surface, one expert and n_tok vectors: h [n_tok x I] from x [n_tok x D],
+// out [n_tok x D] from h (rows multiples of 32, groups of 32, 64 or 128)
+hipError_t launch_gate_up_tokens(const MoeDims& d, const ExpertPtrs& e, const float* x, float* h, uint32_t n_tok,
+                                 hipStream_t s);
+hipError_t launch_down_tokens(const MoeDims& d, const ExpertPtrs& e, const float* h, float* out, uint32_t n_tok,
+                              hipStream_t s);
 // hidden[t][row] += sum_r w[t][r] * (down_r . h[t][r])  (weighted combine + residual);
 // zeroes ll [T x (E+1)] for the next launch_moe_up
 hipError_t launch_down_combine(const MoeDims& d, const ExpertPtrs* tbl, const float* h, const float* w,
@@ -152,11 +164,6 @@ bool chain_supported(const MoeDims& d, const LayerDesc* layers_host, uint32_t n_
 hipError_t launch_moe_chain(const MoeDims& d, const LayerDesc* layers_dev, uint32_t n_layers, float* hidden,
                             uint64_t* xch, float* hcopy, uint32_t* cnt, uint32_t* ids, float* w, uint32_t* err,
                             hipStream_t s);
-// out[slot * out_stride + row] = down_slot . h_slot   (per-expert outputs)
-hipError_t launch_down_slots(const MoeDims& d, const ExpertPtrs* tbl, uint32_t n_exp,
-                             const float* h, uint32_t h_stride, float* out,
-                             uint32_t out_stride, uint32_t n_tok, uint32_t tbl_tok_stride,
-                             uint32_t h_tok_stride, uint32_t out_tok_stride, hipStream_t s);
 // softmax + top-k over rows of scores (scout.cpp:77-123)
 hipError_t launch_topk(const float* scores, uint32_t rows, uint32_t n, uint32_t k,
                        uint32_t norm, uint32_t* ids, float* w, hipStream_t s);

@@ -128,3 +128,33 @@ def test_scout_matvec_bf16(ctx, oracle):
     for w, x, o in zip(ws, xs, outs):
         ref = oracle.matvec_bf16(w.cpu().numpy().view(np.uint16).reshape(64, 256), x)
         assert np.allclose(o, ref, rtol=1e-5, atol=1e-6 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("D,I,group,Bs", [
+    (128, 96, 32, (8, 9, 17)),            # groups of 32, fewer steps than waves
+    (256, 128, 128, (16, 33)),            # groups of 128
+    (2048, 768, 64, (8, 9, 16, 64)),      # both sides of the few-token rule, the largest batch
+    (8192, 64, 64, (15,)),                # the longest row, one 64-column step in the down rows
+])
+def test_batch_kernel_edges(ctx, D, I, group, Bs):
+    """Token batches of one expert at the edges of the token and column tiles,
+    against fp64 (two chained fp32 dot products of up to 8192 terms: about
+    sqrt(8192) 2^-24 of the rms, 5e-4 at the metric's 1 % floor)."""
+    rng = np.random.default_rng(D + I + group)
+    L = smoe_amd.lib()
+    dev, mats = [], []
+    for r, c in ((I, D), (I, D), (D, I)):
+        codes = rng.integers(0, 16, (r, c), dtype=np.uint8)
+        scales = (0.02 + 0.05 * rng.random((r, c // group))).astype(np.float16)
+        mats.append((codes.astype(np.float64) - 7.5) / 7.5 * np.repeat(scales.astype(np.float64), group, 1))
+        dev += [torch.from_numpy(codes[:, 0::2] | (codes[:, 1::2] << 4)).cuda(), torch.from_numpy(scales).cuda()]
+    for B in Bs:
+        print(f"case D={D} I={I} group={group} B={B}", flush=True)
+        X = rng.standard_normal((B, D)).astype(np.float32)
+        h = L.smoe_metal_fused_ffn_batch(ctx.ptr, *[t.data_ptr() for t in dev], X.ctypes.data, B, I, D, D, I, group, 4)
+        assert h
+        out = np.full((B, D), np.nan, np.float32)
+        L.smoe_metal_wait_ffn_batch(ctx.ptr, h, out.ctypes.data, B, D)
+        g, u = X.astype(np.float64) @ mats[0].T, X.astype(np.float64) @ mats[1].T
+        ref = (g / (1.0 + np.exp(-g)) * u) @ mats[2].T
+        assert rel_err(out, ref)[0] <= 1e-3
