@@ -29,6 +29,7 @@ namespace {
 
 constexpr uint32_t kSlots = SMOE_MAX_ACTIVE;   // scratch regions (metal_bridge.mm:205-210)
 static_assert(smoe::ExpertTable::MAX == kSlots, "a dispatch fits the kernel argument");
+constexpr uint32_t kHostIn = 4;                // pinned input copies in flight
 constexpr uint32_t kEvents = 256;              // handle ring
 
 struct DeviceScratch {
@@ -91,14 +92,24 @@ struct SmoeMetalCtx {
     hipStream_t stream = nullptr;
     size_t slot_bytes = 0;
     uint32_t max_rows = 0;
+    uint32_t slot_stride = 0;   // floats between scratch regions: max_rows rounded up to 16 bytes
 
     // reference-surface scratch (metal_bridge.mm:205-217, :269-272)
     float* d_input = nullptr;        // [SMOE_MAX_DIM]
-    float* d_hidden = nullptr;       // [kSlots x max_rows]
-    float* d_output = nullptr;       // [kSlots x max_rows]
+    float* d_hidden = nullptr;       // [kSlots x slot_stride]
+    float* h_output = nullptr;       // [kSlots x slot_stride] pinned, written by the down kernel
     float* d_batch_in = nullptr;     // [64 x 16384]
     float* d_batch_hidden = nullptr;
-    float* d_batch_out = nullptr;
+    float* h_batch_out = nullptr;    // [64 x 16384] pinned, at the first batch
+    // pinned copies of the dispatches' inputs: an entry is free again once the
+    // dispatch that read it is done
+    struct HostIn {
+        float* p = nullptr;
+        size_t cap = 0;      // floats
+        uint64_t handle = 0;
+    };
+    HostIn h_in[kHostIn];
+    uint32_t h_in_next = 0;
 
     hipEvent_t ev[kEvents] = {};
     uint64_t seq = 0;
@@ -150,6 +161,22 @@ bool dalloc(SmoeMetalCtx* ctx, T** p, size_t count)
     *p = nullptr;
     if (count == 0) count = 1;
     return hip_ok(ctx, hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T)), "hipMalloc");
+}
+
+// pinned host memory that the GPU reads and writes in place
+bool halloc(SmoeMetalCtx* ctx, float** p, size_t count)
+{
+    *p = nullptr;
+    if (!hip_ok(ctx, hipHostMalloc(reinterpret_cast<void**>(p), count * sizeof(float), hipHostMallocCoherent),
+                "hipHostMalloc"))
+        return false;
+    std::memset(*p, 0, count * sizeof(float));
+    return true;
+}
+void hfree(float*& p)
+{
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
 }
 
 template <typename T>
@@ -340,10 +367,12 @@ bool timed(SmoeMetalCtx* ctx, uint32_t kind, const char* what, F&& launch)
     return hip_ok(ctx, e, what);
 }
 
-void* record_handle(SmoeMetalCtx* ctx)
+// `in`: the dispatch's pinned input, in use until the handle is done
+void* record_handle(SmoeMetalCtx* ctx, SmoeMetalCtx::HostIn* in)
 {
     const uint64_t h = ++ctx->seq;
     if (!hip_ok(ctx, hipEventRecord(ctx->ev[h % kEvents], ctx->stream), "hipEventRecord")) return nullptr;
+    in->handle = h;
     return reinterpret_cast<void*>(static_cast<uintptr_t>(h));
 }
 
@@ -356,25 +385,45 @@ bool wait_handle(SmoeMetalCtx* ctx, void* handle)
     return hip_ok(ctx, hipEventSynchronize(ctx->ev[h % kEvents]), "hipEventSynchronize");
 }
 
+// Copies the caller's input into a free pinned entry (so the caller's buffer is
+// its own again on return) and queues the device copy.  A pageable hipMemcpyAsync
+// in its place costs the call about 10 us, a synchronous hipMemcpy of each
+// output as much again: a group of 8 experts took 143 us of which 16 were kernels.
+SmoeMetalCtx::HostIn* stage_input(SmoeMetalCtx* ctx, const float* src, float* dst, size_t n)
+{
+    SmoeMetalCtx::HostIn& in = ctx->h_in[ctx->h_in_next];
+    ctx->h_in_next = (ctx->h_in_next + 1) % kHostIn;
+    if (in.handle && !wait_handle(ctx, reinterpret_cast<void*>(static_cast<uintptr_t>(in.handle)))) return nullptr;
+    in.handle = 0;
+    if (in.cap < n) {
+        hfree(in.p);
+        in.cap = 0;
+        if (!halloc(ctx, &in.p, n)) return nullptr;
+        in.cap = n;
+    }
+    std::memcpy(in.p, src, n * sizeof(float));
+    if (!hip_ok(ctx, smoe::launch_stage_in(in.p, dst, static_cast<uint32_t>(n), ctx->stream), "stage_in")) return nullptr;
+    return &in;
+}
+
 // one group of same-shaped experts on ctx->d_input (reference surface)
 void* dispatch_group(SmoeMetalCtx* ctx, const smoe::ExpertTable& tbl, uint32_t n, const float* input_vec,
                      uint32_t gate_rows, uint32_t gate_cols, uint32_t group_size)
 {
     const MoeDims d{gate_cols, 0, n, gate_rows, group_size, 0};
-    if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_input, input_vec, gate_cols * sizeof(float), hipMemcpyHostToDevice,
-                                    ctx->stream), "hipMemcpyAsync(input)"))
-        return nullptr;
+    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_vec, ctx->d_input, gate_cols);
+    if (!in) return nullptr;
     if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up", [&] {
-            return smoe::launch_gate_up(d, tbl, n, ctx->d_input, ctx->d_hidden, ctx->max_rows, ctx->stream);
+            return smoe::launch_gate_up(d, tbl, n, ctx->d_input, ctx->d_hidden, ctx->slot_stride, ctx->stream);
         }))
         return nullptr;
     if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down", [&] {
-            return smoe::launch_down_slots(d, tbl, n, ctx->d_hidden, ctx->max_rows, ctx->d_output, ctx->max_rows,
+            return smoe::launch_down_slots(d, tbl, n, ctx->d_hidden, ctx->slot_stride, ctx->h_output, ctx->slot_stride,
                                            ctx->stream);
         }))
         return nullptr;
     ctx->dispatches.fetch_add(n, std::memory_order_relaxed);
-    return record_handle(ctx);
+    return record_handle(ctx, in);
 }
 
 }  // namespace
@@ -394,11 +443,12 @@ extern "C" SmoeMetalCtx* smoe_metal_init(size_t slot_bytes)
     ctx->slot_bytes = slot_bytes;
     ctx->max_rows = static_cast<uint32_t>(std::min(slot_bytes / sizeof(float), size_t(32768)));
     if (ctx->max_rows < SMOE_MAX_DIM) ctx->max_rows = SMOE_MAX_DIM;
+    ctx->slot_stride = (ctx->max_rows + 3u) & ~3u;
     const size_t plane = size_t(SMOE_MAX_FFN_BATCH) * SMOE_MAX_FFN_BATCH_DIM;
     bool ok = hip_ok(ctx, hipStreamCreateWithFlags(&ctx->own_stream, hipStreamNonBlocking), "hipStreamCreate") &&
-              dalloc(ctx, &ctx->d_input, SMOE_MAX_DIM) && dalloc(ctx, &ctx->d_hidden, size_t(kSlots) * ctx->max_rows) &&
-              dalloc(ctx, &ctx->d_output, size_t(kSlots) * ctx->max_rows) && dalloc(ctx, &ctx->d_batch_in, plane) &&
-              dalloc(ctx, &ctx->d_batch_hidden, plane) && dalloc(ctx, &ctx->d_batch_out, plane) &&
+              dalloc(ctx, &ctx->d_input, SMOE_MAX_DIM) && dalloc(ctx, &ctx->d_hidden, size_t(kSlots) * ctx->slot_stride) &&
+              halloc(ctx, &ctx->h_output, size_t(kSlots) * ctx->slot_stride) && dalloc(ctx, &ctx->d_batch_in, plane) &&
+              dalloc(ctx, &ctx->d_batch_hidden, plane) &&
               dalloc(ctx, &ctx->d_err, 1) &&
               hip_ok(ctx, hipMemset(ctx->d_err, 0, sizeof(uint32_t)), "hipMemset");
     for (uint32_t i = 0; ok && i < kEvents; ++i)
@@ -436,10 +486,11 @@ extern "C" void smoe_metal_destroy(SmoeMetalCtx* ctx)
     dfree(ctx->d_err);
     dfree(ctx->d_input);
     dfree(ctx->d_hidden);
-    dfree(ctx->d_output);
+    hfree(ctx->h_output);
+    hfree(ctx->h_batch_out);
+    for (auto& in : ctx->h_in) hfree(in.p);
     dfree(ctx->d_batch_in);
     dfree(ctx->d_batch_hidden);
-    dfree(ctx->d_batch_out);
     for (uint32_t i = 0; i < kEvents; ++i)
         if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
     for (auto& p : ctx->prof) {
@@ -474,8 +525,7 @@ extern "C" void smoe_metal_wait(SmoeMetalCtx* ctx, void* handle, float* output_v
 {
     if (!ctx || !handle || !output_vec || expert_index >= kSlots || cols > ctx->max_rows) return;
     if (!wait_handle(ctx, handle)) return;
-    (void)hip_ok(ctx, hipMemcpy(output_vec, ctx->d_output + size_t(expert_index) * ctx->max_rows,
-                                cols * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy(output)");
+    std::memcpy(output_vec, ctx->h_output + size_t(expert_index) * ctx->slot_stride, cols * sizeof(float));
 }
 
 extern "C" void* smoe_metal_fused_ffn_group(SmoeMetalCtx* ctx, const SmoeExpertBlob* experts, uint32_t n_experts,
@@ -512,19 +562,20 @@ extern "C" void* smoe_metal_fused_ffn_batch(SmoeMetalCtx* ctx, const uint8_t* pa
     if (!ref_shape_ok(nullptr, gate_rows, gate_cols, down_rows, down_cols, group_size, bits)) return nullptr;
     const MoeDims d{gate_cols, 0, 1, gate_rows, group_size, 0};
     const ExpertPtrs e{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, 0, 0};
-    if (!hip_ok(ctx, hipMemcpyAsync(ctx->d_batch_in, input_mat, size_t(batch) * gate_cols * sizeof(float),
-                                    hipMemcpyHostToDevice, ctx->stream), "hipMemcpyAsync(batch)"))
+    if (!ctx->h_batch_out && !halloc(ctx, &ctx->h_batch_out, size_t(SMOE_MAX_FFN_BATCH) * SMOE_MAX_FFN_BATCH_DIM))
         return nullptr;
+    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_mat, ctx->d_batch_in, size_t(batch) * gate_cols);
+    if (!in) return nullptr;
     if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up(batch)", [&] {
             return smoe::launch_gate_up_tokens(d, e, ctx->d_batch_in, ctx->d_batch_hidden, batch, ctx->stream);
         }))
         return nullptr;
     if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down(batch)", [&] {
-            return smoe::launch_down_tokens(d, e, ctx->d_batch_hidden, ctx->d_batch_out, batch, ctx->stream);
+            return smoe::launch_down_tokens(d, e, ctx->d_batch_hidden, ctx->h_batch_out, batch, ctx->stream);
         }))
         return nullptr;
     ctx->dispatches.fetch_add(1, std::memory_order_relaxed);
-    return record_handle(ctx);
+    return record_handle(ctx, in);
 }
 
 extern "C" void smoe_metal_wait_ffn_batch(SmoeMetalCtx* ctx, void* handle, float* out_mat, uint32_t batch,
@@ -532,9 +583,8 @@ extern "C" void smoe_metal_wait_ffn_batch(SmoeMetalCtx* ctx, void* handle, float
 {
     if (!ctx || !handle || !out_mat || batch == 0 || batch > SMOE_MAX_FFN_BATCH || cols > SMOE_MAX_FFN_BATCH_DIM)
         return;
-    if (!wait_handle(ctx, handle)) return;
-    (void)hip_ok(ctx, hipMemcpy(out_mat, ctx->d_batch_out, size_t(batch) * cols * sizeof(float),
-                                hipMemcpyDeviceToHost), "hipMemcpy(batch out)");
+    if (!wait_handle(ctx, handle) || !ctx->h_batch_out) return;
+    std::memcpy(out_mat, ctx->h_batch_out, size_t(batch) * cols * sizeof(float));
 }
 
 extern "C" void smoe_metal_register_buffer(SmoeMetalCtx* ctx, const void* ptr, size_t size_in_bytes)

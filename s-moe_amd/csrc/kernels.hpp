@@ -84,6 +84,8 @@ struct LayerDesc {
 // err receives 1 if the routing exchange timed out.
 hipError_t launch_moe_up(const MoeDims& d, const LayerDesc& L, const float* hidden, uint32_t n_tok, uint64_t* ll,
                          float* h, uint32_t* ids, float* w, ExpertPtrs* tbl, uint32_t* err, hipStream_t s);
+// n floats (a multiple of 4) from pinned host memory to the device
+hipError_t launch_stage_in(const float* src, float* dst, uint32_t n, hipStream_t s);
 // reference surface, one vector: h[slot * h_stride + row] = silu(gate.x) * (up.x)
 // for n_exp table entries, and out[slot * out_stride + row] = down_slot . h_slot
 hipError_t launch_gate_up(const MoeDims& d, const ExpertTable& tbl, uint32_t n_exp, const float* x, float* h,

@@ -397,6 +397,8 @@ void k_q4_rows(MoeDims d, ExpertTable tbl, uint32_t n_exp, const float* __restri
         for (int q = 0; q < 32; ++q) xsum[j] += xr[j][q];
     }
     float* o = out + static_cast<size_t>(tok) * out_tok_stride + static_cast<size_t>(e.slot) * out_stride;
+    static_assert(RB == 4, "four rows a store");
+    float y[RB];
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
         float aa = 0.f, ab = 0.f;
@@ -408,11 +410,11 @@ void k_q4_rows(MoeDims d, ExpertTable tbl, uint32_t n_exp, const float* __restri
         }
         aa = wave_sum(aa);
         if (GATE_UP) ab = wave_sum(ab);
-        if (lane == 0) {
-            // silu(z) = z * (1 / (1 + exp(-z)))  (kernels.metal:61-63, :334-336)
-            o[row0 + i] = GATE_UP ? (aa * (1.0f / (1.0f + expf(-aa)))) * ab : aa;
-        }
+        // silu(z) = z * (1 / (1 + exp(-z)))  (kernels.metal:61-63, :334-336)
+        y[i] = GATE_UP ? (aa * (1.0f / (1.0f + expf(-aa)))) * ab : aa;
     }
+    // one store a wave: `out` of the down rows is host memory
+    if (lane == 0) *reinterpret_cast<float4*>(o + row0) = make_float4(y[0], y[1], y[2], y[3]);
 }
 
 // ---------------------------------------------------------------------------
@@ -751,6 +753,25 @@ static hipError_t launch_tokens(const MoeDims& d, const ExpertPtrs& e, const flo
     else if (kb == 64) launch_kernel(k_ffn_tokens<GATE_UP, 64, 4>, grid, dim3(256), s, d, e, x, out, n_tok);
     else if (w8) launch_kernel(k_ffn_tokens<GATE_UP, 32, 8>, grid, dim3(512), s, d, e, x, out, n_tok);
     else launch_kernel(k_ffn_tokens<GATE_UP, 32, 4>, grid, dim3(256), s, d, e, x, out, n_tok);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// k_stage_in: n4 float4 from pinned host memory to the device, in stream order
+// ahead of the kernels that read them.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256)
+void k_stage_in(const float4* __restrict__ src, float4* __restrict__ dst, uint32_t n4)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) dst[i] = src[i];
+}
+
+hipError_t launch_stage_in(const float* src, float* dst, uint32_t n, hipStream_t s)
+{
+    if (n == 0 || n % 4) return hipErrorInvalidValue;
+    launch_kernel(k_stage_in, dim3((n / 4 + 255) / 256), dim3(256), s, reinterpret_cast<const float4*>(src),
+                  reinterpret_cast<float4*>(dst), n / 4);
     return hipGetLastError();
 }
 

@@ -158,3 +158,30 @@ def test_batch_kernel_edges(ctx, D, I, group, Bs):
         g, u = X.astype(np.float64) @ mats[0].T, X.astype(np.float64) @ mats[1].T
         ref = (g / (1.0 + np.exp(-g)) * u) @ mats[2].T
         assert rel_err(out, ref)[0] <= 1e-3
+
+
+def test_more_dispatches_in_flight_than_input_copies(ctx):
+    """Eight group dispatches queued before the first wait (the context keeps
+    four input copies), each with its own input and slots, the caller's input
+    buffer overwritten after every call; every slot equals the same dispatch
+    waited for at once."""
+    D, I = 256, 128
+    layer = Layer(ctx, D, 2, 2, I, layer_id=31)
+    rng = np.random.default_rng(7)
+    X = rng.standard_normal((8, D)).astype(np.float32)
+    blob = lambda e, slot: smoe_amd.SmoeExpertBlob(*blob_ptrs(layer, e), slot)
+    one = np.zeros((8, 2, D), np.float32)
+    for i in range(8):
+        h = ctx.fused_ffn_group([blob(0, 0), blob(1, 1)], X[i].ctypes.data, I, D)
+        for e in range(2):
+            ctx.wait(h, one[i, e].ctypes.data, e, D)
+    buf, handles = np.zeros(D, np.float32), []
+    for i in range(8):
+        buf[:] = X[i]
+        handles.append(ctx.fused_ffn_group([blob(0, 2 * i), blob(1, 2 * i + 1)], buf.ctypes.data, I, D))
+        buf[:] = np.nan
+    for i in range(8):
+        out = np.zeros((2, D), np.float32)
+        for e in range(2):
+            ctx.wait(handles[i], out[e].ctypes.data, 2 * i + e, D)
+        assert np.array_equal(out, one[i]) and np.any(out)
