@@ -199,7 +199,8 @@ struct AttnDims {
     float scale;
 };
 struct AttnPlan {
-    uint32_t gb;        // query heads per block (power of two <= 8)
+    bool wide;          // k_attn_wide
+    uint32_t gb;        // query heads per block (16, or a power of two <= 8)
     uint32_t n_sub;     // blocks per KV head along the query heads
     uint32_t splits;    // context splits
     uint32_t chunk;     // positions per split

@@ -26,6 +26,8 @@
 //                     3. the waves merged in LDS: with one split the output
 //                        normalised (softmax, decode.cpp:207-226), else the
 //                        block's partial (maximum, sum, weighted V) stored.
+//   k_attn_wide     the same for more than eight query heads per KV head, scores
+//                   and weighted V on MFMA.
 //   k_attn_combine  the splits of each head rescaled to their common maximum
 //                   and normalised.  A kernel of its own: the launch boundary
 //                   publishes every partial at once, where an in-kernel
@@ -444,6 +446,287 @@ void k_attn_decode(AttnArgs p)
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_attn_wide: one block per (KV head, group of up to 16 query heads, context split)
+// ---------------------------------------------------------------------------
+constexpr int AW_HEADS = 16;            // query heads per block (MFMA columns)
+constexpr int AW_TILE = 16;             // positions per wave step (MFMA rows)
+// waves per block: two per SIMD, one where a head's registers leave no room for two
+constexpr int wide_waves(uint32_t head_dim) { return head_dim > 128 ? 4 : 8; }
+
+// maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float quad_max(float v)
+{
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float quad_sum(float v)
+{
+    swap16_sum(v, v);
+    swap32_sum(v, v);
+    return v;
+}
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// v_mfma_f32_16x16x4_f32: lane l = (m16 = l & 15, q = l >> 4) holds A[m16][q] and
+// B[q][m16] and receives D[4 q + i][m16].  Scores: A = K (row = position, K
+// index q of step 4 s + j = dim 16 s + 4 q + j), B = the query heads; a lane
+// then has the scores of positions 4 q + i of head m16, which are the B operand
+// (K index q of step i = position 4 q + i) of the weighted sum, whose A is V
+// transposed (row m16 of result (h, j) = dim 64 h + 4 m16 + j).  No value moves
+// between lanes but the maximum and the final sums.
+//
+// Bound by reading K and V: the attention layer over 32768 positions of the 235B
+// layout (134 MB of K and V, 16 query heads a KV head) takes 59 us, 27 of them its two
+// GEMVs, against 80 with k_attn_decode, whose two blocks per KV head and split, on
+// different XCDs, each read every row and whose dot products are the VALU's.
+// Sums run in chains of eight terms that are then added, as there: 3.73e-7 from
+// fp64 over 32768 positions (12 inputs) against 3.69e-7, 3.96e-7 against 3.95e-7
+// over 5000; in chains of 64 it was 4.4e-7.
+template <int HD>
+__global__ __launch_bounds__(wide_waves(HD) * WAVE, 1)
+void k_attn_wide(AttnArgs p)
+{
+    constexpr int NW = wide_waves(HD), NT = NW * WAVE;
+    constexpr int NS = HD / 16, NH = HD / 64;
+    constexpr int HALF = HD / 2;
+    constexpr int DV = HD / WAVE;               // dims per lane in the norm pass
+    constexpr int RS = HD + 4;                  // padded row of a head in LDS
+
+    __shared__ __align__(16) float qs[AW_HEADS * RS];
+    __shared__ __align__(16) float kn[HD];
+    __shared__ __align__(16) float accw[NW * AW_HEADS * RS];
+    __shared__ float mw[NW * AW_HEADS], lw[NW * AW_HEADS];
+
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m16 = lane & 15, q = lane >> 4;
+    const uint32_t G = p.a.num_heads / p.a.num_kv_heads;
+    const uint32_t kvh = blockIdx.x / p.n_sub, sg = blockIdx.x % p.n_sub, sp = blockIdx.y;
+    const uint32_t hbase = kvh * G + sg * AW_HEADS;   // first query head of the block
+    const uint32_t ng = min(static_cast<uint32_t>(AW_HEADS), G - sg * AW_HEADS);
+    const uint32_t S = p.splits;
+    const uint32_t i0 = sp * p.chunk, n = min(p.chunk, p.valid - i0);
+
+    // ---- K and V of 16 positions from t0 (past the split: its last, masked) ----
+    const float* kbase = p.k_cache + kvh * HD + 4 * q;
+    const float* vbase = p.v_cache + kvh * HD + 4 * m16;
+    struct Tile {
+        float4 k[NS], v[4][NH];
+    };
+    auto ring = [&](uint32_t pos) {
+        const uint32_t ip = i0 + min(pos, n - 1);
+        return static_cast<size_t>(p.slot >= ip ? p.slot - ip : p.slot + p.a.ctx - ip) * p.a.kv_dim;
+    };
+    auto load_tile = [&](uint32_t t0, Tile& t) {
+        const float* k = kbase + ring(t0 + m16);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) t.k[s] = load_f4(k + 16 * s);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* v = vbase + ring(t0 + 4 * q + i);
+#pragma unroll
+            for (int h = 0; h < NH; ++h) t.v[i][h] = load_f4(v + 64 * h);
+        }
+    };
+    // the first tile does not wait for the projections' results (position 0,
+    // the new token, is put in below)
+    Tile ta;
+    const uint32_t first = wv * AW_TILE;
+    if (first < n) load_tile(first, ta);
+
+    // ---- query heads (and the new K row in split 0): RMSNorm ----------------
+    // rms_norm_bf16 per head (common.hpp:245-256): (x * inv) * w
+    auto norm_head = [&](const float* src, const uint16_t* nw, float* dst, bool live) {
+        float xv[DV];
+#pragma unroll
+        for (int j = 0; j < DV; ++j) xv[j] = live ? src[lane * DV + j] : 0.f;
+        if (nw && live) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < DV; ++j) ss = fmaf(xv[j], xv[j], ss);
+            ss = wave_sum(ss);
+            const float inv = 1.0f / sqrtf(ss / static_cast<float>(HD) + 1e-6f);
+#pragma unroll
+            for (int j = 0; j < DV; ++j) xv[j] = (xv[j] * inv) * bf16_to_f32(nw[lane * DV + j]);
+        }
+#pragma unroll
+        for (int j = 0; j < DV; ++j) dst[lane * DV + j] = xv[j];
+    };
+    for (int g = wv; g < AW_HEADS; g += NW)
+        norm_head(p.q + static_cast<size_t>(hbase + g) * HD, p.q_norm_w, qs + g * RS, g < static_cast<int>(ng));
+    if (sp == 0 && wv == NW - 1) norm_head(p.k + static_cast<size_t>(kvh) * HD, p.k_norm_w, kn, true);
+    __syncthreads();
+    // RoPE in place: (x_d, x_{d+half}) rotated by angle d (decode.cpp:168-186)
+    const uint32_t npairs = (ng + (sp == 0 ? 1 : 0)) * HALF;
+    for (uint32_t t = threadIdx.x; t < npairs; t += NT) {
+        const uint32_t g = t / HALF, d = t % HALF;
+        float* r = g < ng ? qs + g * RS : kn;
+        const float c = p.rope_cos[d], sn = p.rope_sin[d];
+        const float x0 = r[d], x1 = r[d + HALF];
+        r[d] = x0 * c - x1 * sn;
+        r[d + HALF] = x0 * sn + x1 * c;
+    }
+    __syncthreads();
+    if (sp == 0) {
+        // KV ring append (every split-0 block of this KV head writes the same
+        // values), and the new row into position 0 of the first tile
+        for (uint32_t d = threadIdx.x; d < HD; d += NT) {
+            const size_t co = static_cast<size_t>(p.slot) * p.a.kv_dim + kvh * HD + d;
+            p.k_cache[co] = kn[d];
+            p.v_cache[co] = p.v[kvh * HD + d];
+        }
+        if (wv == 0) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const float4 f = *reinterpret_cast<const float4*>(kn + 16 * s + 4 * q);
+                if (min(static_cast<uint32_t>(m16), n - 1) == 0) ta.k[s] = f;
+            }
+            // (also where a masked position repeats position 0: its weight is 0,
+            // but what the ring held there before need not be a number)
+            const float* v = p.v + kvh * HD + 4 * m16;
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                const float4 f = make_float4(v[64 * h], v[64 * h + 1], v[64 * h + 2], v[64 * h + 3]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (min(static_cast<uint32_t>(4 * q + i), n - 1) == 0) ta.v[i][h] = f;
+            }
+        }
+    }
+
+    // ---- the split's positions ----------------------------------------------
+    float4 qv[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qv[s] = *reinterpret_cast<const float4*>(qs + m16 * RS + 16 * s + 4 * q);
+    const float scale = p.a.scale;
+    float mx = -INFINITY, lsum = 0.f;           // of head m16 (the sum: this lane's positions)
+    f32x4_t acc[NH][4];
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[h][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](uint32_t t0, const Tile& t) {
+        // chains of 8 terms, then added up: the rounding of short sums, as the VALU kernel has
+        f32x4_t sc[4];
+#pragma unroll
+        for (int s0 = 0; s0 < NS; s0 += 2) {
+            f32x4_t c[4];
+#pragma unroll
+            for (int s = s0; s < s0 + 2; ++s) {
+                const float kf[4] = {t.k[s].x, t.k[s].y, t.k[s].z, t.k[s].w};
+                const float qf[4] = {qv[s].x, qv[s].y, qv[s].z, qv[s].w};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+                    c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j], qf[j], s > s0 ? c[j] : z, 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sc[j] = s0 ? sc[j] + c[j] : c[j];
+        }
+        float sv[4], mt = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sv[i] = t0 + 4 * q + i < n ? ((sc[0][i] + sc[1][i]) + (sc[2][i] + sc[3][i])) * scale : -INFINITY;
+            mt = fmaxf(mt, sv[i]);
+        }
+        mt = quad_max(mt);
+        if (__ballot(mt > mx)) {
+            const float mn = fmaxf(mx, mt), f = mx > -INFINITY ? __expf(mx - mn) : 0.f;
+            lsum *= f;
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[h][j][i] *= f;
+            mx = mn;
+        }
+        float pe[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            pe[i] = __expf(sv[i] - mx);
+            lsum += pe[i];
+        }
+        // (the tile's own sums first, then into the running ones)
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int jj = 0; jj < 4; jj += 2) {
+                f32x4_t ts[2][2];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float va[4] = {t.v[i][h].x, t.v[i][h].y, t.v[i][h].z, t.v[i][h].w};
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+                        ts[i >> 1][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[jj + j], pe[i],
+                                                                             i & 1 ? ts[i >> 1][j] : z, 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[h][jj + j] += ts[0][j] + ts[1][j];
+            }
+    };
+    constexpr uint32_t STRIDE = NW * AW_TILE;
+    if constexpr (HD <= 128) {
+        Tile tb;
+        for (uint32_t t0 = first; t0 < n; t0 += 2 * STRIDE) {
+            if (t0 + STRIDE < n) load_tile(t0 + STRIDE, tb);
+            step(t0, ta);
+            if (t0 + STRIDE >= n) break;
+            if (t0 + 2 * STRIDE < n) load_tile(t0 + 2 * STRIDE, ta);
+            step(t0 + STRIDE, tb);
+        }
+    } else {
+        // (no registers for a second tile)
+        for (uint32_t t0 = first; t0 < n; t0 += STRIDE) {
+            step(t0, ta);
+            if (t0 + STRIDE < n) load_tile(t0 + STRIDE, ta);
+        }
+    }
+
+    // ---- merge: the four lanes of a head, then the waves, then splits -------
+    lsum = quad_sum(lsum);
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)             // dims 64 h + 4 (4 q + i) + j of head m16
+            *reinterpret_cast<float4*>(accw + (wv * AW_HEADS + m16) * RS + 64 * h + 16 * q + 4 * i) =
+                make_float4(acc[h][0][i], acc[h][1][i], acc[h][2][i], acc[h][3][i]);
+    if (q == 0) {
+        mw[wv * AW_HEADS + m16] = mx;
+        lw[wv * AW_HEADS + m16] = lsum;
+    }
+    __syncthreads();
+    for (uint32_t o = threadIdx.x; o < ng * HD; o += NT) {
+        const uint32_t g = o / HD, d = o % HD;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, mw[w * AW_HEADS + g]);
+        float L = 0.f, A = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float f = __expf(mw[w * AW_HEADS + g] - M);
+            L = fmaf(f, lw[w * AW_HEADS + g], L);
+            A = fmaf(f, accw[(w * AW_HEADS + g) * RS + d], A);
+        }
+        const uint32_t h = hbase + g;
+        if (S == 1) {
+            p.out[static_cast<size_t>(h) * HD + d] = A * (1.0f / L);
+        } else {
+            p.part_acc[(static_cast<size_t>(h) * ATTN_MAX_SPLITS + sp) * HD + d] = A;
+            if (d == 0) {
+                p.part_ml[(static_cast<size_t>(h) * ATTN_MAX_SPLITS + sp) * 2] = M;
+                p.part_ml[(static_cast<size_t>(h) * ATTN_MAX_SPLITS + sp) * 2 + 1] = L;
+            }
+        }
+    }
+}
+
 // one wave per (query head, 64 dims): the splits rescaled to their common
 // maximum and normalised, out = sum_s f_s acc_s / sum_s f_s l_s with
 // f_s = exp(m_s - max_s m_s); every split's load is in flight at once
@@ -473,13 +756,22 @@ AttnPlan attn_plan(const AttnDims& a, uint32_t valid)
 {
     AttnPlan pl{};
     const uint32_t G = a.num_heads / a.num_kv_heads;
+    // The MFMA kernel reads each K and V row once for all query heads of a KV
+    // head, the other one once per block of up to eight.  Long contexts with more than
+    // eight: 16 heads of 128 over 32768 positions 80 -> 59 us for the layer, ten of 256 92
+    // -> 61.  Over 1000 positions, where the launches' latencies decide, it loses (39.5
+    // against 38.7; ten of 256 over 2048 27.1 against 24.0), at 3000 the two are even,
+    // and with eight heads or fewer its columns are half or more empty (8 heads over
+    // 32768 positions 39.3 against 41.8, one head 31.5 against 30.0).
+    pl.wide = G > static_cast<uint32_t>(AT_MAX_GB) && valid >= 4096;
     uint32_t gb = 1;
     while (gb < G && gb < static_cast<uint32_t>(AT_MAX_GB) && gb * 2 * a.head_dim <= AT_MAX_GHD) gb *= 2;
-    pl.gb = gb;
-    pl.n_sub = (G + gb - 1) / gb;
+    pl.gb = pl.wide ? AW_HEADS : gb;
+    pl.n_sub = (G + pl.gb - 1) / pl.gb;
     const uint32_t bx = a.num_kv_heads * pl.n_sub;
     // at least one tile per wave; about one block per CU (256) in all
-    const uint32_t tile_all = AT_WAVES * (WAVE / (a.head_dim / 8)) * AT_U;
+    const uint32_t tile_all =
+        pl.wide ? wide_waves(a.head_dim) * AW_TILE : AT_WAVES * (WAVE / (a.head_dim / 8)) * AT_U;
     const uint32_t cap = std::max<uint32_t>(1, std::min<uint32_t>(ATTN_MAX_SPLITS, (256 + bx - 1) / bx));
     uint32_t S = std::min<uint32_t>((valid + tile_all - 1) / tile_all, cap);
     S = std::max<uint32_t>(S, 1);
@@ -498,6 +790,12 @@ template <int HD, int GB>
 static void attn_launch(const AttnArgs& args, dim3 grid, hipStream_t s)
 {
     launch_kernel(k_attn_decode<HD, GB>, grid, dim3(AT_THREADS), s, args);
+}
+
+template <int HD>
+static void attn_launch_wide(const AttnArgs& args, dim3 grid, hipStream_t s)
+{
+    launch_kernel(k_attn_wide<HD>, grid, dim3(wide_waves(HD) * WAVE), s, args);
 }
 
 hipError_t launch_attention(const AttnDims& a, const float* q, const float* k, const float* v,
@@ -530,6 +828,11 @@ hipError_t launch_attention(const AttnDims& a, const float* q, const float* k, c
     args.splits = pl.splits;
     args.n_sub = pl.n_sub;
     const dim3 grid(a.num_kv_heads * pl.n_sub, pl.splits);
+    if (pl.wide) {
+        if (a.head_dim == 64) attn_launch_wide<64>(args, grid, s);
+        else if (a.head_dim == 128) attn_launch_wide<128>(args, grid, s);
+        else attn_launch_wide<256>(args, grid, s);
+    } else
     switch (a.head_dim * 16 + pl.gb) {
         case 64 * 16 + 1: attn_launch<64, 1>(args, grid, s); break;
         case 64 * 16 + 2: attn_launch<64, 2>(args, grid, s); break;

@@ -94,6 +94,11 @@ def rope(pos, head_dim, theta=1e6):
     (1024, 16, 16, 64, 2048, 100, 1500, True),   # MHA, several context splits
     (2048, 8, 2, 256, 512, 300, 400, True),      # head_dim 256
     (1280, 10, 2, 128, 1024, 50, 800, False),    # 5 query heads per KV head (padded group)
+    (4096, 64, 4, 128, 8192, 3000, 4095, True),  # 16 query heads per KV head: the last VALU context,
+    (4096, 64, 4, 128, 8192, 3000, 4096, True),  # and the first on MFMA, wrapped
+    (1024, 18, 2, 64, 5000, 4999, 5000, False),  # 9 of 16 MFMA columns, uneven splits
+    (512, 34, 2, 64, 4200, 7, 4161, True),       # 17 query heads: a second block with one
+    (512, 12, 1, 256, 4300, 100, 4100, True),    # head_dim 256 on MFMA
 ])
 def test_attention_layer_vs_oracle(ctx, oracle, d_model, nh, nkv, hd, ctx_len, slot, valid, qk):
     run_attention_case(ctx, oracle, d_model, nh, nkv, hd, ctx_len, slot, valid, qk)
