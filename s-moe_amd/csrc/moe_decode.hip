@@ -21,6 +21,7 @@
 //
 // Loads of packed nibbles are 128-bit and non-temporal; activations and h
 // planes are tiny and stay in L2.
+#include <algorithm>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -59,7 +60,7 @@ void k_topk(const float* __restrict__ scores, uint32_t n, uint32_t k, uint32_t n
 
 // ---------------------------------------------------------------------------
 // k_moe_up: RMSNorm + router + softmax/top-k + gate/up/SiLU for one layer.
-// One wave per block; grid (I / 8, K, T).  Lane l owns the 32 columns of
+// One wave per block; grid (at most I / 8, K, T).  Lane l owns the 32 columns of
 // chunk l (+64 j) of the hidden dimension throughout.  Every wave:
 //   1. loads its hidden and norm-weight chunks and its router rows,
 //   2. RMS-normalises them, normed = (x * inv) * w (common.hpp:245-256),
@@ -68,8 +69,8 @@ void k_topk(const float* __restrict__ scores, uint32_t n, uint32_t k, uint32_t n
 //      (common.hpp:293-306), published as flag-carrying 64-bit words,
 //   5. polls the E logits of its token and selects the experts itself
 //      (softmax + top-k, scout.cpp:77-123; renormalised, decode.cpp:296-302),
-//   6. streams 8 rows of gate and up of the expert of rank blockIdx.y and
-//      writes h = silu(gate) * up (kernels.metal:240-337).
+//   6. streams its blocks of 8 rows of gate and up of the expert of rank
+//      blockIdx.y and writes h = silu(gate) * up (kernels.metal:240-337).
 // The logit exchange is XCD-local when the token's block count is a multiple
 // of 8: the dispatcher deals consecutive blocks round-robin over the 8 XCDs
 // (from some starting XCD), so block b is the (b/8)-th of its XCD, and the
@@ -87,7 +88,7 @@ constexpr uint32_t SPIN_LIMIT = 1u << 22;
 constexpr int UP_RB = 8;   // rows per wave
 constexpr int SMOE_G = 64; // SMOE-Q4 group size (shatter_moe.py Q2_GROUP_SIZE)
 
-template <int CPL, int VPL, bool LOCAL>
+template <int CPL, int VPL, bool LOCAL, bool LOOP>
 __device__ __forceinline__ void moe_up_body(const MoeDims& d, const LayerDesc& L, const float* __restrict__ hv,
                                             uint64_t* __restrict__ ll, float* __restrict__ h,
                                             uint32_t* __restrict__ ids_out, float* __restrict__ w_out,
@@ -269,53 +270,81 @@ __device__ __forceinline__ void moe_up_body(const MoeDims& d, const LayerDesc& L
         tbl_out[o] = e;
     }
 
-    // 6. 8 rows of gate and up: every weight load in flight before any is used
-    const uint32_t rowg = blockIdx.x * RB;
+    // 6. row block blockIdx.x of 8 rows of gate and up, and with LOOP + gridDim.x,
+    // ...: every weight load of a block in flight before any is used, and with one
+    // chunk a lane the next block's as well
     const uint8_t* blob = L.experts + static_cast<size_t>(expert) * L.stride;
     const uint8_t* pa = blob + L.off[0];
     const uint16_t* sa = reinterpret_cast<const uint16_t*>(blob + L.off[1]);
     const uint8_t* pb = blob + L.off[2];
     const uint16_t* sb = reinterpret_cast<const uint16_t*>(blob + L.off[3]);
     const uint32_t row_bytes = D >> 1, row_scales = D / SMOE_G;
-    uint4 va[RB][CPL], vb[RB][CPL];
-    uint16_t sva[RB][CPL], svb[RB][CPL];
-#pragma unroll
-    for (int i = 0; i < RB; ++i) {
-        const size_t row = rowg + i;
-#pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-            const uint32_t c = min(lane + WAVE * j, nch - 1);
-            va[i][j] = load_stream_u4(pa + row * row_bytes + c * 16);
-            vb[i][j] = load_stream_u4(pb + row * row_bytes + c * 16);
-            sva[i][j] = load_stream_u16(sa + row * row_scales + (c * 32) / SMOE_G);
-            svb[i][j] = load_stream_u16(sb + row * row_scales + (c * 32) / SMOE_G);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    // per-lane partial dots: value 2i = gate row i, 2i + 1 = up row i
-    float part[2 * RB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i) {
-        float ga = 0.f, ua = 0.f;
-#pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-            ga = fmaf(f16_bits_to_f32(sva[i][j]), q4_chunk_dot8(va[i][j], qa[j]), ga);
-            ua = fmaf(f16_bits_to_f32(svb[i][j]), q4_chunk_dot8(vb[i][j], qa[j]), ua);
-        }
-        part[2 * i] = ga;
-        part[2 * i + 1] = ua;
-    }
-    // lane l holds the total of value l >> SH
-    constexpr int SH = 6 - ilog2(2 * RB);
-    const float tot = wave_sum_rows<2 * RB>(part);
-    const float gv = __shfl(tot, (2 * lane) << SH);
-    const float uv = __shfl(tot, (2 * lane + 1) << SH);
-    // silu(z) = z * (1 / (1 + exp(-z)))  (kernels.metal:61-63, :334-336), all rows at once
     float* o = h + (static_cast<size_t>(tok) * d.K + r) * d.I;
-    if (lane < RB) o[rowg + lane] = (gv * (1.0f / (1.0f + expf(-gv)))) * uv;
+    struct Rows {
+        uint4 va[RB][CPL], vb[RB][CPL];
+        uint16_t sva[RB][CPL], svb[RB][CPL];
+    };
+    auto load_rows = [&](uint32_t rb, Rows& w) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const size_t row = rb * RB + i;
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                const uint32_t c = min(lane + WAVE * j, nch - 1);
+                w.va[i][j] = load_stream_u4(pa + row * row_bytes + c * 16);
+                w.vb[i][j] = load_stream_u4(pb + row * row_bytes + c * 16);
+                w.sva[i][j] = load_stream_u16(sa + row * row_scales + (c * 32) / SMOE_G);
+                w.svb[i][j] = load_stream_u16(sb + row * row_scales + (c * 32) / SMOE_G);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto do_rows = [&](uint32_t rb, const Rows& w) {
+        // per-lane partial dots: value 2i = gate row i, 2i + 1 = up row i
+        float part[2 * RB];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            float ga = 0.f, ua = 0.f;
+#pragma unroll
+            for (int j = 0; j < CPL; ++j) {
+                ga = fmaf(f16_bits_to_f32(w.sva[i][j]), q4_chunk_dot8(w.va[i][j], qa[j]), ga);
+                ua = fmaf(f16_bits_to_f32(w.svb[i][j]), q4_chunk_dot8(w.vb[i][j], qa[j]), ua);
+            }
+            part[2 * i] = ga;
+            part[2 * i + 1] = ua;
+        }
+        // lane l holds the total of value l >> SH
+        constexpr int SH = 6 - ilog2(2 * RB);
+        const float tot = wave_sum_rows<2 * RB>(part);
+        const float gv = __shfl(tot, (2 * lane) << SH);
+        const float uv = __shfl(tot, (2 * lane + 1) << SH);
+        // silu(z) = z * (1 / (1 + exp(-z)))  (kernels.metal:61-63, :334-336), all rows at once
+        if (lane < RB) o[rb * RB + lane] = (gv * (1.0f / (1.0f + expf(-gv)))) * uv;
+    };
+    const uint32_t nrb = d.I / RB, step = gridDim.x;
+    Rows wa;
+    if constexpr (!LOOP) {
+        load_rows(blockIdx.x, wa);
+        do_rows(blockIdx.x, wa);
+    } else if constexpr (CPL == 1) {
+        Rows wb;
+        load_rows(blockIdx.x, wa);
+        for (uint32_t rb = blockIdx.x; rb < nrb; rb += 2 * step) {
+            if (rb + step < nrb) load_rows(rb + step, wb);
+            do_rows(rb, wa);
+            if (rb + step >= nrb) break;
+            if (rb + 2 * step < nrb) load_rows(rb + 2 * step, wa);
+            do_rows(rb + step, wb);
+        }
+    } else {
+        for (uint32_t rb = blockIdx.x; rb < nrb; rb += step) {
+            load_rows(rb, wa);
+            do_rows(rb, wa);
+        }
+    }
 }
 
-template <int CPL, int VPL, bool LOCAL>
+template <int CPL, int VPL, bool LOCAL, bool LOOP>
 __global__ __launch_bounds__(WAVE)
 void k_moe_up(MoeDims d, LayerDesc L, const float* __restrict__ hidden, uint64_t* __restrict__ ll_all,
               float* __restrict__ h, uint32_t* __restrict__ ids_out, float* __restrict__ w_out,
@@ -324,7 +353,7 @@ void k_moe_up(MoeDims d, LayerDesc L, const float* __restrict__ hidden, uint64_t
     const uint32_t tok = blockIdx.z;
     const float* hv = hidden + static_cast<size_t>(tok) * d.D;
     uint64_t* ll = ll_all + static_cast<size_t>(tok) * ll_token_words(d.E);
-    moe_up_body<CPL, VPL, LOCAL>(d, L, hv, ll, h, ids_out, w_out, tbl_out, err);
+    moe_up_body<CPL, VPL, LOCAL, LOOP>(d, L, hv, ll, h, ids_out, w_out, tbl_out, err);
 }
 
 // ---------------------------------------------------------------------------
@@ -538,7 +567,7 @@ void k_ffn_tokens(MoeDims d, ExpertPtrs e, const float* __restrict__ x, float* _
 constexpr int DOWN_RB = 8;
 constexpr int DOWN_MAX_WAVES = 8;
 
-template <int PPL>
+template <int PPL, bool LOOP>
 __global__ __launch_bounds__(DOWN_MAX_WAVES * WAVE)
 void k_down_combine(MoeDims d, const ExpertPtrs* __restrict__ tbl, const float* __restrict__ h,
                     const float* __restrict__ w, float* __restrict__ hidden, uint64_t* __restrict__ ll_all)
@@ -551,10 +580,9 @@ void k_down_combine(MoeDims d, const ExpertPtrs* __restrict__ tbl, const float* 
         for (uint32_t i = threadIdx.x; i < LL_COPIES * d.E; i += blockDim.x)
             ll[(i / d.E) * ll_copy_words(d.E) + i % d.E] = 0;
     }
-    __shared__ float part[DOWN_MAX_WAVES][RB];
+    __shared__ float part[2][DOWN_MAX_WAVES][RB];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int nw = blockDim.x >> 6;
-    const uint32_t row0 = blockIdx.x * RB;
     const uint32_t tok = blockIdx.y;
     tbl += static_cast<size_t>(tok) * d.K;
     h += static_cast<size_t>(tok) * d.K * d.I;
@@ -588,18 +616,27 @@ void k_down_combine(MoeDims d, const ExpertPtrs* __restrict__ tbl, const float* 
         wr[j] = w[rr[j]];
     }
     __builtin_amdgcn_sched_barrier(0);
-    uint4 v[RB][PPL];
-    uint16_t sv[RB][PPL];
+    // row block blockIdx.x of RB rows, and with LOOP + gridDim.x, ..., the next
+    // block's weights requested before this one's are used
+    struct Rows {
+        uint4 v[RB][PPL];
+        uint16_t sv[RB][PPL];
+    };
+    auto load_rows = [&](uint32_t rb, Rows& x) {
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-        const size_t row = row0 + i;
+        for (int i = 0; i < RB; ++i) {
+            const size_t row = rb * RB + i;
 #pragma unroll
-        for (int j = 0; j < PPL; ++j) {
-            v[i][j] = load_stream_u4(pd[j] + row * row_bytes + cc[j] * 16);
-            sv[i][j] = load_stream_u16(sd[j] + row * row_scales + (cc[j] * 32) / SMOE_G);
+            for (int j = 0; j < PPL; ++j) {
+                x.v[i][j] = load_stream_u4(pd[j] + row * row_bytes + cc[j] * 16);
+                x.sv[i][j] = load_stream_u16(sd[j] + row * row_scales + (cc[j] * 32) / SMOE_G);
+            }
         }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const uint32_t nrb = d.D / RB, step = gridDim.x;
+    Rows xa;
+    load_rows(blockIdx.x, xa);
     Q4Act qh[PPL];
 #pragma unroll
     for (int j = 0; j < PPL; ++j) {
@@ -614,26 +651,42 @@ void k_down_combine(MoeDims d, const ExpertPtrs* __restrict__ tbl, const float* 
         q4_act_from_floats(a, qh[j]);
         if (!ok[j]) wr[j] = 0.f;   // pairs past the end contribute nothing
     }
-    float acc[RB];
+    auto do_rows = [&](uint32_t rb, const Rows& x, int buf) {
+        float acc[RB];
 #pragma unroll
-    for (int i = 0; i < RB; ++i) {
-        acc[i] = 0.f;
+        for (int i = 0; i < RB; ++i) {
+            acc[i] = 0.f;
 #pragma unroll
-        for (int j = 0; j < PPL; ++j) {
-            const float y = f16_bits_to_f32(sv[i][j]) * q4_chunk_dot8(v[i][j], qh[j]);
-            acc[i] = fmaf(wr[j], y, acc[i]);
+            for (int j = 0; j < PPL; ++j) {
+                const float y = f16_bits_to_f32(x.sv[i][j]) * q4_chunk_dot8(x.v[i][j], qh[j]);
+                acc[i] = fmaf(wr[j], y, acc[i]);
+            }
         }
-    }
-    // lane l holds the wave's total of row l >> SH
-    constexpr int SH = 6 - ilog2(RB);
-    const float tot = wave_sum_rows<RB>(acc);
-    if ((lane & ((1 << SH) - 1)) == 0) part[wv][lane >> SH] = tot;
-    __syncthreads();
-    if (threadIdx.x < RB) {
-        float t = 0.f;
-        for (int q = 0; q < nw; ++q) t += part[q][threadIdx.x];
-        const uint32_t row = row0 + threadIdx.x;
-        hidden[row] = hidden[row] + t;
+        // lane l holds the wave's total of row l >> SH
+        constexpr int SH = 6 - ilog2(RB);
+        const float tot = wave_sum_rows<RB>(acc);
+        if ((lane & ((1 << SH) - 1)) == 0) part[buf][wv][lane >> SH] = tot;
+        // (two buffers: the next block's partials go to the other one, and the
+        // one after that is past the barrier that every reader has reached)
+        __syncthreads();
+        if (threadIdx.x < RB) {
+            float t = 0.f;
+            for (int q = 0; q < nw; ++q) t += part[buf][q][threadIdx.x];
+            const uint32_t row = rb * RB + threadIdx.x;
+            hidden[row] = hidden[row] + t;
+        }
+    };
+    if constexpr (LOOP) {
+        Rows xb;
+        for (uint32_t rb = blockIdx.x; rb < nrb; rb += 2 * step) {
+            if (rb + step < nrb) load_rows(rb + step, xb);
+            do_rows(rb, xa, 0);
+            if (rb + step >= nrb) break;
+            if (rb + 2 * step < nrb) load_rows(rb + 2 * step, xa);
+            do_rows(rb + step, xb, 1);
+        }
+    } else {
+        do_rows(blockIdx.x, xa, 0);
     }
 }
 
@@ -641,7 +694,7 @@ void k_down_combine(MoeDims d, const ExpertPtrs* __restrict__ tbl, const float* 
 // launchers
 // ---------------------------------------------------------------------------
 template <int CPL, int VPL>
-static void moe_up_v(dim3 grid, hipStream_t s, const MoeDims& d, const LayerDesc& L, const float* hidden,
+static void moe_up_v(dim3 grid, bool loop, hipStream_t s, const MoeDims& d, const LayerDesc& L, const float* hidden,
                      uint64_t* ll, float* h, uint32_t* ids, float* w, ExpertPtrs* tbl, uint32_t* err)
 {
     // XCD-local logit exchange when every XCD receives the same number of
@@ -649,32 +702,41 @@ static void moe_up_v(dim3 grid, hipStream_t s, const MoeDims& d, const LayerDesc
     // and the whole grid is resident at once (the dispatcher's round-robin
     // over the XCDs is then unbroken)
     const uint32_t nb = grid.x * grid.y;
-    if (nb % 8 == 0 && nb / 8 * 2 >= d.E && nb * grid.z <= 1024)
-        launch_kernel(k_moe_up<CPL, VPL, true>, grid, dim3(WAVE), s, d, L, hidden, ll, h, ids, w, tbl, err);
-    else
-        launch_kernel(k_moe_up<CPL, VPL, false>, grid, dim3(WAVE), s, d, L, hidden, ll, h, ids, w, tbl, err);
+    const bool local = nb % 8 == 0 && nb / 8 * 2 >= d.E && nb * grid.z <= 1024;
+    auto go = [&](auto* k) { launch_kernel(k, grid, dim3(WAVE), s, d, L, hidden, ll, h, ids, w, tbl, err); };
+    if (local) loop ? go(k_moe_up<CPL, VPL, true, true>) : go(k_moe_up<CPL, VPL, true, false>);
+    else loop ? go(k_moe_up<CPL, VPL, false, true>) : go(k_moe_up<CPL, VPL, false, false>);
 }
 
 template <int CPL>
-static void moe_up_c(dim3 grid, hipStream_t s, const MoeDims& d, const LayerDesc& L, const float* hidden,
+static void moe_up_c(dim3 grid, bool loop, hipStream_t s, const MoeDims& d, const LayerDesc& L, const float* hidden,
                      uint64_t* ll, float* h, uint32_t* ids, float* w, ExpertPtrs* tbl, uint32_t* err)
 {
     if (d.E <= 128)
-        moe_up_v<CPL, 2>(grid, s, d, L, hidden, ll, h, ids, w, tbl, err);
+        moe_up_v<CPL, 2>(grid, loop, s, d, L, hidden, ll, h, ids, w, tbl, err);
     else
-        moe_up_v<CPL, 8>(grid, s, d, L, hidden, ll, h, ids, w, tbl, err);
+        moe_up_v<CPL, 8>(grid, loop, s, d, L, hidden, ll, h, ids, w, tbl, err);
 }
 
 hipError_t launch_moe_up(const MoeDims& d, const LayerDesc& L, const float* hidden, uint32_t n_tok, uint64_t* ll,
                          float* h, uint32_t* ids, float* w, ExpertPtrs* tbl, uint32_t* err, hipStream_t s)
 {
     if (d.group != 64 || d.E > SMOE_TOPK_MAX_N || d.I % UP_RB) return hipErrorInvalidValue;
-    const uint32_t row_blocks = d.I / UP_RB;                              // one wave per 8 rows
-    const dim3 grid(row_blocks, d.K, n_tok);
+    const uint32_t row_blocks = d.I / UP_RB;
+    // Several row blocks a wave once the waves outnumber what the chip holds at
+    // two a SIMD (2048): the norm, the digits and the top-k, half of a wave's
+    // VALU work with one block, are then done once per wave (11 tokens of the
+    // 30B shape 52 -> 33 us, 24 tokens 107 -> 60; with waves for one or three a
+    // SIMD 40 and 36).  Grids between one and two a SIMD fold to one, whose logit
+    // exchange is XCD-local (2 tokens 14.0 -> 12.7).
+    const uint32_t waves = row_blocks * d.K * n_tok;
+    const uint32_t most = std::max(1u, (n_tok > 1 && waves > 1024 && waves <= 2048 ? 1024u : 2048u) / (d.K * n_tok));
+    const uint32_t iters = (row_blocks + most - 1) / most;
+    const dim3 grid((row_blocks + iters - 1) / iters, d.K, n_tok);
     const uint32_t cpl = (d.D / 32 + WAVE - 1) / WAVE;   // 32-column chunks per lane
-    if (cpl == 1) moe_up_c<1>(grid, s, d, L, hidden, ll, h, ids, w, tbl, err);
-    else if (cpl == 2) moe_up_c<2>(grid, s, d, L, hidden, ll, h, ids, w, tbl, err);
-    else if (cpl <= 4) moe_up_c<4>(grid, s, d, L, hidden, ll, h, ids, w, tbl, err);
+    if (cpl == 1) moe_up_c<1>(grid, iters > 1, s, d, L, hidden, ll, h, ids, w, tbl, err);
+    else if (cpl == 2) moe_up_c<2>(grid, iters > 1, s, d, L, hidden, ll, h, ids, w, tbl, err);
+    else if (cpl <= 4) moe_up_c<4>(grid, iters > 1, s, d, L, hidden, ll, h, ids, w, tbl, err);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -796,18 +858,18 @@ hipError_t launch_down_combine(const MoeDims& d, const ExpertPtrs* tbl, const fl
     while (ppl < 4 && (npairs + 64u * ppl - 1) / (64u * ppl) > DOWN_MAX_WAVES) ppl *= 2;
     const uint32_t nw = (npairs + 64u * ppl - 1) / (64u * ppl);
     if (nw > DOWN_MAX_WAVES || d.D % DOWN_RB) return hipErrorInvalidValue;
-    dim3 grid(d.D / DOWN_RB, n_tok), block(nw * WAVE);
-    switch (ppl) {
-        case 1:
-            launch_kernel(k_down_combine<1>, grid, block, s, d, tbl, h, w, hidden, ll);
-            break;
-        case 2:
-            launch_kernel(k_down_combine<2>, grid, block, s, d, tbl, h, w, hidden, ll);
-            break;
-        default:
-            launch_kernel(k_down_combine<4>, grid, block, s, d, tbl, h, w, hidden, ll);
-            break;
-    }
+    // Several row blocks a block, with one pair a lane (the next rows' registers),
+    // once the waves outnumber what the chip holds at three a SIMD: h is converted
+    // once for all of them (11 tokens of the 30B shape 22.4 -> 20.1 us, of
+    // the 235B shape 69.6 -> 63.4; for two a SIMD 22.1 and 84).
+    const uint32_t row_blocks = d.D / DOWN_RB;
+    const uint32_t most = ppl == 1 ? std::max(1u, 3072u / (nw * n_tok)) : row_blocks;
+    const uint32_t iters = (row_blocks + most - 1) / most;
+    const dim3 grid((row_blocks + iters - 1) / iters, n_tok), block(nw * WAVE);
+    if (ppl == 1 && iters > 1) launch_kernel(k_down_combine<1, true>, grid, block, s, d, tbl, h, w, hidden, ll);
+    else if (ppl == 1) launch_kernel(k_down_combine<1, false>, grid, block, s, d, tbl, h, w, hidden, ll);
+    else if (ppl == 2) launch_kernel(k_down_combine<2, false>, grid, block, s, d, tbl, h, w, hidden, ll);
+    else launch_kernel(k_down_combine<4, false>, grid, block, s, d, tbl, h, w, hidden, ll);
     return hipGetLastError();
 }
 

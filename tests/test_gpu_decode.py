@@ -89,3 +89,32 @@ def test_graph_replay_matches_eager(ctx, oracle):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(buf, eager)
+
+
+@pytest.mark.parametrize("D,E,K,I,Ts", [
+    (2048, 128, 8, 768, (2, 5, 11, 24)),    # one, two, four and ten row blocks a wave
+    (4096, 128, 8, 1536, (5,)),             # two chunks a lane: rows loaded block by block
+    (1280, 60, 6, 704, (11, 40)),           # an odd number of row blocks
+    (512, 200, 6, 256, (90,)),              # more than 128 experts
+])
+def test_batch_equals_single_calls(ctx, D, E, K, I, Ts):
+    """Each token of a batch equals its own two-launch call bit for bit,
+    however many row blocks a wave of the batch takes."""
+    import smoe_amd
+    layer = Layer(ctx, D, E, K, I, layer_id=D + I + 5, host=False)
+    for T in Ts:
+        print(f"case D={D} E={E} K={K} I={I} T={T}", flush=True)
+        x = hidden_states(ctx, T, D, 300)
+        batch, one = x.clone(), x.clone()
+        ids = torch.zeros((2, T, K), dtype=torch.int32, device="cuda")
+        w = torch.zeros((2, T, K), dtype=torch.float32, device="cuda")
+        ctx.moe_decode(layer.shape, layer.layer, batch.data_ptr(), T, ids[0].data_ptr(), w[0].data_ptr())
+        ctx.set_decode_engine(smoe_amd.DECODE_SPLIT)
+        try:
+            for t in range(T):
+                ctx.moe_decode(layer.shape, layer.layer, one[t].data_ptr(), 1, ids[1, t].data_ptr(), w[1, t].data_ptr())
+        finally:
+            ctx.set_decode_engine(smoe_amd.DECODE_CHAIN)
+        ctx.synchronize()
+        assert torch.equal(ids[0], ids[1]) and torch.equal(w[0], w[1])
+        assert torch.equal(batch, one) and not torch.equal(batch, x)
