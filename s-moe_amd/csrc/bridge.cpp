@@ -54,7 +54,7 @@ struct PrefillScratch {
     uint32_t* ids = nullptr;        // [T x K]
     float* w = nullptr;             // [T x K]
     uint32_t* offsets = nullptr;    // [E + 1]
-    uint32_t* units = nullptr;      // [2 + max_units] grouped GEMM work list
+    uint4* units = nullptr;         // [unit_slots] grouped GEMM work list
     uint32_t* seg_cnt = nullptr;    // [perm_segments x E] pairs per segment
     uint32_t* pairs = nullptr;      // [P] sorted pair ids
     float* h = nullptr;             // [P x I]
@@ -301,7 +301,7 @@ int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T)
     const bool ok = dalloc(ctx, &n.x_hi, T_ * n.D) &&
                     dalloc(ctx, &n.x_lo, T_ * n.D) && dalloc(ctx, &n.x_sc, T_) &&
                     dalloc(ctx, &n.ids, P) && dalloc(ctx, &n.w, P) && dalloc(ctx, &n.offsets, size_t(n.E) + 1) &&
-                    dalloc(ctx, &n.units, 2 + size_t(smoe::max_units(P, n.E, ~0u))) &&
+                    dalloc(ctx, &n.units, size_t(smoe::unit_slots(P, n.E, ~0u))) &&
                     dalloc(ctx, &n.seg_cnt, size_t(smoe::perm_segments(P, n.E)) * n.E) &&
                     dalloc(ctx, &n.pairs, P) && dalloc(ctx, &n.h, P * n.I) && dalloc(ctx, &n.h_hi, P * n.I) &&
                     dalloc(ctx, &n.h_lo, P * n.I) && dalloc(ctx, &n.h_sc, P) && dalloc(ctx, &n.y, P * n.D) &&
@@ -1070,12 +1070,12 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
                 return smoe::launch_permute_seg(ids, P, d.E, offs, s.pairs, s.units, few, s.seg_cnt, ctx->d_err, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_GATE_UP, "grouped_gate_up", [&] {
-                return smoe::launch_grouped_gate_up(d, L, P, few, offs, s.units, s.pairs, s.x_hi, s.x_lo, s.x_sc, s.h, st);
+                return smoe::launch_grouped_gate_up(d, L, P, few, s.units, s.pairs, s.x_hi, s.x_lo, s.x_sc, s.h, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SPLIT, "split(h)",
                    [&] { return smoe::launch_split_rows(s.h, P, d.I, s.h_hi, s.h_lo, s.h_sc, st); }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_DOWN, "grouped_down", [&] {
-                return smoe::launch_grouped_down(d, L, P, few, offs, s.units, s.pairs, s.h_hi, s.h_lo, s.h_sc, s.y, st);
+                return smoe::launch_grouped_down(d, L, P, few, s.units, s.pairs, s.h_hi, s.h_lo, s.h_sc, s.y, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SCATTER, "combine",
                    [&] { return smoe::launch_combine_pairs(s.y, w, T, d.K, d.D, hv, st); }))

@@ -228,13 +228,18 @@ hipError_t launch_split_rows(const float* src, uint32_t rows, uint32_t cols, uin
                              float* scale, hipStream_t s);
 // Stable counting sort of the P pairs by expert: offsets [E+1],
 // sorted_pairs [P] (pair = token * K + rank); sorted_tokens, sorted_w,
-// union_ids [E], union_size [1] optional (nullptr).  units [2 + max_units(P,
-// E)] optional: the grouped GEMMs' work list of (expert, pass) units, of up to
+// union_ids [E], union_size [1] optional (nullptr).  units [unit_slots(P,
+// E, few_units)] optional: the grouped GEMMs' work list of (expert, pass) units, of up to
 // 64 pairs, or up to 32 where fewer than few_units would result.  Bad ids set err bit 1.
 constexpr size_t PERMUTE_MAX_LDS = 48 * 1024;
 constexpr uint32_t max_units(uint32_t P, uint32_t E, uint32_t few_units)
 {
     return P / (P / 64 >= few_units ? 64 : 32) + (E < P ? E : P);
+}
+// records of the work list: eight XCDs' shares
+constexpr uint32_t unit_slots(uint32_t P, uint32_t E, uint32_t few_units)
+{
+    return (max_units(P, E, few_units) + 7u) / 8u * 8u;
 }
 // The list length below which units are of up to 32 pairs: 512 gate/up blocks,
 // one round of two per CU.  64 Zipf-routed tokens of the 30B shape (45 experts):
@@ -244,20 +249,20 @@ constexpr uint32_t few_units(const MoeDims& d) { return 512u / ((d.I + 127u) / 1
 size_t permute_lds_bytes(uint32_t P, uint32_t E);
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
-                          uint32_t* union_size, uint32_t* units, uint32_t few_units, uint32_t* err, hipStream_t s);
+                          uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s);
 // The same offsets, sorted pairs and units in segments, one workgroup each, for
 // any P (seg_cnt [perm_segments(P, E) x E]).
 uint32_t perm_segments(uint32_t P, uint32_t E);
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
-                              uint32_t* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
+                              uint4* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):
 // h [P x I] = silu(x G^T) * (x U^T); y [P x D] = h Dn^T, over the permute's
 // work list.
-hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
-                                  const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* x_hi,
+hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+                                  const uint32_t* sorted_pairs, const uint16_t* x_hi,
                                   const uint16_t* x_lo, const float* x_scale, float* h, hipStream_t s);
-hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
-                               const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* h_hi,
+hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+                               const uint32_t* sorted_pairs, const uint16_t* h_hi,
                                const uint16_t* h_lo, const float* h_scale, float* y, hipStream_t s);
 // hidden[t] += sum_r w[t][r] * y[t*K + r] (rank order).
 hipError_t launch_combine_pairs(const float* y, const float* w, uint32_t T, uint32_t K, uint32_t D, float* hidden,

@@ -477,10 +477,14 @@ void k_split_rows(const float* __restrict__ src, uint32_t rows, uint32_t cols, u
 // ---------------------------------------------------------------------------
 constexpr int PERM_THREADS = 1024;
 
-// The grouped GEMMs' work list: units[0] = the number U of units, units[1] = the
-// most rows of a unit (cap: 64 or 32), units[2 + u] = expert | pass << 16,
-// experts ascending, passes ascending.  An expert's M pairs take as few passes
-// as cap allows, of equal numbers of 16-row tiles.
+// The grouped GEMMs' work list: units of up to cap (64 or 32) pairs of one
+// expert, experts ascending, an expert's M pairs in as few units as cap allows,
+// of equal numbers of 16-row tiles.  XCD x takes the x-th eighth of the list
+// (block id mod 8 is a block's XCD), so an expert's blocks run together on one
+// XCD and share its activation rows and, between its units, its weights in the
+// L2.  The record of the j-th unit of XCD x stands at 8 j + x, all 8 slots of
+// every j the grid covers are written (no pairs: no unit), and a record holds
+// all that a block needs: one scalar load, then the pairs and the weights.
 __device__ __forceinline__ uint32_t unit_count(uint32_t M, uint32_t cap) { return (M + cap - 1u) / cap; }
 __device__ __forceinline__ uint32_t unit_rows(uint32_t M, uint32_t cap)
 {
@@ -533,16 +537,26 @@ __device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, ui
     }
 }
 
-// a workgroup writes the work list (s_unit, cap: scan_units)
-__device__ __forceinline__ void write_units(const uint32_t* s_unit, uint32_t E, uint32_t cap, uint32_t* units)
+// a workgroup writes the n_slots records (s_off, s_unit, cap: scan_units):
+// x = expert | rows of a pass << 16, y = first pair, z = pairs
+__device__ __forceinline__ void write_units(const uint32_t* s_off, const uint32_t* s_unit, uint32_t E, uint32_t cap,
+                                            uint4* units, uint32_t n_slots)
 {
-    for (uint32_t e = threadIdx.x; e < E; e += blockDim.x) {
-        const uint32_t u0 = s_unit[e], n = s_unit[e + 1] - u0;
-        for (uint32_t i = 0; i < n; ++i) units[2 + u0 + i] = e | (i << 16);
-    }
-    if (threadIdx.x == 0) {
-        units[0] = s_unit[E];
-        units[1] = cap;
+    const uint32_t U = s_unit[E], per = (U + 7u) >> 3;
+    for (uint32_t i = threadIdx.x; i < n_slots; i += blockDim.x) {
+        const uint32_t j = i >> 3, u = (i & 7u) * per + j;
+        uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+        if (j < per && u < U) {
+            uint32_t e = 0, hi = E;              // the expert: s_unit[e] <= u < s_unit[e + 1]
+            while (hi - e > 1) {
+                const uint32_t mid = (e + hi) >> 1;
+                if (s_unit[mid] <= u) e = mid;
+                else hi = mid;
+            }
+            const uint32_t M = s_off[e + 1] - s_off[e], rows = unit_rows(M, cap), m0 = (u - s_unit[e]) * rows;
+            rec = make_uint4(e | (rows << 16), s_off[e] + m0, min(M - m0, rows), 0u);
+        }
+        units[i] = rec;
     }
 }
 
@@ -550,7 +564,7 @@ __global__ __launch_bounds__(PERM_THREADS)
 void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, uint32_t P, uint32_t K, uint32_t E,
                uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs,
                uint32_t* __restrict__ sorted_tokens, float* __restrict__ sorted_w, uint32_t* __restrict__ union_ids,
-               uint32_t* __restrict__ union_size, uint32_t* __restrict__ units, uint32_t few_units,
+               uint32_t* __restrict__ union_size, uint4* __restrict__ units, uint32_t n_slots, uint32_t few_units,
                uint32_t* __restrict__ err)
 {
     extern __shared__ uint32_t s_mem[];
@@ -674,7 +688,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
         for (uint32_t e = 0; e < E; ++e) n += s_tot[e] != 0;
         *union_size = n;
     }
-    if (units) write_units(s_unit, E, s_cap, units);
+    if (units) write_units(s_off, s_unit, E, s_cap, units, n_slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -710,8 +724,8 @@ void k_perm_count(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, uint
 
 __global__ __launch_bounds__(PERM_THREADS)
 void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, const uint32_t* __restrict__ seg_cnt,
-                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs, uint32_t* __restrict__ units,
-                    uint32_t few_units)
+                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs, uint4* __restrict__ units,
+                    uint32_t n_slots, uint32_t few_units)
 {
     extern __shared__ uint32_t s_mem[];
     __shared__ uint32_t s_cap;
@@ -790,7 +804,7 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
     }
     if (seg == 0) {
         for (uint32_t e = threadIdx.x; e <= E; e += PERM_THREADS) offsets[e] = s_off[e];
-        write_units(s_unit, E, s_cap, units);
+        write_units(s_off, s_unit, E, s_cap, units, n_slots);
     }
 }
 
@@ -880,6 +894,13 @@ __device__ __forceinline__ void vm_wait()
     static_assert(N >= 0 && N < 64, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
+// the same, and this wave's LDS reads are done
+template <int N>
+__device__ __forceinline__ void vm_lds_wait()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
+}
 __device__ __forceinline__ void mem_fence_compiler() { asm volatile("" ::: "memory"); }
 __device__ __forceinline__ void gm_barrier()
 {
@@ -890,7 +911,7 @@ __device__ __forceinline__ void gm_barrier()
 
 template <bool GATE_UP, int MS>
 __device__ __forceinline__ void grouped_mm_expert(
-    const MoeDims& d, const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t mb, uint32_t M,
+    const MoeDims& d, const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t M,
     const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi, const uint16_t* __restrict__ a_lo,
     const float* __restrict__ a_scale, uint32_t a_row_div, float* __restrict__ out, uint32_t n_dim, uint32_t k_dim,
     GmW& w0, GmW& w1, GmW& w2, GmW& w3, GmA& a0, GmA& a1, GmA& a2, GmA& a3, uint32_t (&s_row)[GM_PASS],
@@ -944,154 +965,136 @@ __device__ __forceinline__ void grouped_mm_expert(
 #pragma unroll
         for (int pl = 0; pl < 2; ++pl) aoff[stp][pl] = m16 * 256 + 16 * ((8 * pl + 2 * q + stp) ^ m16);
 
-    for (uint32_t m0 = mb; m0 < M; m0 += PASS) {
-        __syncthreads();
-        if (threadIdx.x < PASS) {
-            const uint32_t p = sorted_pairs[base + min(m0 + threadIdx.x, M - 1)];
-            s_pair[threadIdx.x] = p;
-            s_row[threadIdx.x] = p / a_row_div;
-        }
-        __syncthreads();
-        const uint16_t* a_src[AN];
+    if (threadIdx.x < PASS) {
+        const uint32_t p = sorted_pairs[base + min(threadIdx.x, M - 1)];
+        s_pair[threadIdx.x] = p;
+        s_row[threadIdx.x] = p / a_row_div;
+    }
+    __syncthreads();
+    const uint16_t* a_src[AN];
 #pragma unroll
-        for (int u = 0; u < AN; ++u) {
-            const uint32_t r = wv * 4 * AN + 4 * u + (lane >> 4);
-            const uint32_t x = (lane & 15) ^ (r & 15);
-            const uint32_t srow = s_row[min(r, static_cast<uint32_t>(PASS - 1))];
-            a_src[u] = ((x >> 3) ? a_lo : a_hi) + static_cast<size_t>(srow) * k_dim + 8 * (x & 7);
-        }
-        auto issue_a = [&](GmA& S, uint32_t c) {
+    for (int u = 0; u < AN; ++u) {
+        const uint32_t r = wv * 4 * AN + 4 * u + (lane >> 4);
+        const uint32_t x = (lane & 15) ^ (r & 15);
+        const uint32_t srow = s_row[min(r, static_cast<uint32_t>(PASS - 1))];
+        a_src[u] = ((x >> 3) ? a_lo : a_hi) + static_cast<size_t>(srow) * k_dim + 8 * (x & 7);
+    }
+    auto issue_a = [&](GmA& S, uint32_t c) {
 #pragma unroll
-            for (int u = 0; u < AN; ++u)
-                __builtin_amdgcn_global_load_lds(a_src[u] + c * 64, SMOE_LDS_AS(&S.a[(wv * 4 * AN + 4 * u) * 256]), 16,
-                                                 0, 0);
-        };
+        for (int u = 0; u < AN; ++u)
+            __builtin_amdgcn_global_load_lds(a_src[u] + c * 64, SMOE_LDS_AS(&S.a[(wv * 4 * AN + 4 * u) * 256]), 16,
+                                             0, 0);
+    };
 
-        f32x4_t acc[MS][2];
+    f32x4_t acc[MS][2];
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms)
+    for (int ms = 0; ms < MS; ++ms)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[ms][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 2; ++j) acc[ms][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-        // Issue order of the loop: body c issues the activation stage c + 3 and then the
-        // weight stage c / 2 + 3 (if c is even).  The prologue replays bodies -6 .. -1.
-        const uint32_t NWS = (G + 1) / 2;        // weight stages
-        if (0 < NWS) issue_w(w0, 0);
-        if (1 < NWS) issue_w(w1, 1);
-        if (0 < G) issue_a(a0, 0);
-        if (1 < G) issue_a(a1, 1);
-        if (2 < NWS) issue_w(w2, 2);
-        if (2 < G) issue_a(a2, 2);
+    // Issue order of the loop: body c issues the activation stage c + 3 and then the
+    // weight stage c / 2 + 3 (if c is even).  The prologue replays bodies -6 .. -1.
+    const uint32_t NWS = (G + 1) / 2;        // weight stages
+    if (0 < NWS) issue_w(w0, 0);
+    if (1 < NWS) issue_w(w1, 1);
+    if (0 < G) issue_a(a0, 0);
+    if (1 < G) issue_a(a1, 1);
+    if (2 < NWS) issue_w(w2, 2);
+    if (2 < G) issue_a(a2, 2);
+    mem_fence_compiler();
+
+    auto body = [&](uint32_t c, GmW& W, uint32_t g, GmW& WN, GmA& A, GmA& AN_) {
+        // A(c) was the first load of body c - 3; after it came the weight stage of body
+        // c - 3 when c - 3 is even, A(c + 1), A(c + 2) and the weight stage of the even
+        // one of bodies c - 2, c - 1 ((c + 4 + (c & 1)) / 2, the later of the two).  When
+        // all of those were issued, 2 AN + 3 (even c) or 2 AN + 6 (odd c) loads may still
+        // be pending; near the end fewer were, and the wait covers everything.
+        if (c + 2 < G && (c + 4 + (c & 1)) / 2 < NWS) {
+            if (g) vm_wait<2 * AN + 6>();
+            else vm_wait<2 * AN + 3>();
+        } else {
+            vm_wait<0>();
+        }
+        gm_barrier();
+        if (c + 3 < G) issue_a(AN_, c + 3);
+        if (g == 0 && c / 2 + 3 < NWS) issue_w(WN, c / 2 + 3);
         mem_fence_compiler();
-
-        auto body = [&](uint32_t c, GmW& W, uint32_t g, GmW& WN, GmA& A, GmA& AN_) {
-            // A(c) was the first load of body c - 3; after it came the weight stage of body
-            // c - 3 when c - 3 is even, A(c + 1), A(c + 2) and the weight stage of the even
-            // one of bodies c - 2, c - 1 ((c + 4 + (c & 1)) / 2, the later of the two).  When
-            // all of those were issued, 2 AN + 3 (even c) or 2 AN + 6 (odd c) loads may still
-            // be pending; near the end fewer were, and the wait covers everything.
-            if (c + 2 < G && (c + 4 + (c & 1)) / 2 < NWS) {
-                if (g) vm_wait<2 * AN + 6>();
-                else vm_wait<2 * AN + 3>();
-            } else {
-                vm_wait<0>();
-            }
-            gm_barrier();
-            if (c + 3 < G) issue_a(AN_, c + 3);
-            if (g == 0 && c / 2 + 3 < NWS) issue_w(WN, c / 2 + 3);
-            mem_fence_compiler();
-            half8_t b[2][2];
-            float sc[2];
+        half8_t b[2][2];
+        float sc[2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const uint2 v = *reinterpret_cast<const uint2*>(&W.w[boff[g] + 1024 * j]);
-                b[j][0] = q4_codes_to_f16(v.x);
-                b[j][1] = q4_codes_to_f16(v.y);
-                sc[j] = f16_bits_to_f32(static_cast<uint16_t>(W.sc[wv * 64 + 32 * g + 16 * j + m16]));
-            }
-#pragma unroll
-            for (int ms = 0; ms < MS; ++ms) {
-                half8_t xa[2][2];
-#pragma unroll
-                for (int stp = 0; stp < 2; ++stp)
-#pragma unroll
-                    for (int pl = 0; pl < 2; ++pl) xa[stp][pl] = lds_half8(A.a + ms * 4096 + aoff[stp][pl]);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    f32x4_t t = {0.f, 0.f, 0.f, 0.f};
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][0], b[j][0], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][1], b[j][0], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][0], b[j][1], t, 0, 0, 0);
-                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][1], b[j][1], t, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[i], acc[ms][j][i]);
-                }
-            }
-            mem_fence_compiler();
-        };
-        for (uint32_t c = 0; c < G; c += 8) {
-            body(c, w0, 0, w3, a0, a3);
-            if (c + 1 < G) body(c + 1, w0, 1, w3, a1, a0);
-            if (c + 2 < G) body(c + 2, w1, 0, w0, a2, a1);
-            if (c + 3 < G) body(c + 3, w1, 1, w0, a3, a2);
-            if (c + 4 < G) body(c + 4, w2, 0, w1, a0, a3);
-            if (c + 5 < G) body(c + 5, w2, 1, w1, a1, a0);
-            if (c + 6 < G) body(c + 6, w3, 0, w2, a2, a1);
-            if (c + 7 < G) body(c + 7, w3, 1, w2, a3, a2);
+        for (int j = 0; j < 2; ++j) {
+            const uint2 v = *reinterpret_cast<const uint2*>(&W.w[boff[g] + 1024 * j]);
+            b[j][0] = q4_codes_to_f16(v.x);
+            b[j][1] = q4_codes_to_f16(v.y);
+            sc[j] = f16_bits_to_f32(static_cast<uint16_t>(W.sc[wv * 64 + 32 * g + 16 * j + m16]));
         }
 #pragma unroll
         for (int ms = 0; ms < MS; ++ms) {
+            half8_t xa[2][2];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t m = 16 * ms + 4 * q + i;
-                if (m0 + m >= M) continue;
-                const float rs = a_scale[s_row[m]] * (8.0f / 15.0f);   // weights are (2c - 15) / 8
-                float* o = out + static_cast<size_t>(s_pair[m]) * n_dim;
-                if (GATE_UP) {
-                    const uint32_t n = tile * GM_ROWS_GU + 16 * wv + m16;
-                    if (n < n_dim) {
-                        const float v0 = acc[ms][0][i] * rs, v1 = acc[ms][1][i] * rs;
-                        o[n] = (v0 * (1.0f / (1.0f + expf(-v0)))) * v1;
-                    }
-                } else {
+            for (int stp = 0; stp < 2; ++stp)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const uint32_t n = tile * GM_ROWS_DN + 32 * wv + 16 * j + m16;
-                        if (n < n_dim) o[n] = acc[ms][j][i] * rs;
-                    }
+                for (int pl = 0; pl < 2; ++pl) xa[stp][pl] = lds_half8(A.a + ms * 4096 + aoff[stp][pl]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                f32x4_t t = {0.f, 0.f, 0.f, 0.f};
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][0], b[j][0], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[0][1], b[j][0], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][0], b[j][1], t, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[1][1], b[j][1], t, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[i], acc[ms][j][i]);
+            }
+        }
+        mem_fence_compiler();
+    };
+    for (uint32_t c = 0; c < G; c += 8) {
+        body(c, w0, 0, w3, a0, a3);
+        if (c + 1 < G) body(c + 1, w0, 1, w3, a1, a0);
+        if (c + 2 < G) body(c + 2, w1, 0, w0, a2, a1);
+        if (c + 3 < G) body(c + 3, w1, 1, w0, a3, a2);
+        if (c + 4 < G) body(c + 4, w2, 0, w1, a0, a3);
+        if (c + 5 < G) body(c + 5, w2, 1, w1, a1, a0);
+        if (c + 6 < G) body(c + 6, w3, 0, w2, a2, a1);
+        if (c + 7 < G) body(c + 7, w3, 1, w2, a3, a2);
+    }
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t m = 16 * ms + 4 * q + i;
+            if (m >= M) continue;
+            const float rs = a_scale[s_row[m]] * (8.0f / 15.0f);   // weights are (2c - 15) / 8
+            float* o = out + static_cast<size_t>(s_pair[m]) * n_dim;
+            if (GATE_UP) {
+                const uint32_t n = tile * GM_ROWS_GU + 16 * wv + m16;
+                if (n < n_dim) {
+                    const float v0 = acc[ms][0][i] * rs, v1 = acc[ms][1][i] * rs;
+                    o[n] = (v0 * (1.0f / (1.0f + expf(-v0)))) * v1;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t n = tile * GM_ROWS_DN + 32 * wv + 16 * j + m16;
+                    if (n < n_dim) o[n] = acc[ms][j][i] * rs;
                 }
             }
         }
     }
 }
 
-// block b of a grid over units x n_tiles -> unit and tile: XCD b mod 8 (the
-// round-robin deal) takes a contiguous eighth of the list, tile by tile of a
-// unit, so an expert's blocks run together on one XCD, sharing its activation
-// rows and, between its passes, its weights in the L2.
-__device__ __forceinline__ bool unit_of_block(const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ units,
-                                              uint32_t n_tiles, uint32_t& e, uint32_t& tile, uint32_t& base,
-                                              uint32_t& mb, uint32_t& me, uint32_t& rows)
+// block b of a grid over units x n_tiles -> the unit's record (its own slot,
+// see write_units) and the tile: XCD b mod 8, tile by tile of a unit
+__device__ __forceinline__ uint4 unit_of_block(const uint4* __restrict__ units, uint32_t n_tiles, uint32_t& tile)
 {
-    const uint32_t U = units[0], cap = units[1], per = (U + 7u) >> 3;
-    const uint32_t b = blockIdx.x, xcd = b & 7u, jb = b >> 3;
-    const uint32_t j = jb / n_tiles, u = xcd * per + j;
+    const uint32_t b = blockIdx.x, jb = b >> 3;
     tile = jb % n_tiles;
-    if (j >= per || u >= U) return false;
-    const uint32_t word = units[2 + u], pass = word >> 16;
-    e = word & 0xFFFFu;
-    base = offsets[e];
-    const uint32_t M = offsets[e + 1] - base;
-    rows = unit_rows(M, cap);
-    mb = pass * rows;
-    me = min(M, mb + rows);
-    return true;
+    return units[8u * (jb / n_tiles) + (b & 7u)];
 }
 
 template <bool GATE_UP>
 __global__ __launch_bounds__(GM_WAVES * WAVE, 1)
-void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
-                  const uint32_t* __restrict__ units, const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
+void k_grouped_mm(MoeDims d, LayerDesc L, const uint4* __restrict__ units, const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
                   const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale, uint32_t a_row_div,
                   float* __restrict__ out, uint32_t n_dim, uint32_t k_dim, uint32_t n_tiles)
 {
@@ -1099,10 +1102,12 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
     __shared__ __align__(16) GmA a0, a1, a2, a3;
     __shared__ uint32_t s_row[GM_PASS];
     __shared__ uint32_t s_pair[GM_PASS];
-    uint32_t e, tile, base, mb, me, rows;
-    if (!unit_of_block(offsets, units, n_tiles, e, tile, base, mb, me, rows)) return;
+    uint32_t tile;
+    const uint4 rec = unit_of_block(units, n_tiles, tile);
+    if (rec.z == 0) return;
+    const uint32_t rows = rec.x >> 16;
     auto go = [&](auto ms) {
-        grouped_mm_expert<GATE_UP, decltype(ms)::value>(d, L, e, tile, base, mb, me, sorted_pairs, a_hi, a_lo, a_scale,
+        grouped_mm_expert<GATE_UP, decltype(ms)::value>(d, L, rec.x & 0xFFFFu, tile, rec.y, rec.z, sorted_pairs, a_hi, a_lo, a_scale,
                                                         a_row_div, out, n_dim, k_dim, w0, w1, w2, w3, a0, a1, a2, a3,
                                                         s_row, s_pair);
     };
@@ -1121,15 +1126,23 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
 // blocks of a CU pass their barriers independently, so one block's MFMAs
 // overlap the other's conversion.  Needs an even number of groups (a stage's
 // two scales are one dword).
-//   stage    two 64-column groups; while one is computed the next one's
-//            weights are on their way into registers and its activation rows
-//            into the other LDS buffer, one wait and one barrier per stage;
-//   weights  subtile j: lane l loads row l & 15, bytes 16 (l >> 4) .. + 15 of
-//            the stage's 64; v_permlane16_swap and v_permlane32_swap then
-//            leave quad q = l >> 4, MFMA step s the 8-column unit 2 q + s of
-//            either group, as in k_grouped_mm;
+//   stage    two 64-column groups; gd_depth stages are in flight while one is
+//            computed: their codes in registers, their activation rows in a ring
+//            in LDS, one counted wait and one barrier per stage;
+//   weights  up to two m-tiles a unit (HBM-bound): a load takes 128 bytes of 8
+//            rows, the codes of two stages, marked non-temporal (each weight
+//            line is read once).  Whole lines set the stream's rate: the loads
+//            alone run 805 MB of gate/up in 153 us as 64 bytes of 16 rows (194
+//            non-temporal), 141 as whole lines, 125 (6.4 TB/s) as whole lines
+//            non-temporal.  Lane l loads row l & 7, unit l >> 3; a rotation by
+//            8 in each 16 lanes, v_permlane32_swap and v_permlane16_swap leave
+//            quad q = l >> 4, MFMA step s the 8-column unit 4 s + q of each
+//            group, row l & 15.  More m-tiles (bound by the matrix cores; their
+//            registers hold fewer stages): 64 bytes of 16 rows, lane l row
+//            l & 15, bytes 16 (l >> 4) .. + 15, and the two swaps leave the
+//            same units: a pair's sums do not depend on its unit's size;
 //   acts     [plane][row][16 units of 8 columns], unit x of row r in slot
-//            x ^ (r & 15): conflict-free for the fragment reads (units 2 q + s
+//            x ^ (r & 15): conflict-free for the fragment reads (units 4 s + q
 //            of rows 0 .. 15), filled by direct loads (4 rows x 256 bytes each)
 //            issued from inline asm: the compiler does not track them, so it
 //            adds no waits of its own;
@@ -1140,20 +1153,23 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets,
 //            interleaved, the next m-tile's fragments are read during them, and
 //            the sums are scaled into the accumulators during the next
 //            m-tile's chains.
-// Up to two m-tiles a pass (HBM-bound: few pairs per weight byte) a stage is
-// two such steps, so a CU has 64 KB of weights in flight; with more m-tiles
-// LDS and registers hold one.  Measured against the kernels before it (weights
-// of gate/up through LDS, 8 waves and one block per CU; passes of at most 736
-// tokens): 4096 tokens of the 30B shape gate/up 700 -> 407 us (1.05 PFLOP/s
-// of f16 products; a library f16 GEMM reaches 1.19 on the same card), down 407
-// -> 243; 512 tokens gate/up 97 -> 88, down 54 -> 51; 64 tokens of the 235B
-// shape gate/up 248 -> 195 (4.4 TB/s), down 125 -> 113.  Three blocks per CU with 168
-// registers: no faster (spills).
+// Nothing stands between a block's start and its weights but its record; the
+// pairs, the rows' addresses and their scales stay in registers.
+// Measured against the kernels before it (weights of gate/up through LDS, 8
+// waves and one block per CU; passes of at most 736 tokens): 4096 tokens of the
+// 30B shape gate/up 700 -> 396 us (1.08 PFLOP/s of f16 products; a library f16
+// GEMM reaches 1.19 on the same card), down 407 -> 229; 512 tokens gate/up 97 ->
+// 82, down 54 -> 45; 64 tokens of the 235B shape gate/up 248 -> 186 (4.6 TB/s;
+// one stage in flight and 64-byte loads: 202), down 125 -> 106 (115).  Three
+// blocks per CU with 168 registers: no faster (spills).
 // ---------------------------------------------------------------------------
 constexpr int GD_WAVES = 4;
 constexpr int GD_SUB = 4;                                  // 16-row subtiles a wave
 constexpr uint32_t GD_ROWS = 16 * GD_SUB * GD_WAVES;       // weight rows per block
-constexpr uint32_t GD_STAGE = GM_PASS * 512;               // bytes of an activation stage of 64 rows
+constexpr int GD_NT = 2;                                   // the loads' non-temporal bit
+constexpr uint32_t GD_LDS = 80 * 1024;                     // the activation ring: half of a CU's LDS
+// stages in flight: what the ring (DP + 1 stages of 8 KB an m-tile) and the registers hold
+constexpr int gd_depth(int ms) { return ms <= 2 ? 4 : ms == 3 ? 2 : 1; }
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p)
 {
@@ -1171,218 +1187,291 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t l
                  : "memory", "m0");
 }
 
-// Pairs [mb, me) of expert e (passes of 16 MS), one tile of GD_ROWS weight rows.
+// The np <= 16 MS pairs from sorted_pairs[first] on, all of expert e; one tile of GD_ROWS weight rows.
 template <bool GATE_UP, int MS>
 __device__ __forceinline__ void grouped_reg_expert(
-    const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t base, uint32_t mb, uint32_t me,
+    const LayerDesc& L, uint32_t e, uint32_t tile, uint32_t first, uint32_t np,
     const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi, const uint16_t* __restrict__ a_lo,
     const float* __restrict__ a_scale, uint32_t a_row_div, float* __restrict__ out, uint32_t n_dim, uint32_t k_dim,
-    uint8_t* abuf, uint32_t (&s_row)[GM_PASS], uint32_t (&s_pair)[GM_PASS])
+    uint8_t* abuf)
 {
     constexpr int PASS = 16 * MS;
-    constexpr int NH = MS <= 2 ? 2 : 1;          // pairs of groups in a stage
-    constexpr uint32_t PLANE = PASS * 256, HALF = 2 * PLANE, STAGE = NH * HALF;
-    static_assert(STAGE <= GD_STAGE, "a stage fits its buffer");
+    constexpr int DP = gd_depth(MS);             // stages in flight
+    // QUAD: the codes of two stages in one load, 128 bytes of 8 rows (a whole
+    // line a row: the stream's rate hangs on it); else 64 bytes of 16 rows
+    constexpr bool QUAD = DP == 4;
+    constexpr int WL = QUAD ? 2 * GD_SUB : GD_SUB, WD = QUAD ? DP / 2 : DP;
+    constexpr uint32_t PLANE = PASS * 256, STAGE = 2 * PLANE;
+    static_assert((DP + 1) * STAGE <= GD_LDS, "the ring fits");
     const int lane = threadIdx.x & 63;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t G = k_dim >> 6, NHS = G / 2, NST = (NHS + NH - 1) / NH;
+    const uint32_t G = k_dim >> 6, NST = G / 2;
     const uint32_t m16 = lane & 15, q = lane >> 4;
+    const uint32_t pair = sorted_pairs[first + min(static_cast<uint32_t>(lane), np - 1)];
 
     // codes and scales through buffer resources: a scalar base and one offset
     // register a subtile (64-bit addresses took 16 registers more and spilled)
     const uint8_t* blob = L.experts + static_cast<size_t>(e) * L.stride;
     constexpr int NM = GATE_UP ? 2 : 1, SM = GD_SUB / NM;   // matrices, subtiles of each
-    __amdgpu_buffer_rsrc_t w_mat[NM], s_mat[NM];
+    const uint32_t w_bytes = n_dim * (k_dim >> 1);
+    const uint8_t* w_mat[NM];
+    __amdgpu_buffer_rsrc_t s_mat[NM];
 #pragma unroll
     for (int i = 0; i < NM; ++i) {
         const int o = GATE_UP ? 2 * i : 4;
-        w_mat[i] = weight_rsrc(blob + L.off[o], n_dim * (k_dim >> 1));
+        w_mat[i] = blob + L.off[o];
         s_mat[i] = weight_rsrc(blob + L.off[o + 1], n_dim * G * 2);
     }
-    // gate/up: subtiles 0, 1 are 32 gate rows, 2, 3 the same rows of up
-    const uint32_t row_w = tile * (GD_ROWS / NM) + 16 * SM * wv;
-    uint32_t w_off[SM];
+    // gate/up: subtiles 0, 1 are 32 gate rows, 2, 3 the same rows of up (n_dim is
+    // a multiple of 64: a subtile past the end is a repeat of the last one)
+    const uint32_t row_w = tile * (GD_ROWS / NM) + 16 * SM * wv, row_bytes = k_dim >> 1;
+    auto row_j = [&](int j) { return min(row_w + 16 * (j % SM), n_dim - 16); };
+    uint32_t w_off[SM];                          // QUAD: w_off[0] only, the subtile is a scalar offset
 #pragma unroll
-    for (int j = 0; j < SM; ++j) w_off[j] = min(row_w + 16 * j + m16, n_dim - 1) * (k_dim >> 1) + 16 * q;
+    for (int j = 0; j < SM; ++j)
+        w_off[j] = QUAD ? (lane & 7) * row_bytes + 16 * (lane >> 3) : (row_j(j) + m16) * row_bytes + 16 * q;
     // scales: lane l loads eight groups of the wave's row l (% 32) at once
     // (every load instruction costs the CU a request slot whatever its width:
     // one load per four pairs of groups instead of four per pair); the lanes
     // that use them fetch them across the wave
     const uint32_t s_off = min(row_w + (lane & (16 * SM - 1)), n_dim - 1) * G * 2;
-    u32x4_t wr[NH][GD_SUB];                      // the next stage's codes
     u32x4_t sc_next[NM], sc_cur[NM];             // scales of eight groups: the next ones, the current ones
-    auto issue_w = [&](uint32_t st) {
-#pragma unroll
-        for (int j = 0; j < GD_SUB; ++j)
-#pragma unroll
-            for (int h = 0; h < NH; ++h)
-                wr[h][j] = __builtin_amdgcn_raw_buffer_load_b128(w_mat[j / SM], w_off[j % SM],
-                                                                 64 * min(NH * st + h, NHS - 1), 0);
-    };
     auto issue_s = [&](uint32_t piece) {
 #pragma unroll
         for (int i = 0; i < NM; ++i) sc_next[i] = __builtin_amdgcn_raw_buffer_load_b128(s_mat[i], s_off, 16 * piece, 0);
     };
-    // fragment of group g, step s of this lane: 16 bytes at aoff[g][s] (m-tile ms: + 4096 ms; lo plane: + PLANE)
+    // (past the last stage the resource is empty: the load returns 0 and moves
+    // nothing, and every stage issues the same number of loads)
+    u32x4_t wr[WD][WL];                          // the codes in flight
+    auto issue_w = [&](u32x4_t (&W)[WL], uint32_t k) {
+        if constexpr (QUAD) {
+            const bool in = 2 * k < NST;
+            // (an odd last stage: both halves of the lanes load it)
+            const uint32_t off = 2 * k + 1 < NST ? w_off[0] : w_off[0] - 2 * (lane & 32);
+#pragma unroll
+            for (int j = 0; j < WL; ++j)
+                W[j] = __builtin_amdgcn_raw_buffer_load_b128(
+                    weight_rsrc(w_mat[j / 2 / SM], in ? w_bytes : 0u), off,
+                    in ? (row_j(j / 2) + 8 * (j & 1)) * row_bytes + 128 * k : 0u, GD_NT);
+        } else {
+            const bool in = k < NST;
+#pragma unroll
+            for (int j = 0; j < WL; ++j)
+                W[j] = __builtin_amdgcn_raw_buffer_load_b128(weight_rsrc(w_mat[j / SM], in ? w_bytes : 0u),
+                                                             w_off[j % SM], in ? 64 * k : 0u, 0);
+        }
+    };
+    issue_s(0);
+#pragma unroll
+    for (int i = 0; i < WD; ++i) issue_w(wr[i], i);
+
+    // lane l: the row of pair l of the unit, and its scale
+    const uint32_t arow = GATE_UP ? pair / a_row_div : pair;
+    const float ascale = a_scale[arow];
+    // activation fill: waves 0, 1 the hi plane, 2, 3 the lo plane, 2 MS loads of 4 rows each
+    const uint16_t* plane = wv >= 2 ? a_lo : a_hi;
+    const uint32_t row0 = (wv & 1) * 8 * MS;
+    uint32_t a_off[2 * MS];
+#pragma unroll
+    for (int u = 0; u < 2 * MS; ++u) {
+        const uint32_t r = row0 + 4 * u + q;
+        a_off[u] = (__builtin_amdgcn_ds_bpermute(4 * r, arow) * k_dim + 8 * (m16 ^ (r & 15))) * 2;
+    }
+    const uint32_t a_dst = lds_addr(abuf) + (wv >> 1) * PLANE + row0 * 256;
+    auto issue_a = [&](uint32_t slot, uint32_t st) {
+        const uint8_t* src = reinterpret_cast<const uint8_t*>(plane) + 256 * st;
+#pragma unroll
+        for (int u = 0; u < 2 * MS; ++u) dma16(src, a_off[u], a_dst + slot * STAGE + u * 1024);
+    };
+    mem_fence_compiler();
+#pragma unroll
+    for (int i = 0; i < DP; ++i)
+        if (static_cast<uint32_t>(i) < NST) issue_a(i, i);
+    mem_fence_compiler();
+
+    // fragment of group g, step s of this lane (unit 4 s + q): 16 bytes at aoff[g][s] (m-tile ms: + 4096 ms; lo plane: + PLANE)
     uint32_t aoff[2][2];
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int stp = 0; stp < 2; ++stp) aoff[g][stp] = m16 * 256 + 16 * ((8 * g + 2 * q + stp) ^ m16);
+        for (int stp = 0; stp < 2; ++stp)
+            aoff[g][stp] = m16 * 256 + 16 * ((8 * g + 4 * stp + q) ^ m16);
 
-    for (uint32_t m0 = mb; m0 < me; m0 += PASS) {
-        __syncthreads();
-        if (threadIdx.x < PASS) {
-            const uint32_t p = sorted_pairs[base + min(m0 + threadIdx.x, me - 1)];
-            s_pair[threadIdx.x] = p;
-            s_row[threadIdx.x] = GATE_UP ? p / a_row_div : p;
+    f32x4_t acc[MS][GD_SUB];
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+        for (int j = 0; j < GD_SUB; ++j) acc[ms][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    uint32_t slot = 0;                           // st % (DP + 1): the ring slot of stage st
+    uint32_t gw[QUAD ? 2 : 1][GD_SUB][2][2];     // [stage of a quad][subtile][group][MFMA step]
+    auto stage = [&](auto dc, uint32_t st) {
+        constexpr int D = decltype(dc)::value;   // st % DP
+        // What may still be pending when stage st's codes and rows are needed:
+        // what stages st - DP + 1 .. st - 1 issued, each its rows (2 MS loads;
+        // none past the end) before its codes.  The first DP stages' codes all
+        // went before their rows.
+        constexpr bool EVEN = !QUAD || D % 2 == 0;
+        constexpr int A_N = 2 * MS * (DP - 1), W_N = QUAD ? WL * (EVEN ? 1 : 2) : WL * (DP - 1);
+        if (st + DP > NST) {
+            if (st < DP) vm_lds_wait<0>();
+            else vm_lds_wait<W_N>();
+        } else if (st < DP) {
+            vm_lds_wait<A_N + (QUAD ? WL * ((D + 1) / 2) : WL * D)>();
+        } else {
+            vm_lds_wait<A_N + W_N>();
         }
-        __syncthreads();
-        // activation fill: waves 0, 1 the hi plane, 2, 3 the lo plane, 2 MS loads of 4 rows each
-        const uint16_t* plane = wv >= 2 ? a_lo : a_hi;
-        const uint32_t row0 = (wv & 1) * 8 * MS;
-        uint32_t a_off[2 * MS];
+        gm_barrier();
+        if constexpr (!QUAD) {
 #pragma unroll
-        for (int u = 0; u < 2 * MS; ++u) {
-            const uint32_t r = row0 + 4 * u + q;
-            a_off[u] = (s_row[r] * k_dim + 8 * (m16 ^ (r & 15))) * 2;
-        }
-        const uint32_t a_dst = lds_addr(abuf) + (wv >> 1) * PLANE + row0 * 256;
-        auto issue_a = [&](uint32_t buf, uint32_t st) {
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                const uint8_t* src = reinterpret_cast<const uint8_t*>(plane) + 256 * min(NH * st + h, NHS - 1);
-#pragma unroll
-                for (int u = 0; u < 2 * MS; ++u) dma16(src, a_off[u], a_dst + buf * STAGE + h * HALF + u * 1024);
-            }
-        };
-
-        f32x4_t acc[MS][GD_SUB];
-#pragma unroll
-        for (int ms = 0; ms < MS; ++ms)
-#pragma unroll
-            for (int j = 0; j < GD_SUB; ++j) acc[ms][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-        issue_s(0);
-        issue_w(0);
-        issue_a(0, 0);
-        mem_fence_compiler();
-
-        for (uint32_t st = 0; st < NST; ++st) {
-            const uint32_t buf = st & 1;
-            vm_wait<0>();
-            gm_barrier();
-            uint32_t gw[NH][GD_SUB][2][2];       // [pair of groups][subtile][group][MFMA step]
-#pragma unroll
-            for (int h = 0; h < NH; ++h)
-#pragma unroll
-                for (int j = 0; j < GD_SUB; ++j)
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        const auto x = __builtin_amdgcn_permlane16_swap(wr[h][j][s], wr[h][j][2 + s], false, false);
-                        const auto r = __builtin_amdgcn_permlane32_swap(x[0], x[1], false, false);
-                        gw[h][j][0][s] = r[0];
-                        gw[h][j][1][s] = r[1];
-                    }
-            // (the last stage requests itself again, into the other buffer)
-            const uint32_t nx = min(st + 1, NST - 1);
-            if ((NH * st) % 4 == 0) {
-#pragma unroll
-                for (int i = 0; i < NM; ++i) sc_cur[i] = sc_next[i];
-                issue_s(min((NH * st) / 4 + 1, (NHS - 1) / 4));
-            }
-            issue_w(nx);
-            issue_a(buf ^ 1u, nx);
-            mem_fence_compiler();
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                if (NH > 1 && h > 0 && NH * st + h >= NHS) break;
-                __builtin_amdgcn_sched_barrier(0);
-                uint32_t sc2[GD_SUB];            // the two groups' fp16 scales
-#pragma unroll
-                for (int j = 0; j < GD_SUB; ++j)
-                    sc2[j] = __builtin_amdgcn_ds_bpermute(4 * (16 * (j % SM) + m16), sc_cur[j / SM][0]);
-#pragma unroll
-                for (int i = 0; i < NM; ++i) {
-                    sc_cur[i][0] = sc_cur[i][1];
-                    sc_cur[i][1] = sc_cur[i][2];
-                    sc_cur[i][2] = sc_cur[i][3];
-                }
-                const uint8_t* A = abuf + buf * STAGE + h * HALF;
-                // fragment c (step c / 2, plane c & 1) of m-tile k % MS of group k / MS
-                half8_t xa[4];
-                auto load_a = [&](int k, int c) {
-                    xa[c] = lds_half8(A + (c & 1) * PLANE + (k % MS) * 4096 + aoff[k / MS][c >> 1]);
-                };
-                // The sched_barriers pin the order (left to itself the compiler reads
-                // each fragment right before its use and runs the chains one after
-                // the other, waiting out every latency).
-#pragma unroll
-                for (int c = 0; c < 4; ++c) load_a(0, c);
+            for (int j = 0; j < GD_SUB; ++j) {
+                const auto u = __builtin_amdgcn_permlane32_swap(wr[D][j][0], wr[D][j][2], false, false);
+                const auto v = __builtin_amdgcn_permlane32_swap(wr[D][j][1], wr[D][j][3], false, false);
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
-                    f32x4_t t[GD_SUB];
-                    half8_t b[GD_SUB][2];
-                    float sc[GD_SUB];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int j = 0; j < GD_SUB; ++j) {
-                        b[j][0] = q4_codes_to_f16(gw[h][j][g][0]);
-                        sc[j] = f16_bits_to_f32(static_cast<uint16_t>(g ? sc2[j] >> 16 : sc2[j]));
-                    }
-                    auto scale_in = [&](int ms, int j) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[j][i], acc[ms][j][i]);
-                    };
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        const int k = g * MS + ms;
-                        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-#pragma unroll
-                            for (int j = 0; j < GD_SUB; ++j) {
-                                const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-                                if (c == 0 && ms > 0) scale_in(ms - 1, j);
-                                t[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c], b[j][c >> 1], c ? t[j] : z, 0, 0,
-                                                                              0);
-                            }
-                            if (ms == 0 && c < 2) {
-                                b[2 * c][1] = q4_codes_to_f16(gw[h][2 * c][g][1]);
-                                b[2 * c + 1][1] = q4_codes_to_f16(gw[h][2 * c + 1][g][1]);
-                            }
-                            __builtin_amdgcn_sched_barrier(0);
-                            if (k + 1 < 2 * MS) load_a(k + 1, c);
-                        }
-                    }
-#pragma unroll
-                    for (int j = 0; j < GD_SUB; ++j) scale_in(MS - 1, j);
+                    const auto r = __builtin_amdgcn_permlane16_swap(u[g], v[g], false, false);
+                    gw[0][j][g][0] = r[0];
+                    gw[0][j][g][1] = r[1];
                 }
             }
-            mem_fence_compiler();
-        }
-        vm_wait<0>();
+        } else if constexpr (EVEN) {
+            // lane bits 5 4 3 | 2 1 0 hold group, group, half of the group | row,
+            // the registers row bit 3 (x, y) and the word of the half.  Half and
+            // row bit 3 change places, then the group's bits and the word's:
+            // quad q has word q of either half of every group, row m16.
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms) {
+            for (int j = 0; j < GD_SUB; ++j) {
+                uint32_t hw[2][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t m = 16 * ms + 4 * q + i;
-                if (m0 + m >= me) continue;
-                const float rs = a_scale[s_row[m]] * (8.0f / 15.0f);   // weights are (2c - 15) / 8
-                float* o = out + static_cast<size_t>(s_pair[m]) * n_dim;
-                if constexpr (GATE_UP) {
+                for (int w = 0; w < 4; ++w) {
+                    const int x = wr[D / 2][2 * j][w], y = wr[D / 2][2 * j + 1][w];
+                    hw[0][w] = __builtin_amdgcn_update_dpp(x, y, 0x128, 0xF, 0xC, false);   // row_ror:8
+                    hw[1][w] = __builtin_amdgcn_update_dpp(y, x, 0x128, 0xF, 0x3, false);
+                }
 #pragma unroll
-                    for (int j = 0; j < GD_SUB / 2; ++j) {
-                        const uint32_t n = tile * (GD_ROWS / 2) + 8 * GD_SUB * wv + 16 * j + m16;
-                        const float v0 = acc[ms][j][i] * rs, v1 = acc[ms][j + GD_SUB / 2][i] * rs;
-                        if (n < n_dim) o[n] = (v0 * (1.0f / (1.0f + expf(-v0)))) * v1;
+                for (int h = 0; h < 2; ++h) {
+                    const auto u = __builtin_amdgcn_permlane32_swap(hw[h][0], hw[h][2], false, false);
+                    const auto v = __builtin_amdgcn_permlane32_swap(hw[h][1], hw[h][3], false, false);
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const auto r = __builtin_amdgcn_permlane16_swap(u[p], v[p], false, false);
+                        gw[p][j][0][h] = r[0];
+                        gw[p][j][1][h] = r[1];
                     }
-                } else {
+                }
+            }
+        }
+        if (st % 4 == 0) {
+#pragma unroll
+            for (int i = 0; i < NM; ++i) sc_cur[i] = sc_next[i];
+            issue_s(min(st / 4 + 1, (NST - 1) / 4));
+        }
+        // every wave is past stage st - 1: its slot takes stage st + DP
+        if (st + DP < NST) issue_a(slot == 0 ? DP : slot - 1, st + DP);
+        if constexpr (!QUAD) issue_w(wr[D], st + DP);
+        else if constexpr (EVEN) issue_w(wr[D / 2], (st + DP) / 2);
+        mem_fence_compiler();
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t sc2[GD_SUB];                    // the two groups' fp16 scales
+#pragma unroll
+        for (int j = 0; j < GD_SUB; ++j)
+            sc2[j] = __builtin_amdgcn_ds_bpermute(4 * (16 * (j % SM) + m16), sc_cur[j / SM][0]);
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            sc_cur[i][0] = sc_cur[i][1];
+            sc_cur[i][1] = sc_cur[i][2];
+            sc_cur[i][2] = sc_cur[i][3];
+        }
+        const uint8_t* A = abuf + slot * STAGE;
+        slot = slot == DP ? 0 : slot + 1;
+        // fragment c (step c / 2, plane c & 1) of m-tile k % MS of group k / MS
+        half8_t xa[4];
+        auto load_a = [&](int k, int c) {
+            xa[c] = lds_half8(A + (c & 1) * PLANE + (k % MS) * 4096 + aoff[k / MS][c >> 1]);
+        };
+        // The sched_barriers pin the order (left to itself the compiler reads
+        // each fragment right before its use and runs the chains one after
+        // the other, waiting out every latency).
+#pragma unroll
+        for (int c = 0; c < 4; ++c) load_a(0, c);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            f32x4_t t[GD_SUB];
+            half8_t b[GD_SUB][2];
+            float sc[GD_SUB];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < GD_SUB; ++j) {
+                b[j][0] = q4_codes_to_f16(gw[QUAD ? D % 2 : 0][j][g][0]);
+                sc[j] = f16_bits_to_f32(static_cast<uint16_t>(g ? sc2[j] >> 16 : sc2[j]));
+            }
+            auto scale_in = [&](int ms, int j) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[ms][j][i] = fmaf(sc[j], t[j][i], acc[ms][j][i]);
+            };
+#pragma unroll
+            for (int ms = 0; ms < MS; ++ms) {
+                const int k = g * MS + ms;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
 #pragma unroll
                     for (int j = 0; j < GD_SUB; ++j) {
-                        const uint32_t n = tile * GD_ROWS + 16 * GD_SUB * wv + 16 * j + m16;
-                        if (n < n_dim) o[n] = acc[ms][j][i] * rs;
+                        const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+                        if (c == 0 && ms > 0) scale_in(ms - 1, j);
+                        t[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[c], b[j][c >> 1], c ? t[j] : z, 0, 0, 0);
                     }
+                    if (ms == 0 && c < 2) {
+                        b[2 * c][1] = q4_codes_to_f16(gw[QUAD ? D % 2 : 0][2 * c][g][1]);
+                        b[2 * c + 1][1] = q4_codes_to_f16(gw[QUAD ? D % 2 : 0][2 * c + 1][g][1]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (k + 1 < 2 * MS) load_a(k + 1, c);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < GD_SUB; ++j) scale_in(MS - 1, j);
+        }
+        mem_fence_compiler();
+    };
+    for (uint32_t st = 0;;) {
+        stage(std::integral_constant<int, 0>{}, st);
+        if (++st >= NST) break;
+        if constexpr (DP > 1) {
+            stage(std::integral_constant<int, 1>{}, st);
+            if (++st >= NST) break;
+        }
+        if constexpr (DP > 2) {
+            stage(std::integral_constant<int, 2 % DP>{}, st);
+            if (++st >= NST) break;
+        }
+        if constexpr (DP > 3) {
+            stage(std::integral_constant<int, 3 % DP>{}, st);
+            if (++st >= NST) break;
+        }
+    }
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t m = 16 * ms + 4 * q + i;
+            const uint32_t p = __builtin_amdgcn_ds_bpermute(4 * m, pair);
+            const float as = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * m, __builtin_bit_cast(int, ascale)));
+            if (m >= np) continue;
+            const float rs = as * (8.0f / 15.0f);   // weights are (2c - 15) / 8
+            float* o = out + static_cast<size_t>(p) * n_dim;
+            if constexpr (GATE_UP) {
+#pragma unroll
+                for (int j = 0; j < GD_SUB / 2; ++j) {
+                    const uint32_t n = tile * (GD_ROWS / 2) + 8 * GD_SUB * wv + 16 * j + m16;
+                    const float v0 = acc[ms][j][i] * rs, v1 = acc[ms][j + GD_SUB / 2][i] * rs;
+                    if (n < n_dim) o[n] = (v0 * (1.0f / (1.0f + expf(-v0)))) * v1;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < GD_SUB; ++j) {
+                    const uint32_t n = tile * GD_ROWS + 16 * GD_SUB * wv + 16 * j + m16;
+                    if (n < n_dim) o[n] = acc[ms][j][i] * rs;
                 }
             }
         }
@@ -1391,19 +1480,19 @@ __device__ __forceinline__ void grouped_reg_expert(
 
 template <bool GATE_UP>
 __global__ __launch_bounds__(GD_WAVES * WAVE, 2)
-void k_grouped_reg(MoeDims d, LayerDesc L, const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ units,
+void k_grouped_reg(MoeDims d, LayerDesc L, const uint4* __restrict__ units,
                    const uint32_t* __restrict__ sorted_pairs, const uint16_t* __restrict__ a_hi,
                    const uint16_t* __restrict__ a_lo, const float* __restrict__ a_scale, uint32_t a_row_div,
                    float* __restrict__ out, uint32_t n_dim, uint32_t k_dim, uint32_t n_tiles)
 {
-    __shared__ __align__(16) uint8_t abuf[2 * GD_STAGE];
-    __shared__ uint32_t s_row[GM_PASS];
-    __shared__ uint32_t s_pair[GM_PASS];
-    uint32_t e, tile, base, mb, me, rows;
-    if (!unit_of_block(offsets, units, n_tiles, e, tile, base, mb, me, rows)) return;
+    __shared__ __align__(16) uint8_t abuf[GD_LDS];
+    uint32_t tile;
+    const uint4 rec = unit_of_block(units, n_tiles, tile);
+    if (rec.z == 0) return;
+    const uint32_t rows = rec.x >> 16;
     auto go = [&](auto ms) {
-        grouped_reg_expert<GATE_UP, decltype(ms)::value>(L, e, tile, base, mb, me, sorted_pairs, a_hi, a_lo, a_scale,
-                                                         a_row_div, out, n_dim, k_dim, abuf, s_row, s_pair);
+        grouped_reg_expert<GATE_UP, decltype(ms)::value>(L, rec.x & 0xFFFFu, tile, rec.y, rec.z, sorted_pairs, a_hi,
+                                                         a_lo, a_scale, a_row_div, out, n_dim, k_dim, abuf);
     };
     if (rows == 16) go(std::integral_constant<int, 1>{});
     else if (rows == 32) go(std::integral_constant<int, 2>{});
@@ -1510,12 +1599,12 @@ static size_t permute_lds_alloc(uint32_t P, uint32_t E)
 
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
-                          uint32_t* union_size, uint32_t* units, uint32_t few_units, uint32_t* err, hipStream_t s)
+                          uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s)
 {
     if (P == 0 || E == 0 || permute_lds_bytes(P, E) > PERMUTE_MAX_LDS) return hipErrorInvalidValue;
     const size_t lds = permute_lds_alloc(P, E);
     launch_kernel_lds(k_permute, dim3(1), dim3(PERM_THREADS), static_cast<uint32_t>(lds), s, ids, w, P, K, E,
-                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, units, few_units, err);
+                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, units, unit_slots(P, E, few_units), few_units, err);
     return hipGetLastError();
 }
 
@@ -1526,14 +1615,14 @@ uint32_t perm_segments(uint32_t P, uint32_t E)
 }
 
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
-                              uint32_t* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
+                              uint4* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
 {
     if (P == 0 || E == 0 || E > SMOE_TOPK_MAX_N) return hipErrorInvalidValue;
     const uint32_t nseg = perm_segments(P, E);
     launch_kernel(k_perm_count, dim3(nseg), dim3(PERM_THREADS), s, ids, P, E, seg_cnt, err);
     const uint32_t lds = (E * (perm_seg_chunks(E) | 1u) + 4 * E + 2) * static_cast<uint32_t>(sizeof(uint32_t));
     launch_kernel_lds(k_perm_scatter, dim3(nseg), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt, offsets,
-                      sorted_pairs, units, few_units);
+                      sorted_pairs, units, unit_slots(P, E, few_units), few_units);
     return hipGetLastError();
 }
 
@@ -1547,37 +1636,37 @@ static bool reg_supported(const LayerDesc& L, uint32_t k_dim)
 }
 
 template <bool GATE_UP>
-static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
-                                 const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* a_hi,
+static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+                                 const uint32_t* sorted_pairs, const uint16_t* a_hi,
                                  const uint16_t* a_lo, const float* a_scale, float* out, hipStream_t s)
 {
-    if (d.group != 64 || d.I % 64 || d.D % 64 || P == 0 || !offsets || !units) return hipErrorInvalidValue;
+    if (d.group != 64 || d.I % 64 || d.D % 64 || P == 0 || !units) return hipErrorInvalidValue;
     const uint32_t n_dim = GATE_UP ? d.I : d.D, k_dim = GATE_UP ? d.D : d.I, div = GATE_UP ? d.K : 1u;
-    const uint32_t per = (max_units(P, d.E, few_units) + 7) / 8;
+    const uint32_t slots = unit_slots(P, d.E, few_units);
     if (reg_supported(L, k_dim)) {
         const uint32_t rows = GATE_UP ? GD_ROWS / 2 : GD_ROWS, nt = (n_dim + rows - 1) / rows;
-        launch_kernel(k_grouped_reg<GATE_UP>, dim3(8 * per * nt), dim3(GD_WAVES * WAVE), s, d, L, offsets, units,
+        launch_kernel(k_grouped_reg<GATE_UP>, dim3(slots * nt), dim3(GD_WAVES * WAVE), s, d, L, units,
                       sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
     } else {
         const uint32_t rows = GATE_UP ? GM_ROWS_GU : GM_ROWS_DN, nt = (n_dim + rows - 1) / rows;
-        launch_kernel(k_grouped_mm<GATE_UP>, dim3(8 * per * nt), dim3(GM_WAVES * WAVE), s, d, L, offsets, units,
+        launch_kernel(k_grouped_mm<GATE_UP>, dim3(slots * nt), dim3(GM_WAVES * WAVE), s, d, L, units,
                       sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
-                                  const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* x_hi,
+hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+                                  const uint32_t* sorted_pairs, const uint16_t* x_hi,
                                   const uint16_t* x_lo, const float* x_scale, float* h, hipStream_t s)
 {
-    return launch_grouped<true>(d, L, P, few_units, offsets, units, sorted_pairs, x_hi, x_lo, x_scale, h, s);
+    return launch_grouped<true>(d, L, P, few_units, units, sorted_pairs, x_hi, x_lo, x_scale, h, s);
 }
 
-hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint32_t* offsets,
-                               const uint32_t* units, const uint32_t* sorted_pairs, const uint16_t* h_hi,
+hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+                               const uint32_t* sorted_pairs, const uint16_t* h_hi,
                                const uint16_t* h_lo, const float* h_scale, float* y, hipStream_t s)
 {
-    return launch_grouped<false>(d, L, P, few_units, offsets, units, sorted_pairs, h_hi, h_lo, h_scale, y, s);
+    return launch_grouped<false>(d, L, P, few_units, units, sorted_pairs, h_hi, h_lo, h_scale, y, s);
 }
 
 hipError_t launch_combine_pairs(const float* y, const float* w, uint32_t T, uint32_t K, uint32_t D, float* hidden,

@@ -31,6 +31,7 @@ def prefill(ctx, layer, h, step):
     (128, 1, 1, 640, (16, 33, 65)),      # one pair of groups in, five out
     (1280, 4, 2, 704, (37, 150)),        # an odd number of groups in the down rows
     (320, 8, 3, 192, (50,)),             # and in both
+    (1152, 4, 2, 896, (9, 70)),          # odd numbers of pairs of groups past the first ring of stages
     (256, 512, 8, 128, (300,)),          # segments of 16 chunks
     (256, 128, 8, 128, (1000, 5000)),    # several segments, several passes
 ])
