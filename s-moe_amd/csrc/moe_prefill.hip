@@ -1566,12 +1566,14 @@ hipError_t launch_route(const MoeDims& d, const LayerDesc& L, const float* hidde
 {
     if (d.E > SMOE_TOPK_MAX_N || d.K > SMOE_TOPK_MAX_K || d.D % 64 || T == 0) return hipErrorInvalidValue;
     const uint32_t cpl = (d.D / 32 + WAVE - 1) / WAVE;
-    // tokens per block: as many as keep one block per CU busy (each block
-    // reads the whole router matrix from L2 once), at most what the registers
-    // of a chunk per lane allow.  Under 128 tokens (one per block) the router
+    // tokens per block: as few as give at most one block per CU (each block
+    // reads the whole router matrix from L2 once, and a second round of blocks
+    // costs as much as the first: 384 tokens of the 30B shape 24.8 us with one
+    // token a block, 16.9 with two, 400 of the 235B shape 42.9 and 31), at most what the registers of a chunk per
+    // lane allow.  Under 128 tokens (one per block) the router
     // rows of a token are split over 4 blocks (needs E <= 128: 4 rows a wave).
     const uint32_t cus = 256;
-    const uint32_t tb = T >= 4 * cus ? 4 : T >= 2 * cus ? 2 : 1;
+    const uint32_t tb = T > 2 * cus ? 4 : T > cus ? 2 : 1;
     const bool split = T < 128 && d.E <= 128 && logits && counters;
     if (cpl == 1) {
         if (tb == 4) return route_c<1, 4>(d, L, hidden, T, x_hi, x_lo, x_sc, ids, w, logits, counters, s);

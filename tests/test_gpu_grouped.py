@@ -33,7 +33,7 @@ def prefill(ctx, layer, h, step):
     (320, 8, 3, 192, (50,)),             # and in both
     (1152, 4, 2, 896, (9, 70)),          # odd numbers of pairs of groups past the first ring of stages
     (256, 512, 8, 128, (300,)),          # segments of 16 chunks
-    (256, 128, 8, 128, (1000, 5000)),    # several segments, several passes
+    (256, 128, 8, 128, (257, 1000, 5000)),   # several segments, several passes
 ])
 def test_passes_and_segments(ctx, D, E, K, I, Ts):
     layer = Layer(ctx, D, E, K, I, layer_id=500 + D + I)
