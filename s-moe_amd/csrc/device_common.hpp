@@ -44,12 +44,6 @@ __device__ __forceinline__ uint4 load_stream_u4(const void* p)
     return r;
 }
 
-__device__ __forceinline__ float4 load_stream_f4(const float* p)
-{
-    const uint4 v = load_stream_u4(p);
-    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-}
-
 __device__ __forceinline__ uint16_t load_stream_u16(const uint16_t* p)
 {
     return __builtin_nontemporal_load(gptr(p));

@@ -473,19 +473,16 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // v_mfma_f32_16x16x4_f32: lane l = (m16 = l & 15, q = l >> 4) holds A[m16][q] and
 // B[q][m16] and receives D[4 q + i][m16].  Scores: A = K (row = position, K
-// index q of step 4 s + j = dim 32 (s / 2) + 8 q + 4 (s & 1) + j), B = the query heads; a lane
+// index q of step 4 s + j = dim 16 s + 4 q + j), B = the query heads; a lane
 // then has the scores of positions 4 q + i of head m16, which are the B operand
 // (K index q of step i = position 4 q + i) of the weighted sum, whose A is V
 // transposed (row m16 of result (h, j) = dim 64 h + 4 m16 + j).  No value moves
 // between lanes but the maximum and the final sums.
 //
 // Bound by reading K and V: the attention layer over 32768 positions of the 235B
-// layout (134 MB of K and V, 16 query heads a KV head) takes 59.4 us, 27 of them its
-// two GEMVs, against 79 with k_attn_decode, whose two blocks per KV head and split,
-// on different XCDs, each read every row and whose dot products are the VALU's.
-// Loads take whole 128-byte lines, non-temporal (each row is read once): K as 128
-// bytes of 8 positions, then a rotation by 8 in each 16 lanes puts 16 positions
-// in the MFMA's rows (K as 64 bytes of 16 positions: 61.1 us).
+// layout (134 MB of K and V, 16 query heads a KV head) takes 59 us, 27 of them its two
+// GEMVs, against 80 with k_attn_decode, whose two blocks per KV head and split, on
+// different XCDs, each read every row and whose dot products are the VALU's.
 // Sums run in chains of eight terms that are then added, as there: 3.73e-7 from
 // fp64 over 32768 positions (12 inputs) against 3.69e-7, 3.96e-7 against 3.95e-7
 // over 5000; in chains of 64 it was 4.4e-7.
@@ -514,8 +511,7 @@ void k_attn_wide(AttnArgs p)
     const uint32_t i0 = sp * p.chunk, n = min(p.chunk, p.valid - i0);
 
     // ---- K and V of 16 positions from t0 (past the split: its last, masked) ----
-    // k[2 u + i]: position 8 i + (lane & 7), dims 32 u + 4 (lane >> 3) .. + 3
-    const float* kbase = p.k_cache + kvh * HD + 4 * (lane >> 3);
+    const float* kbase = p.k_cache + kvh * HD + 4 * q;
     const float* vbase = p.v_cache + kvh * HD + 4 * m16;
     struct Tile {
         float4 k[NS], v[4][NH];
@@ -525,17 +521,14 @@ void k_attn_wide(AttnArgs p)
         return static_cast<size_t>(p.slot >= ip ? p.slot - ip : p.slot + p.a.ctx - ip) * p.a.kv_dim;
     };
     auto load_tile = [&](uint32_t t0, Tile& t) {
+        const float* k = kbase + ring(t0 + m16);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float* k = kbase + ring(t0 + 8 * i + (lane & 7));
-#pragma unroll
-            for (int u = 0; u < NS / 2; ++u) t.k[2 * u + i] = load_stream_f4(k + 32 * u);
-        }
+        for (int s = 0; s < NS; ++s) t.k[s] = load_f4(k + 16 * s);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float* v = vbase + ring(t0 + 4 * q + i);
 #pragma unroll
-            for (int h = 0; h < NH; ++h) t.v[i][h] = load_stream_f4(v + 64 * h);
+            for (int h = 0; h < NH; ++h) t.v[i][h] = load_f4(v + 64 * h);
         }
     };
     // the first tile does not wait for the projections' results (position 0,
@@ -588,8 +581,8 @@ void k_attn_wide(AttnArgs p)
         if (wv == 0) {
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
-                const float4 f = *reinterpret_cast<const float4*>(kn + 32 * (s / 2) + 4 * (lane >> 3));
-                if (min(static_cast<uint32_t>(8 * (s & 1) + (lane & 7)), n - 1) == 0) ta.k[s] = f;
+                const float4 f = *reinterpret_cast<const float4*>(kn + 16 * s + 4 * q);
+                if (min(static_cast<uint32_t>(m16), n - 1) == 0) ta.k[s] = f;
             }
             // (also where a masked position repeats position 0: its weight is 0,
             // but what the ring held there before need not be a number)
@@ -607,8 +600,7 @@ void k_attn_wide(AttnArgs p)
     // ---- the split's positions ----------------------------------------------
     float4 qv[NS];
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
-        qv[s] = *reinterpret_cast<const float4*>(qs + m16 * RS + 32 * (s / 2) + 8 * q + 4 * (s & 1));
+    for (int s = 0; s < NS; ++s) qv[s] = *reinterpret_cast<const float4*>(qs + m16 * RS + 16 * s + 4 * q);
     const float scale = p.a.scale;
     float mx = -INFINITY, lsum = 0.f;           // of head m16 (the sum: this lane's positions)
     f32x4_t acc[NH][4];
@@ -622,19 +614,9 @@ void k_attn_wide(AttnArgs p)
 #pragma unroll
         for (int s0 = 0; s0 < NS; s0 += 2) {
             f32x4_t c[4];
-            // lane bit 3 (dims 4 .. 7 of 8) and the position's bit 3 (which load) change places
-            const float kx[4] = {t.k[s0].x, t.k[s0].y, t.k[s0].z, t.k[s0].w};
-            const float ky[4] = {t.k[s0 + 1].x, t.k[s0 + 1].y, t.k[s0 + 1].z, t.k[s0 + 1].w};
-            float kk[2][4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int x = __builtin_bit_cast(int, kx[j]), y = __builtin_bit_cast(int, ky[j]);   // row_ror:8
-                kk[0][j] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, y, 0x128, 0xF, 0xC, false));
-                kk[1][j] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(y, x, 0x128, 0xF, 0x3, false));
-            }
 #pragma unroll
             for (int s = s0; s < s0 + 2; ++s) {
-                const float (&kf)[4] = kk[s - s0];
+                const float kf[4] = {t.k[s].x, t.k[s].y, t.k[s].z, t.k[s].w};
                 const float qf[4] = {qv[s].x, qv[s].y, qv[s].z, qv[s].w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
