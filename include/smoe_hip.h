@@ -341,7 +341,7 @@ int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape,
  * prompt in chunks of 64 tokens inside every layer (prefill.hpp:33); tokens
  * are independent inside the MoE block, so a layer over all tokens gives the
  * same results and streams each touched expert's weights once per pass of up
- * to 736 tokens instead of once per chunk.  ids_out / weights_out
+ * to 4096 tokens (32768 / top_k) instead of once per chunk.  ids_out / weights_out
  * [n_layers x n_tokens x top_k] are optional. */
 int smoe_hip_moe_prefill_stack(SmoeMetalCtx* ctx, const SmoeMoeShape* shape,
                                const SmoeMoeLayer* layers, uint32_t n_layers, float* hidden,
