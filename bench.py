@@ -905,24 +905,24 @@ def grouped_line(workload, replicas, steps, warmup, calibrate_mib=0):
         "layer_bytes": layer_bytes, "layer_gbs": round(layer_bytes / (us_per_layer * 1e-6) / 1e9, 1),
         "layer_tflops": round(flops / (us_per_layer * 1e-6) / 1e12, 2),
         "roofline": {
-            "bound": "hbm", "kernel": "k_grouped_mm<true>",
+            "bound": "hbm", "kernel": "k_grouped_reg<true>",
             "achieved": round(gu_bytes / (gu_us * 1e-6) / 1e9, 1) if gu else None,
             "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gu_bytes / (gu_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4) if gu else None,
-            "traffic": grouped_traffic(g["workload"], "k_grouped_mm<true>"), "bytes_per_launch": gu_bytes,
+            "traffic": grouped_traffic(g["workload"], "k_grouped_reg<true>"), "bytes_per_launch": gu_bytes,
             "avg_us": gu_us,
         },
         "mfma": {
-            "kernel": "k_grouped_mm<true>", "tflops_algorithmic": round(4 * D * I * pairs / (gu_us * 1e-6) / 1e12, 1)
+            "kernel": "k_grouped_reg<true>", "tflops_algorithmic": round(4 * D * I * pairs / (gu_us * 1e-6) / 1e12, 1)
             if gu else None,
             "tflops_executed": round(mfma_flops / (gu_us * 1e-6) / 1e12, 1) if gu else None,
             "peak_tflops": MFMA_F16_PEAK_TFLOPS,
             "frac_executed": round(mfma_flops / (gu_us * 1e-6) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4) if gu else None,
             "layer_frac": round(flops / (us_per_layer * 1e-6) / 1e12 / MFMA_F16_PEAK_TFLOPS, 4),
         },
-        "down": {"kernel": "k_grouped_down", "bytes_per_launch": dn_bytes,
+        "down": {"kernel": "k_grouped_reg<false>", "bytes_per_launch": dn_bytes,
                  "gbs": round(dn_bytes / (dn["avg_us"] * 1e-6) / 1e9, 1) if dn else None,
-                 "traffic": grouped_traffic(g["workload"], "k_grouped_down")},
+                 "traffic": grouped_traffic(g["workload"], "k_grouped_reg<false>")},
         "kernels": kern,
     }
     ctx.close()
@@ -990,7 +990,7 @@ def rocprof_summary(d, config, pmc_out, copy_mib, workload="decode"):
     data = json.load(open(pmc_out)) if os.path.exists(pmc_out) else {}
     if workload in GROUPED:
         ent = data.setdefault(GROUPED[workload]["workload"], {})
-        symbols = ("k_grouped_mm<true>", "k_grouped_down", "k_grouped_mm<false>")
+        symbols = ("k_grouped_reg<true>", "k_grouped_reg<false>")
     else:
         ent = data.setdefault(CONFIGS[config]["workload"], {})
         symbols = tuple(KERNEL_SYMBOLS.values())
