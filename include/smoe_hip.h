@@ -487,7 +487,9 @@ int smoe_hip_moe_decode_static(const SmoeMoeShape* shape, const SmoeMoeLayer* la
  * decode.hpp:36-74, and smoe_metal_kernel_dispatches) ------------------------
  * When enabled, every kernel the context launches outside graph capture is
  * bracketed by HIP events on the stream it runs on; profile_read returns the
- * launch count and summed event time of one kernel kind. */
+ * launch count and summed event time of one kernel kind.  A kind that takes two
+ * dispatches a call (PERMUTE over several segments, ATTENTION over several
+ * context splits) counts one launch with the time of both. */
 #define SMOE_KERNEL_MOE_UP        0   /* RMSNorm + router + top-k + gate/up GEMV + SiLU */
 #define SMOE_KERNEL_GATE_UP       1   /* gate/up GEMV + SiLU (reference surface)        */
 #define SMOE_KERNEL_MOE_DOWN      2   /* down GEMV + weighted combine + residual        */

@@ -136,13 +136,14 @@ struct SmoeMetalCtx {
         hipEvent_t a = nullptr, b = nullptr;
         uint32_t kind = 0;
         bool pending = false;
+        bool first = false;    // the launcher's first dispatch: counted as the launch
     };
     bool profiling = false;
     std::vector<ProfSlot> prof;
     size_t prof_head = 0;
     uint64_t prof_launches[SMOE_KERNEL_KINDS] = {};
     double prof_ms[SMOE_KERNEL_KINDS] = {};
-    int prof_open = -1;   // slot index between prof_begin and prof_end
+    bool prof_open = false;   // between prof_begin and prof_end
 };
 
 namespace {
@@ -327,34 +328,38 @@ void prof_flush_slot(SmoeMetalCtx* ctx, SmoeMetalCtx::ProfSlot& p)
     if (!p.pending) return;
     float ms = 0.f;
     if (hipEventSynchronize(p.b) == hipSuccess && hipEventElapsedTime(&ms, p.a, p.b) == hipSuccess) {
-        ctx->prof_launches[p.kind] += 1;
+        ctx->prof_launches[p.kind] += p.first;
         ctx->prof_ms[p.kind] += ms;
     }
     p.pending = false;
 }
 
-// Time one kernel launch (no-op unless profiling; skipped under stream
-// capture): the slot's events are handed to the launcher, which records them
-// at the dispatch's own start and end.
+// Time one launcher's dispatches (no-op unless profiling; skipped under stream
+// capture): the events of the ring's next slots, one a dispatch, are handed to
+// the launcher, which records them at each dispatch's own start and end.
 void prof_begin(SmoeMetalCtx* ctx, uint32_t kind)
 {
-    ctx->prof_open = -1;
+    ctx->prof_open = false;
     if (!ctx->profiling || stream_capturing(ctx->stream)) return;
-    const size_t i = ctx->prof_head % kProfSlots;
-    auto& p = ctx->prof[i];
-    prof_flush_slot(ctx, p);
-    p.kind = kind;
-    smoe::dispatch_timer() = smoe::DispatchTimer{p.a, p.b};
-    ctx->prof_open = static_cast<int>(i);
+    smoe::DispatchTimer t;
+    for (; t.n < smoe::DispatchTimer::MAX; ++t.n) {
+        auto& p = ctx->prof[(ctx->prof_head + t.n) % kProfSlots];
+        prof_flush_slot(ctx, p);
+        p.kind = kind;
+        p.first = t.n == 0;
+        t.pair[t.n] = {p.a, p.b};
+    }
+    smoe::dispatch_timer() = t;
+    ctx->prof_open = true;
 }
 
 void prof_end(SmoeMetalCtx* ctx)
 {
-    if (ctx->prof_open < 0) return;
+    if (!ctx->prof_open) return;
+    const int used = smoe::dispatch_timer().used;
     smoe::dispatch_timer() = smoe::DispatchTimer{};
-    ctx->prof[ctx->prof_open].pending = true;
-    ctx->prof_head++;
-    ctx->prof_open = -1;
+    for (int i = 0; i < used; ++i) ctx->prof[ctx->prof_head++ % kProfSlots].pending = true;
+    ctx->prof_open = false;
 }
 
 // launch helper: times the launch when profiling

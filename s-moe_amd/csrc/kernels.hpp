@@ -12,21 +12,29 @@ namespace smoe {
 constexpr int SMOE_TOPK_MAX_N = 512;
 constexpr int SMOE_TOPK_MAX_K = 16;
 
-// Events that time the next kernel dispatches of this thread: when set, the
-// launchers dispatch through hipExtLaunchKernel, which records `start` when
-// the kernel begins executing and `stop` when it completes (the dispatch's
-// own timestamps, no marker packets around it).  Set only around eager
-// launches by the profiling path of the C ABI.
+// Events that time the next kernel dispatches of this thread, a pair for each
+// (a launcher may dispatch twice): while pairs are left, the launchers dispatch
+// through hipExtLaunchKernel, which records `start` when the kernel begins
+// executing and `stop` when it completes (the dispatch's own timestamps, no
+// marker packets around it).  Set only around eager launches by the profiling
+// path of the C ABI.
 struct DispatchTimer {
-    hipEvent_t start = nullptr;
-    hipEvent_t stop = nullptr;
+    static constexpr int MAX = 2;             // dispatches of one launcher
+    struct Pair {
+        hipEvent_t start = nullptr;
+        hipEvent_t stop = nullptr;
+    };
+    Pair pair[MAX];
+    int n = 0;                                // pairs given
+    int used = 0;                             // pairs that dispatches have taken
+    Pair take() { return used < n ? pair[used++] : Pair{}; }
 };
 DispatchTimer& dispatch_timer();
 
 template <typename... KArgs, typename... Args>
 inline void launch_kernel_lds(void (*k)(KArgs...), dim3 grid, dim3 block, uint32_t lds, hipStream_t s, Args... args)
 {
-    const DispatchTimer& t = dispatch_timer();
+    const DispatchTimer::Pair t = dispatch_timer().take();
     if (t.start)
         hipExtLaunchKernelGGL(k, grid, block, lds, s, t.start, t.stop, 0, static_cast<KArgs>(args)...);
     else
@@ -246,13 +254,20 @@ constexpr uint32_t unit_slots(uint32_t P, uint32_t E, uint32_t few_units)
 // 103 us with units of 64, 89 with 32; 512 even ones (128 experts of 32): 186
 // with 64, 215 with 32, so the shorter units stay below one round.
 constexpr uint32_t few_units(const MoeDims& d) { return 512u / ((d.I + 127u) / 128u); }
-size_t permute_lds_bytes(uint32_t P, uint32_t E);
+constexpr size_t permute_lds_bytes(uint32_t P, uint32_t E)
+{
+    return (size_t((P + 63) / 64) * E + 3 * size_t(E) + 1) * sizeof(uint32_t);
+}
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
                           uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s);
 // The same offsets, sorted pairs and units in segments, one workgroup each, for
 // any P (seg_cnt [perm_segments(P, E) x E]).
-uint32_t perm_segments(uint32_t P, uint32_t E);
+__host__ __device__ constexpr uint32_t perm_seg_chunks(uint32_t E) { return E <= 256 ? 32u : 16u; }
+constexpr uint32_t perm_segments(uint32_t P, uint32_t E)
+{
+    return (P + 64u * perm_seg_chunks(E) - 1) / (64u * perm_seg_chunks(E));
+}
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
                               uint4* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):

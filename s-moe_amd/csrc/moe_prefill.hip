@@ -705,8 +705,6 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
 // it itself (ONE) and is the only launch (64 tokens of the 30B shape 115.9 ->
 // 113.5 us a call).
 // ---------------------------------------------------------------------------
-constexpr uint32_t perm_seg_chunks(uint32_t E) { return E <= 256 ? 32u : 16u; }
-
 __global__ __launch_bounds__(PERM_THREADS)
 void k_perm_count(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, uint32_t* __restrict__ seg_cnt,
                   uint32_t* __restrict__ err)
@@ -1599,12 +1597,6 @@ hipError_t launch_split_rows(const float* src, uint32_t rows, uint32_t cols, uin
     return hipGetLastError();
 }
 
-size_t permute_lds_bytes(uint32_t P, uint32_t E)
-{
-    const size_t C = (P + 63) / 64;
-    return (C * E + 3 * size_t(E) + 1) * sizeof(uint32_t);
-}
-
 // what k_permute allocates: the count table's odd row stride and the unit
 // offsets add at most 2 E + 1 words to permute_lds_bytes (which bounds the batch)
 static size_t permute_lds_alloc(uint32_t P, uint32_t E)
@@ -1622,12 +1614,6 @@ hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint3
     launch_kernel_lds(k_permute, dim3(1), dim3(PERM_THREADS), static_cast<uint32_t>(lds), s, ids, w, P, K, E,
                       offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, units, unit_slots(P, E, few_units), few_units, err);
     return hipGetLastError();
-}
-
-uint32_t perm_segments(uint32_t P, uint32_t E)
-{
-    const uint32_t len = 64u * perm_seg_chunks(E);
-    return (P + len - 1) / len;
 }
 
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,

@@ -1,0 +1,94 @@
+"""The host side of the C ABI (csrc/bridge.cpp) on the CPU: compiled against a
+HIP runtime and launchers that only keep books (fake_hip.cpp), so that memory
+that runs out, launches that fail and stream capture can be forced."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+import smoe_amd
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SHAPE_30B = dict(d_model=2048, n_experts=128, top_k=8, d_ff=768)
+DEV = 1 << 20        # stands for any device address
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    cxx = "/opt/rocm/llvm/bin/clang++"
+    cxx = cxx if os.path.exists(cxx) else shutil.which("clang++")
+    so = str(tmp_path_factory.mktemp("fake") / "libbridge_fake.so")
+    r = subprocess.run(
+        [cxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+         "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "s-moe_amd", "csrc"),
+         os.path.join(ROOT, "s-moe_amd", "csrc", "bridge.cpp"), os.path.join(ROOT, "tests", "fake_hip.cpp"),
+         "-Wl,-Bsymbolic", "-o", so], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return so
+
+
+class Bridge:
+    """A context of the library built on the fake runtime."""
+
+    def __init__(self, so):
+        self.lib = C.CDLL(so)
+        for name, res, args in smoe_amd.SIGNATURES:
+            if hasattr(self.lib, name):
+                getattr(self.lib, name).restype, getattr(self.lib, name).argtypes = res, args
+        self.lib.fake_count.restype, self.lib.fake_count.argtypes = C.c_uint64, [C.c_char_p]
+        self.lib.fake_budget.argtypes = [C.c_size_t]
+        self.lib.fake_is_live.argtypes = [C.c_uint64]
+        self.lib.fake_fail.argtypes = [C.c_char_p]
+        self.budget()
+        self.capturing(False)
+        self.ctx = self.lib.smoe_metal_init(1 << 15)
+        assert self.ctx
+
+    def close(self):
+        self.capturing(False)
+        self.lib.smoe_metal_destroy(self.ctx)
+        assert self.count("allocations") == 0 and self.count("host_allocations") == 0   # all given back
+
+    def count(self, what):
+        return self.lib.fake_count(what.encode())
+
+    def budget(self, n=None):
+        self.lib.fake_budget(C.c_size_t(-1).value if n is None else n)
+
+    def capturing(self, on):
+        self.lib.fake_capturing(int(on))
+
+    def live(self, p):
+        return bool(self.lib.fake_is_live(p))
+
+    def prefill(self, shape, T, perm=False):
+        s = smoe_amd.make_shape(shape["d_model"], shape["n_experts"], shape["top_k"], shape["d_ff"])
+        off, _raw, stride = smoe_amd.blob_layout(shape["d_model"], shape["d_ff"])
+        layer = smoe_amd.make_layer(DEV, DEV, DEV, stride, off)
+        p = DEV if perm else None
+        return self.lib.smoe_hip_moe_prefill(self.ctx, C.byref(s), C.byref(layer), DEV, T, None, None, p, p, p, p)
+
+
+@pytest.fixture
+def bridge(built):
+    b = Bridge(built)
+    yield b
+    b.close()
+
+
+@pytest.mark.parametrize("T,dispatches", [(256, 1), (257, 2), (4096, 2)])
+def test_profile_times_every_dispatch_of_a_launcher(bridge, T, dispatches):
+    """The permute of several segments takes two dispatches: both are timed, as one launch."""
+    L = bridge.lib
+    assert L.smoe_hip_profile_enable(bridge.ctx, 1) == 0
+    calls = 5000 if T == 257 else 3      # (past the ring of event slots)
+    for _ in range(calls):
+        assert bridge.prefill(SHAPE_30B, T) == 0
+    n, ms = C.c_uint64(), C.c_double()
+    for kind, each in ((smoe_amd.KERNEL_PERMUTE, dispatches), (smoe_amd.KERNEL_ROUTE, 1), (smoe_amd.KERNEL_SCATTER, 1)):
+        assert L.smoe_hip_profile_read(bridge.ctx, kind, C.byref(n), C.byref(ms)) == 0
+        assert (n.value, ms.value) == (calls, float(calls * each))    # the fake dispatch takes 1 ms
+    assert L.smoe_hip_profile_enable(bridge.ctx, 0) == 0
