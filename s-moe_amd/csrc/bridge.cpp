@@ -43,26 +43,43 @@ struct DeviceScratch {
     uint64_t* lx = nullptr;      // one-launch layer exchange words (lx_words), zero at allocation
 };
 
+// a device buffer of n elements
+template <typename T>
+struct Buf {
+    T* p = nullptr;
+    size_t n = 0;
+    T* grown = nullptr;              // a longer one that is to take its place (ensure_prefill_scratch)
+};
+
 // prefill / permute scratch for one batch of up to T tokens (P = T * K pairs)
 struct PrefillScratch {
-    uint32_t D = 0, E = 0, K = 0, I = 0, T = 0;
-    uint16_t* x_hi = nullptr;       // [T x D] f16
-    uint16_t* x_lo = nullptr;
-    float* x_sc = nullptr;          // [T] row scales
-    float* logits = nullptr;        // [T x E] router logits (short batches)
-    uint32_t* rt_ctr = nullptr;     // [T] route counters (zero between launches)
-    uint32_t* ids = nullptr;        // [T x K]
-    float* w = nullptr;             // [T x K]
-    uint32_t* offsets = nullptr;    // [E + 1]
-    uint4* units = nullptr;         // [unit_slots] grouped GEMM work list
-    uint32_t* seg_cnt = nullptr;    // [perm_segments x E] pairs per segment
-    uint32_t* pairs = nullptr;      // [P] sorted pair ids
-    float* h = nullptr;             // [P x I]
-    uint16_t* h_hi = nullptr;       // [P x I] f16
-    uint16_t* h_lo = nullptr;
-    float* h_sc = nullptr;          // [P] row scales
-    float* y = nullptr;             // [P x D]
+    Buf<uint16_t> x_hi, x_lo;        // [T x D] f16
+    Buf<float> x_sc;                 // [T] row scales
+    Buf<float> logits;               // [T x E] router logits (short batches)
+    Buf<uint32_t> rt_ctr;            // [T] route counters (zero between launches)
+    Buf<uint32_t> ids;               // [P]
+    Buf<float> w;                    // [P]
+    Buf<uint32_t> offsets;           // [E + 1]
+    Buf<uint4> units;                // [unit_slots] grouped GEMM work list
+    Buf<uint32_t> seg_cnt;           // [perm_segments x E] pairs per segment
+    Buf<uint32_t> pairs;             // [P] sorted pair ids
+    Buf<float> h;                    // [P x I]
+    Buf<uint16_t> h_hi, h_lo;        // [P x I] f16
+    Buf<float> h_sc;                 // [P] row scales
+    Buf<float> y;                    // [P x D]
 };
+
+// f(buffer, elements that a pass of T tokens of shape s needs), until one is false
+template <typename F>
+bool each_prefill_buf(PrefillScratch& c, const SmoeMoeShape* s, uint32_t T, F&& f)
+{
+    const size_t E = s->n_experts, x = size_t(T) * s->d_model, P = size_t(T) * s->top_k, h = P * s->d_ff;
+    const uint32_t P32 = static_cast<uint32_t>(P), E32 = s->n_experts;
+    return f(c.x_hi, x) && f(c.x_lo, x) && f(c.x_sc, size_t(T)) && f(c.logits, T * E) && f(c.rt_ctr, size_t(T)) &&
+           f(c.ids, P) && f(c.w, P) && f(c.offsets, E + 1) && f(c.units, size_t(smoe::unit_slots(P32, E32, ~0u))) &&
+           f(c.seg_cnt, smoe::perm_segments(P32, E32) * E) && f(c.pairs, P) && f(c.h, h) && f(c.h_hi, h) &&
+           f(c.h_lo, h) && f(c.h_sc, P) && f(c.y, P * s->d_model);
+}
 
 // the chained decode kernel's device copy of the layer table
 struct LayerTable {
@@ -198,25 +215,14 @@ void free_device_scratch(DeviceScratch& s)
     s = DeviceScratch{};
 }
 
-void free_prefill_scratch(PrefillScratch& s)
+void free_prefill_scratch(PrefillScratch& c)
 {
-    dfree(s.x_hi);
-    dfree(s.x_lo);
-    dfree(s.x_sc);
-    dfree(s.logits);
-    dfree(s.rt_ctr);
-    dfree(s.ids);
-    dfree(s.w);
-    dfree(s.offsets);
-    dfree(s.units);
-    dfree(s.seg_cnt);
-    dfree(s.pairs);
-    dfree(s.h);
-    dfree(s.h_hi);
-    dfree(s.h_lo);
-    dfree(s.h_sc);
-    dfree(s.y);
-    s = PrefillScratch{};
+    const SmoeMoeShape none{};
+    each_prefill_buf(c, &none, 0, [](auto& b, size_t) {
+        dfree(b.p);
+        b.n = 0;
+        return true;
+    });
 }
 
 // reference-surface shape check (kernels.metal:146-152, metal_bridge.mm:460-461)
@@ -284,36 +290,35 @@ uint32_t prefill_max_tokens(uint32_t E, uint32_t K)
     return lo;
 }
 
+// Scratch for passes of T tokens of this shape.  Every buffer grows by itself, to
+// what this call needs of it: a capacity kept as the largest T, K, D and I of all
+// calls would make a long pass of a narrow layer and a short one of a wide layer
+// together ask for a long pass of the wide one.
 int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T)
 {
     PrefillScratch& c = ctx->ps;
-    if (c.x_hi && c.D >= s->d_model && c.E >= s->n_experts && c.K >= s->top_k && c.I >= s->d_ff && c.T >= T)
-        return SMOE_OK;
+    if (each_prefill_buf(c, s, T, [](auto& b, size_t n) { return b.n >= n; })) return SMOE_OK;
     if (stream_capturing(ctx->stream)) return SMOE_ERR_CAPTURE;
     if (!hip_ok(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return SMOE_ERR_HIP;
-    PrefillScratch n;
-    n.D = std::max(c.D, s->d_model);
-    n.E = std::max(c.E, s->n_experts);
-    n.K = std::max(c.K, s->top_k);
-    n.I = std::max(c.I, s->d_ff);
-    n.T = std::max(c.T, T);
+    auto grow = [&] {
+        bool ok = each_prefill_buf(c, s, T, [&](auto& b, size_t n) { return b.n >= n || dalloc(ctx, &b.grown, n); });
+        if (ok && c.rt_ctr.grown) ok = hip_ok(ctx, hipMemset(c.rt_ctr.grown, 0, T * sizeof(uint32_t)), "hipMemset");
+        each_prefill_buf(c, s, T, [&](auto& b, size_t n) {
+            if (b.grown && ok) {
+                dfree(b.p);
+                b.p = b.grown;
+                b.n = n;
+                b.grown = nullptr;
+            }
+            dfree(b.grown);
+            return true;
+        });
+        return ok;
+    };
+    if (grow()) return SMOE_OK;
+    // not beside what the context holds: in its place
     free_prefill_scratch(c);
-    const size_t T_ = n.T, P = T_ * n.K;   // (at most 4096 x 16: pass_max_tokens)
-    const bool ok = dalloc(ctx, &n.x_hi, T_ * n.D) &&
-                    dalloc(ctx, &n.x_lo, T_ * n.D) && dalloc(ctx, &n.x_sc, T_) &&
-                    dalloc(ctx, &n.ids, P) && dalloc(ctx, &n.w, P) && dalloc(ctx, &n.offsets, size_t(n.E) + 1) &&
-                    dalloc(ctx, &n.units, size_t(smoe::unit_slots(P, n.E, ~0u))) &&
-                    dalloc(ctx, &n.seg_cnt, size_t(smoe::perm_segments(P, n.E)) * n.E) &&
-                    dalloc(ctx, &n.pairs, P) && dalloc(ctx, &n.h, P * n.I) && dalloc(ctx, &n.h_hi, P * n.I) &&
-                    dalloc(ctx, &n.h_lo, P * n.I) && dalloc(ctx, &n.h_sc, P) && dalloc(ctx, &n.y, P * n.D) &&
-                    dalloc(ctx, &n.logits, T_ * n.E) && dalloc(ctx, &n.rt_ctr, T_) &&
-                    hip_ok(ctx, hipMemset(n.rt_ctr, 0, T_ * sizeof(uint32_t)), "hipMemset");
-    if (!ok) {
-        free_prefill_scratch(n);
-        return SMOE_ERR_HIP;
-    }
-    c = n;
-    return SMOE_OK;
+    return grow() ? SMOE_OK : SMOE_ERR_HIP;
 }
 
 // tokens of one prefill pass: an expert's weights stream once per pass, and its
@@ -1059,31 +1064,35 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
     for (uint32_t t0 = 0; t0 < n_tokens; t0 += tb) {
         const uint32_t T = std::min(tb, n_tokens - t0), P = T * d.K;
         float* hv = hidden + size_t(t0) * d.D;
-        uint32_t* ids = ids_out ? ids_out + size_t(t0) * d.K : s.ids;
-        float* w = weights_out ? weights_out + size_t(t0) * d.K : s.w;
-        uint32_t* offs = expert_offsets ? expert_offsets : s.offsets;
+        uint32_t* ids = ids_out ? ids_out + size_t(t0) * d.K : s.ids.p;
+        float* w = weights_out ? weights_out + size_t(t0) * d.K : s.w.p;
+        uint32_t* offs = expert_offsets ? expert_offsets : s.offsets.p;
         if (!timed(ctx, SMOE_KERNEL_ROUTE, "route",
                    [&] {
-                       return smoe::launch_route(d, L, hv, T, s.x_hi, s.x_lo, s.x_sc, ids, w, s.logits, s.rt_ctr, st);
+                       return smoe::launch_route(d, L, hv, T, s.x_hi.p, s.x_lo.p, s.x_sc.p, ids, w, s.logits.p,
+                                                 s.rt_ctr.p, st);
                    }) ||
             !timed(ctx, SMOE_KERNEL_PERMUTE, "permute", [&] {
                 // one workgroup where its other outputs are wanted, else in segments
                 // (5.2 against 9.4 us at 512 tokens of the 30B shape, 4.4 against 5.3 at 64)
                 if (want_perm)
-                    return smoe::launch_permute(ids, w, P, d.K, d.E, offs, s.pairs, sorted_tokens, nullptr, union_ids,
-                                                union_size, s.units, few, ctx->d_err, st);
-                return smoe::launch_permute_seg(ids, P, d.E, offs, s.pairs, s.units, few, s.seg_cnt, ctx->d_err, st);
+                    return smoe::launch_permute(ids, w, P, d.K, d.E, offs, s.pairs.p, sorted_tokens, nullptr,
+                                                union_ids, union_size, s.units.p, few, ctx->d_err, st);
+                return smoe::launch_permute_seg(ids, P, d.E, offs, s.pairs.p, s.units.p, few, s.seg_cnt.p, ctx->d_err,
+                                                st);
             }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_GATE_UP, "grouped_gate_up", [&] {
-                return smoe::launch_grouped_gate_up(d, L, P, few, s.units, s.pairs, s.x_hi, s.x_lo, s.x_sc, s.h, st);
+                return smoe::launch_grouped_gate_up(d, L, P, few, s.units.p, s.pairs.p, s.x_hi.p, s.x_lo.p, s.x_sc.p,
+                                                    s.h.p, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SPLIT, "split(h)",
-                   [&] { return smoe::launch_split_rows(s.h, P, d.I, s.h_hi, s.h_lo, s.h_sc, st); }) ||
+                   [&] { return smoe::launch_split_rows(s.h.p, P, d.I, s.h_hi.p, s.h_lo.p, s.h_sc.p, st); }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_DOWN, "grouped_down", [&] {
-                return smoe::launch_grouped_down(d, L, P, few, s.units, s.pairs, s.h_hi, s.h_lo, s.h_sc, s.y, st);
+                return smoe::launch_grouped_down(d, L, P, few, s.units.p, s.pairs.p, s.h_hi.p, s.h_lo.p, s.h_sc.p,
+                                                 s.y.p, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SCATTER, "combine",
-                   [&] { return smoe::launch_combine_pairs(s.y, w, T, d.K, d.D, hv, st); }))
+                   [&] { return smoe::launch_combine_pairs(s.y.p, w, T, d.K, d.D, hv, st); }))
             return SMOE_ERR_HIP;
         ctx->dispatches.fetch_add(uint64_t(P), std::memory_order_relaxed);
     }

@@ -92,3 +92,28 @@ def test_profile_times_every_dispatch_of_a_launcher(bridge, T, dispatches):
         assert L.smoe_hip_profile_read(bridge.ctx, kind, C.byref(n), C.byref(ms)) == 0
         assert (n.value, ms.value) == (calls, float(calls * each))    # the fake dispatch takes 1 ms
     assert L.smoe_hip_profile_enable(bridge.ctx, 0) == 0
+
+
+def prefill_bytes(bridge, shape, T):
+    """What a context that only runs passes of T tokens of this shape holds for them."""
+    before = bridge.count("live")
+    assert bridge.prefill(shape, T) == 0
+    return bridge.count("live") - before
+
+
+def test_prefill_scratch_is_what_the_calls_need(built):
+    """A long pass of a narrow layer, then a short pass of a wide layer with more experts a token: the
+    scratch holds the larger of the two in every buffer, not a long pass of the wide layer, and a
+    budget of little more than that is enough."""
+    narrow, wide = SHAPE_30B, dict(d_model=8192, n_experts=64, top_k=16, d_ff=4096)
+    sizes = []
+    for shape, T in ((narrow, 4096), (wide, 16)):
+        b = Bridge(built)
+        sizes.append(prefill_bytes(b, shape, T))
+        b.close()
+    b = Bridge(built)
+    b.budget(b.count("live") + int(1.1 * sum(sizes)))
+    assert b.prefill(narrow, 4096) == 0
+    assert b.prefill(wide, 16) == 0
+    assert b.prefill(narrow, 4096) == 0 and b.count("T") == 4096
+    b.close()
