@@ -67,6 +67,7 @@ struct PrefillScratch {
     Buf<uint16_t> h_hi, h_lo;        // [P x I] f16
     Buf<float> h_sc;                 // [P] row scales
     Buf<float> y;                    // [P x D]
+    size_t denied = ~size_t(0);      // bytes of the smallest long pass that could not be had
 };
 
 // f(buffer, elements that a pass of T tokens of shape s needs), until one is false
@@ -293,12 +294,21 @@ uint32_t prefill_max_tokens(uint32_t E, uint32_t K)
 // Scratch for passes of T tokens of this shape.  Every buffer grows by itself, to
 // what this call needs of it: a capacity kept as the largest T, K, D and I of all
 // calls would make a long pass of a narrow layer and a short one of a wide layer
-// together ask for a long pass of the wide one.
-int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T)
+// together ask for a long pass of the wide one.  `or_shorter`: the caller can do
+// with shorter passes, so what the context holds stays if T cannot be had, and
+// that much is not asked for again (each layer of each call would synchronise and
+// fail an allocation).
+int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T, bool or_shorter)
 {
     PrefillScratch& c = ctx->ps;
     if (each_prefill_buf(c, s, T, [](auto& b, size_t n) { return b.n >= n; })) return SMOE_OK;
     if (stream_capturing(ctx->stream)) return SMOE_ERR_CAPTURE;
+    size_t bytes = 0;
+    each_prefill_buf(c, s, T, [&](auto& b, size_t n) {
+        bytes += n * sizeof(*b.p);
+        return true;
+    });
+    if (or_shorter && bytes >= c.denied) return SMOE_ERR_HIP;
     if (!hip_ok(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return SMOE_ERR_HIP;
     auto grow = [&] {
         bool ok = each_prefill_buf(c, s, T, [&](auto& b, size_t n) { return b.n >= n || dalloc(ctx, &b.grown, n); });
@@ -316,6 +326,11 @@ int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T)
         return ok;
     };
     if (grow()) return SMOE_OK;
+    (void)hipGetLastError();
+    if (or_shorter) {
+        c.denied = bytes;
+        return SMOE_ERR_HIP;
+    }
     // not beside what the context holds: in its place
     free_prefill_scratch(c);
     return grow() ? SMOE_OK : SMOE_ERR_HIP;
@@ -1049,13 +1064,12 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
     // passes of equal length, as few as wmax allows
     const uint32_t wmax = want_perm ? tmax : pass_max_tokens(d.K), passes = (n_tokens + wmax - 1) / wmax;
     uint32_t tb = (n_tokens + passes - 1) / passes;
-    rc = ensure_prefill_scratch(ctx, shape, tb);
+    rc = ensure_prefill_scratch(ctx, shape, tb, tb > tmax);
     if (rc != SMOE_OK && tb > tmax) {
         // no scratch for passes that long (out of memory, or a capture with the
         // scratch of shorter ones): results do not depend on the length
-        (void)hipGetLastError();
         tb = tmax;
-        rc = ensure_prefill_scratch(ctx, shape, tb);
+        rc = ensure_prefill_scratch(ctx, shape, tb, false);
     }
     if (rc != SMOE_OK) return rc;
     const uint32_t few = smoe::few_units(d);

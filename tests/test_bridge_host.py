@@ -117,3 +117,27 @@ def test_prefill_scratch_is_what_the_calls_need(built):
     assert b.prefill(wide, 16) == 0
     assert b.prefill(narrow, 4096) == 0 and b.count("T") == 4096
     b.close()
+
+
+def test_long_pass_that_cannot_be_had_is_not_asked_for_again(built):
+    """Where there is memory for passes of 736 tokens only, a longer prompt runs in those: the scratch of
+    the calls before stays, and later calls neither allocate nor synchronise."""
+    b = Bridge(built)
+    short = prefill_bytes(b, SHAPE_30B, 736)
+    b.close()
+    b = Bridge(built)
+    b.budget(b.count("live") + int(1.5 * short))
+    assert b.prefill(SHAPE_30B, 736) == 0
+    x_hi, frees = b.count("x_hi"), b.count("frees")
+    assert b.prefill(SHAPE_30B, 4000) == 0
+    assert b.count("failed") > 0 and b.count("T") == 4000 % 736
+    assert b.count("x_hi") == x_hi and b.live(x_hi)
+    held = b.count("live")
+    state = [b.count(w) for w in ("mallocs", "frees", "failed", "syncs")]
+    for T in (4000, 4096, 700, 4000):
+        assert b.prefill(SHAPE_30B, T) == 0
+        assert [b.count(w) for w in ("mallocs", "frees", "failed", "syncs")] == state, T
+    assert b.count("x_hi") == x_hi and b.count("live") == held
+    # short calls of other shapes that do fit are unaffected
+    assert b.prefill(dict(d_model=512, n_experts=8, top_k=2, d_ff=256), 100) == 0 and b.count("T") == 100
+    b.close()
