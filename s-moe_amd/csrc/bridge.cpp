@@ -48,7 +48,9 @@ template <typename T>
 struct Buf {
     T* p = nullptr;
     size_t n = 0;
+    bool captured = false;           // a captured graph may hold p: it lives until the context is destroyed
     T* grown = nullptr;              // a longer one that is to take its place (ensure_prefill_scratch)
+    size_t grown_n = 0;
 };
 
 // prefill / permute scratch for one batch of up to T tokens (P = T * K pairs)
@@ -68,6 +70,7 @@ struct PrefillScratch {
     Buf<float> h_sc;                 // [P] row scales
     Buf<float> y;                    // [P x D]
     size_t denied = ~size_t(0);      // bytes of the smallest long pass that could not be had
+    std::vector<void*> retired;      // outgrown buffers that captured graphs may hold
 };
 
 // f(buffer, elements that a pass of T tokens of shape s needs), until one is false
@@ -216,14 +219,29 @@ void free_device_scratch(DeviceScratch& s)
     s = DeviceScratch{};
 }
 
-void free_prefill_scratch(PrefillScratch& c)
+// gives the buffer back, or keeps it for the graphs that may hold it
+template <typename T>
+void drop_buf(PrefillScratch& c, Buf<T>& b)
+{
+    if (b.p && b.captured) c.retired.push_back(b.p);
+    else dfree(b.p);
+    b = Buf<T>{};
+}
+
+void drop_prefill_scratch(PrefillScratch& c)
 {
     const SmoeMoeShape none{};
-    each_prefill_buf(c, &none, 0, [](auto& b, size_t) {
-        dfree(b.p);
-        b.n = 0;
+    each_prefill_buf(c, &none, 0, [&](auto& b, size_t) {
+        drop_buf(c, b);
         return true;
     });
+}
+
+void free_prefill_scratch(PrefillScratch& c)
+{
+    drop_prefill_scratch(c);
+    for (void* p : c.retired) dfree(p);
+    c.retired.clear();
 }
 
 // reference-surface shape check (kernels.metal:146-152, metal_bridge.mm:460-461)
@@ -310,30 +328,38 @@ int ensure_prefill_scratch(SmoeMetalCtx* ctx, const SmoeMoeShape* s, uint32_t T,
     });
     if (or_shorter && bytes >= c.denied) return SMOE_ERR_HIP;
     if (!hip_ok(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize")) return SMOE_ERR_HIP;
-    auto grow = [&] {
-        bool ok = each_prefill_buf(c, s, T, [&](auto& b, size_t n) { return b.n >= n || dalloc(ctx, &b.grown, n); });
-        if (ok && c.rt_ctr.grown) ok = hip_ok(ctx, hipMemset(c.rt_ctr.grown, 0, T * sizeof(uint32_t)), "hipMemset");
-        each_prefill_buf(c, s, T, [&](auto& b, size_t n) {
+    // a buffer that stays behind for captured graphs is followed by one twice as
+    // long at least, so that all of those take no more than the present ones
+    auto grow = [&](bool twice) {
+        bool ok = each_prefill_buf(c, s, T, [&](auto& b, size_t n) {
+            if (b.n >= n) return true;
+            b.grown_n = twice && b.captured ? std::max(n, 2 * b.n) : n;
+            return dalloc(ctx, &b.grown, b.grown_n);
+        });
+        if (ok && c.rt_ctr.grown)
+            ok = hip_ok(ctx, hipMemset(c.rt_ctr.grown, 0, c.rt_ctr.grown_n * sizeof(uint32_t)), "hipMemset");
+        each_prefill_buf(c, s, T, [&](auto& b, size_t) {
             if (b.grown && ok) {
-                dfree(b.p);
-                b.p = b.grown;
+                auto* p = b.grown;
+                const size_t n = b.grown_n;
+                drop_buf(c, b);
+                b.p = p;
                 b.n = n;
-                b.grown = nullptr;
             }
             dfree(b.grown);
             return true;
         });
         return ok;
     };
-    if (grow()) return SMOE_OK;
+    if (grow(true)) return SMOE_OK;
     (void)hipGetLastError();
     if (or_shorter) {
         c.denied = bytes;
         return SMOE_ERR_HIP;
     }
     // not beside what the context holds: in its place
-    free_prefill_scratch(c);
-    return grow() ? SMOE_OK : SMOE_ERR_HIP;
+    drop_prefill_scratch(c);
+    return grow(false) ? SMOE_OK : SMOE_ERR_HIP;
 }
 
 // tokens of one prefill pass: an expert's weights stream once per pass, and its
@@ -1075,6 +1101,8 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
     const uint32_t few = smoe::few_units(d);
     PrefillScratch& s = ctx->ps;
     hipStream_t st = ctx->stream;
+    if (stream_capturing(st))
+        each_prefill_buf(s, shape, tb, [](auto& b, size_t) { return b.captured = true; });
     for (uint32_t t0 = 0; t0 < n_tokens; t0 += tb) {
         const uint32_t T = std::min(tb, n_tokens - t0), P = T * d.K;
         float* hv = hidden + size_t(t0) * d.D;

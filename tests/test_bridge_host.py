@@ -141,3 +141,36 @@ def test_long_pass_that_cannot_be_had_is_not_asked_for_again(built):
     # short calls of other shapes that do fit are unaffected
     assert b.prefill(dict(d_model=512, n_experts=8, top_k=2, d_ff=256), 100) == 0 and b.count("T") == 100
     b.close()
+
+
+def test_captured_prefill_keeps_its_scratch(bridge):
+    """A graph holds the scratch it was captured with: a later, longer call grows the scratch beside it.
+    Capturing one length after the other, ascending, keeps no more behind than the present scratch."""
+    assert bridge.prefill(SHAPE_30B, 1000) == 0
+    held = []
+    bridge.capturing(True)
+    assert bridge.prefill(SHAPE_30B, 512) == 0
+    bridge.capturing(False)
+    held += [bridge.count("x_hi"), bridge.count("y")]
+    assert bridge.prefill(SHAPE_30B, 4000) == 0
+    assert bridge.count("x_hi") != held[0] and all(bridge.live(p) for p in held)
+    assert bridge.prefill(dict(d_model=4096, n_experts=128, top_k=8, d_ff=1536), 4096) == 0
+    assert all(bridge.live(p) for p in held)
+
+
+def test_ascending_captures_are_bounded(built):
+    b = Bridge(built)
+    full = prefill_bytes(b, SHAPE_30B, 1024)
+    b.close()
+    b = Bridge(built)
+    base = b.count("live")
+    held = []
+    for T in range(1, 513):
+        assert b.prefill(SHAPE_30B, T) == 0
+        b.capturing(True)
+        assert b.prefill(SHAPE_30B, T) == 0
+        b.capturing(False)
+        held.append(b.count("y"))
+    assert all(b.live(p) for p in held)
+    assert b.count("live") - base <= 2 * full
+    b.close()

@@ -46,3 +46,43 @@ def test_prefill_stack_matches_per_layer_calls_chunks_and_oracle(ctx, oracle):
         ctx.moe_prefill_stack(layers[0].shape, [l.layer for l in layers], chunked[t0:].data_ptr(), n)
     ctx.synchronize()
     assert torch.equal(chunked, full)
+
+
+def test_prefill_graphs_and_longer_calls(ctx):
+    """Prefill captured at 300 tokens and at 1500 (whose scratch is not there under capture: passes of what one
+    permute workgroup holds, 736 tokens), then an eager call of 4500 tokens that grows the scratch: every
+    replay, with eager calls between them, equals the eager result bit for bit."""
+    import smoe_amd
+    D, E, K, I = 256, 128, 8, 128
+    layer = Layer(ctx, D, E, K, I, layer_id=95, host=False)
+    x = hidden_states(ctx, 500, D, index0=700).repeat(9, 1)
+    x[:, 0] += torch.arange(len(x), device="cuda") * 1e-3
+    ref = x.clone()
+    ctx.moe_prefill(layer.shape, layer.layer, ref.data_ptr(), len(ref))
+    ctx.synchronize()
+    own = smoe_amd.Context()
+    s = torch.cuda.Stream()
+    own.set_stream(s.cuda_stream)
+    bufs = {T: x[:T].clone() for T in (300, 1500)}
+    graphs = {T: torch.cuda.CUDAGraph() for T in bufs}
+    junk = x.clone()
+    torch.cuda.synchronize()
+    own.moe_prefill(layer.shape, layer.layer, junk.data_ptr(), 900)
+    own.synchronize()
+    with torch.cuda.stream(s):
+        for T, g in graphs.items():
+            with torch.cuda.graph(g, stream=s):
+                own.moe_prefill(layer.shape, layer.layer, bufs[T].data_ptr(), T)
+    torch.cuda.synchronize()
+    for rep in range(4):
+        junk.copy_(x)
+        torch.cuda.synchronize()
+        own.moe_prefill(layer.shape, layer.layer, junk.data_ptr(), 4500 if rep % 2 == 0 else 700)
+        own.synchronize()
+        for T, g in graphs.items():
+            bufs[T].copy_(x[:T])
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(bufs[T], ref[:T]), (rep, T)
+    own.close()
