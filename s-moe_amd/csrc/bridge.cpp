@@ -1087,14 +1087,18 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
     // the permute outputs describe one pass: they need all tokens in one batch
     const bool want_perm = expert_offsets || sorted_tokens || union_ids || union_size;
     if (want_perm && n_tokens > tmax) return SMOE_ERR_SHAPE;
-    // passes of equal length, as few as wmax allows
+    // passes of equal length, as few as wmax allows; the scratch is that of the
+    // longest pass a call of n_tokens or fewer takes, so that all of them can be
+    // captured after this one
     const uint32_t wmax = want_perm ? tmax : pass_max_tokens(d.K), passes = (n_tokens + wmax - 1) / wmax;
+    const uint32_t longest = std::min(n_tokens, wmax);
     uint32_t tb = (n_tokens + passes - 1) / passes;
-    rc = ensure_prefill_scratch(ctx, shape, tb, tb > tmax);
-    if (rc != SMOE_OK && tb > tmax) {
+    const uint32_t shorter = std::min(tb, tmax);
+    rc = ensure_prefill_scratch(ctx, shape, longest, longest > shorter);
+    if (rc != SMOE_OK && longest > shorter) {
         // no scratch for passes that long (out of memory, or a capture with the
         // scratch of shorter ones): results do not depend on the length
-        tb = tmax;
+        tb = shorter;
         rc = ensure_prefill_scratch(ctx, shape, tb, false);
     }
     if (rc != SMOE_OK) return rc;

@@ -174,3 +174,17 @@ def test_ascending_captures_are_bounded(built):
     assert all(b.live(p) for p in held)
     assert b.count("live") - base <= 2 * full
     b.close()
+
+
+@pytest.mark.parametrize("shape", [SHAPE_30B, dict(d_model=256, n_experts=8, top_k=2, d_ff=128)])
+def test_capture_of_shorter_calls_after_a_longer_one(built, shape):
+    """After a call of n tokens, every call of at most n tokens can be captured."""
+    for n in (300, 737, 2500, 4096, 4097, 5000, 9000):
+        b = Bridge(built)
+        assert b.prefill(shape, n) == 0
+        b.capturing(True)
+        for T in (1, 299, 300, 736, 2049, 2500, 4000, 4096, 4097, 5000, 9000):
+            if T <= n:
+                assert b.prefill(shape, T) == 0, (n, T)
+        b.capturing(False)
+        b.close()
