@@ -418,13 +418,18 @@ bool timed(SmoeMetalCtx* ctx, uint32_t kind, const char* what, F&& launch)
     return hip_ok(ctx, e, what);
 }
 
-// `in`: the dispatch's pinned input, in use until the handle is done
-void* record_handle(SmoeMetalCtx* ctx, SmoeMetalCtx::HostIn* in)
+// The end of a dispatch that staged its input in `in`: its handle, until which the
+// entry is in use.  Without one (a launch or the event failed) nothing would say
+// when the queued copy has read the entry, so that is waited for here.
+void* end_dispatch(SmoeMetalCtx* ctx, SmoeMetalCtx::HostIn* in, bool launched)
 {
     const uint64_t h = ++ctx->seq;
-    if (!hip_ok(ctx, hipEventRecord(ctx->ev[h % kEvents], ctx->stream), "hipEventRecord")) return nullptr;
-    in->handle = h;
-    return reinterpret_cast<void*>(static_cast<uintptr_t>(h));
+    if (launched && hip_ok(ctx, hipEventRecord(ctx->ev[h % kEvents], ctx->stream), "hipEventRecord")) {
+        in->handle = h;
+        return reinterpret_cast<void*>(static_cast<uintptr_t>(h));
+    }
+    (void)hipStreamSynchronize(ctx->stream);
+    return nullptr;
 }
 
 bool wait_handle(SmoeMetalCtx* ctx, void* handle)
@@ -464,17 +469,17 @@ void* dispatch_group(SmoeMetalCtx* ctx, const smoe::ExpertTable& tbl, uint32_t n
     const MoeDims d{gate_cols, 0, n, gate_rows, group_size, 0};
     SmoeMetalCtx::HostIn* in = stage_input(ctx, input_vec, ctx->d_input, gate_cols);
     if (!in) return nullptr;
-    if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up", [&] {
-            return smoe::launch_gate_up(d, tbl, n, ctx->d_input, ctx->d_hidden, ctx->slot_stride, ctx->stream);
-        }))
-        return nullptr;
-    if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down", [&] {
-            return smoe::launch_down_slots(d, tbl, n, ctx->d_hidden, ctx->slot_stride, ctx->h_output, ctx->slot_stride,
-                                           ctx->stream);
-        }))
-        return nullptr;
-    ctx->dispatches.fetch_add(n, std::memory_order_relaxed);
-    return record_handle(ctx, in);
+    const bool ok = timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up",
+                          [&] {
+                              return smoe::launch_gate_up(d, tbl, n, ctx->d_input, ctx->d_hidden, ctx->slot_stride,
+                                                          ctx->stream);
+                          }) &&
+                    timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down", [&] {
+                        return smoe::launch_down_slots(d, tbl, n, ctx->d_hidden, ctx->slot_stride, ctx->h_output,
+                                                       ctx->slot_stride, ctx->stream);
+                    });
+    if (ok) ctx->dispatches.fetch_add(n, std::memory_order_relaxed);
+    return end_dispatch(ctx, in, ok);
 }
 
 }  // namespace
@@ -617,16 +622,17 @@ extern "C" void* smoe_metal_fused_ffn_batch(SmoeMetalCtx* ctx, const uint8_t* pa
         return nullptr;
     SmoeMetalCtx::HostIn* in = stage_input(ctx, input_mat, ctx->d_batch_in, size_t(batch) * gate_cols);
     if (!in) return nullptr;
-    if (!timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up(batch)", [&] {
-            return smoe::launch_gate_up_tokens(d, e, ctx->d_batch_in, ctx->d_batch_hidden, batch, ctx->stream);
-        }))
-        return nullptr;
-    if (!timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down(batch)", [&] {
-            return smoe::launch_down_tokens(d, e, ctx->d_batch_hidden, ctx->h_batch_out, batch, ctx->stream);
-        }))
-        return nullptr;
-    ctx->dispatches.fetch_add(1, std::memory_order_relaxed);
-    return record_handle(ctx, in);
+    const bool ok = timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up(batch)",
+                          [&] {
+                              return smoe::launch_gate_up_tokens(d, e, ctx->d_batch_in, ctx->d_batch_hidden, batch,
+                                                                 ctx->stream);
+                          }) &&
+                    timed(ctx, SMOE_KERNEL_DOWN_SLOTS, "down(batch)", [&] {
+                        return smoe::launch_down_tokens(d, e, ctx->d_batch_hidden, ctx->h_batch_out, batch,
+                                                        ctx->stream);
+                    });
+    if (ok) ctx->dispatches.fetch_add(1, std::memory_order_relaxed);
+    return end_dispatch(ctx, in, ok);
 }
 
 extern "C" void smoe_metal_wait_ffn_batch(SmoeMetalCtx* ctx, void* handle, float* out_mat, uint32_t batch,

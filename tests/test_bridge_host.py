@@ -71,6 +71,15 @@ class Bridge:
         p = DEV if perm else None
         return self.lib.smoe_hip_moe_prefill(self.ctx, C.byref(s), C.byref(layer), DEV, T, None, None, p, p, p, p)
 
+    def group(self, n=2, D=2048, I=768):
+        x = np.ones(D, np.float32)
+        blobs = (smoe_amd.SmoeExpertBlob * n)(*[smoe_amd.SmoeExpertBlob(*[DEV] * 6, i) for i in range(n)])
+        return self.lib.smoe_metal_fused_ffn_group(self.ctx, blobs, n, x.ctypes.data, I, D, D, I, 64, 4)
+
+    def batch(self, n, D=2048, I=768):
+        x = np.ones((n, D), np.float32)
+        return self.lib.smoe_metal_fused_ffn_batch(self.ctx, *[DEV] * 6, x.ctypes.data, n, I, D, D, I, 64, 4)
+
 
 @pytest.fixture
 def bridge(built):
@@ -188,3 +197,20 @@ def test_capture_of_shorter_calls_after_a_longer_one(built, shape):
                 assert b.prefill(shape, T) == 0, (n, T)
         b.capturing(False)
         b.close()
+
+
+@pytest.mark.parametrize("fails,batch", [("gate_up", 0), ("down", 0), ("event_record", 0), ("gate_up_tokens", 9),
+                                         ("down_tokens", 9), ("event_record", 9)])
+def test_input_copy_of_a_failed_dispatch_is_waited_for(bridge, fails, batch):
+    """A dispatch that fails after its input's copy was queued has no handle that says when the copy has read
+    the pinned entry: the call waits for it, so that later dispatches may write there."""
+    call = (lambda: bridge.batch(batch)) if batch else bridge.group
+    assert call()
+    dispatches, syncs = bridge.lib.smoe_metal_kernel_dispatches(bridge.ctx), bridge.count("syncs")
+    bridge.lib.fake_fail(fails.encode())
+    assert call() is None and bridge.count("syncs") == syncs + 1
+    if fails != "event_record":
+        assert bridge.lib.smoe_metal_kernel_dispatches(bridge.ctx) == dispatches
+    for _ in range(8):
+        assert call()
+    assert bridge.count("syncs") == syncs + 1
