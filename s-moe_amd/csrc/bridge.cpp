@@ -445,7 +445,10 @@ bool wait_handle(SmoeMetalCtx* ctx, void* handle)
 // its own again on return) and queues the device copy.  A pageable hipMemcpyAsync
 // in its place costs the call about 10 us, a synchronous hipMemcpy of each
 // output as much again: a group of 8 experts took 143 us of which 16 were kernels.
-SmoeMetalCtx::HostIn* stage_input(SmoeMetalCtx* ctx, const float* src, float* dst, size_t n)
+// most: the longest input of this kind; an entry that is too short grows to that
+// at once (pinned memory takes longer to get than the dispatch does, and every
+// batch longer than those before it would wait for it in each entry).
+SmoeMetalCtx::HostIn* stage_input(SmoeMetalCtx* ctx, const float* src, float* dst, size_t n, size_t most)
 {
     SmoeMetalCtx::HostIn& in = ctx->h_in[ctx->h_in_next];
     ctx->h_in_next = (ctx->h_in_next + 1) % kHostIn;
@@ -454,11 +457,12 @@ SmoeMetalCtx::HostIn* stage_input(SmoeMetalCtx* ctx, const float* src, float* ds
     if (in.cap < n) {
         hfree(in.p);
         in.cap = 0;
-        if (!halloc(ctx, &in.p, n)) return nullptr;
-        in.cap = n;
+        if (!halloc(ctx, &in.p, most)) return nullptr;
+        in.cap = most;
     }
     std::memcpy(in.p, src, n * sizeof(float));
-    if (!hip_ok(ctx, smoe::launch_stage_in(in.p, dst, static_cast<uint32_t>(n), ctx->stream), "stage_in")) return nullptr;
+    if (!hip_ok(ctx, smoe::launch_stage_in(in.p, dst, static_cast<uint32_t>(n), ctx->stream), "stage_in"))
+        return nullptr;
     return &in;
 }
 
@@ -467,7 +471,7 @@ void* dispatch_group(SmoeMetalCtx* ctx, const smoe::ExpertTable& tbl, uint32_t n
                      uint32_t gate_rows, uint32_t gate_cols, uint32_t group_size)
 {
     const MoeDims d{gate_cols, 0, n, gate_rows, group_size, 0};
-    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_vec, ctx->d_input, gate_cols);
+    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_vec, ctx->d_input, gate_cols, SMOE_MAX_DIM);
     if (!in) return nullptr;
     const bool ok = timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up",
                           [&] {
@@ -620,7 +624,8 @@ extern "C" void* smoe_metal_fused_ffn_batch(SmoeMetalCtx* ctx, const uint8_t* pa
     const ExpertPtrs e{packed_gate, scales_gate, packed_up, scales_up, packed_down, scales_down, 0, 0};
     if (!ctx->h_batch_out && !halloc(ctx, &ctx->h_batch_out, size_t(SMOE_MAX_FFN_BATCH) * SMOE_MAX_FFN_BATCH_DIM))
         return nullptr;
-    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_mat, ctx->d_batch_in, size_t(batch) * gate_cols);
+    SmoeMetalCtx::HostIn* in = stage_input(ctx, input_mat, ctx->d_batch_in, size_t(batch) * gate_cols,
+                                           size_t(SMOE_MAX_FFN_BATCH) * gate_cols);
     if (!in) return nullptr;
     const bool ok = timed(ctx, SMOE_KERNEL_GATE_UP, "gate_up(batch)",
                           [&] {

@@ -214,3 +214,14 @@ def test_input_copy_of_a_failed_dispatch_is_waited_for(bridge, fails, batch):
     for _ in range(8):
         assert call()
     assert bridge.count("syncs") == syncs + 1
+
+
+def test_longer_batches_find_their_pinned_memory(bridge):
+    """The four input entries are as long as the longest dispatch of their kind from their first use on:
+    batches that grow by a token allocate no pinned memory of their own."""
+    for _ in range(4):
+        assert bridge.batch(2) and bridge.group(D=512, I=256)
+    n = bridge.count("host_mallocs")
+    for k in range(3, 65):
+        assert bridge.batch(k) and bridge.group(D=64 * k, I=256)
+    assert bridge.count("host_mallocs") == n and bridge.count("host_frees") <= n
