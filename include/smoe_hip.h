@@ -321,12 +321,18 @@ int smoe_hip_set_decode_engine(SmoeMetalCtx* ctx, int engine);
  * d_model]: per token RMSNorm + router + top-k, then the layer-major expert
  * grouping (token-by-expert permute, grouped expert GEMMs on MFMA, weighted
  * combine into the residual).  Tokens are processed in passes of up to 4096
- * (32768 / top_k if that is less); results do not depend on the pass size.
- * ids_out / weights_out [n_tokens x top_k] are optional.  Optional device outputs of the permute (these require all tokens
- * in one pass, else SMOE_ERR_SHAPE):
+ * (32768 / top_k if that is less), or, where the scratch for those cannot be
+ * had, of what one permute workgroup holds (below); results do not depend on the
+ * pass size.  Scratch grows on demand; under graph capture a call needs that of
+ * an earlier call of as many tokens (or of one permute workgroup's), else
+ * SMOE_ERR_CAPTURE.  ids_out / weights_out [n_tokens x top_k] are optional.
+ * Optional device outputs of the permute:
  *   expert_offsets [n_experts+1], sorted_tokens [n_tokens*top_k],
  *   union_ids [n_experts] (first-appearance order, prefill.cpp:55-68),
- *   union_size [1]. */
+ *   union_size [1].
+ * With any of them the call is one pass whose permute runs in one workgroup, and
+ * n_tokens is limited by that workgroup's tables as in smoe_hip_permute (736
+ * tokens at 128 experts and top_k 8); more gives SMOE_ERR_SHAPE. */
 int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape,
                          const SmoeMoeLayer* layer, float* hidden, uint32_t n_tokens,
                          uint32_t* ids_out, float* weights_out,

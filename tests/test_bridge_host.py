@@ -3,6 +3,7 @@ HIP runtime and launchers that only keep books (fake_hip.cpp), so that memory
 that runs out, launches that fail and stream capture can be forced."""
 import ctypes as C
 import os
+import re
 import shutil
 import subprocess
 
@@ -225,3 +226,12 @@ def test_longer_batches_find_their_pinned_memory(bridge):
     for k in range(3, 65):
         assert bridge.batch(k) and bridge.group(D=64 * k, I=256)
     assert bridge.count("host_mallocs") == n and bridge.count("host_frees") <= n
+
+
+def test_permute_outputs_take_the_tokens_that_the_header_states(bridge):
+    header = open(os.path.join(ROOT, "include", "smoe_hip.h")).read()
+    text = " ".join(header[:header.index("int smoe_hip_moe_prefill(")].replace("*", " ").split())
+    limit = int(re.search(r"\((\d+) tokens at 128 experts and top_k 8\); more gives SMOE_ERR_SHAPE", text).group(1))
+    assert bridge.prefill(SHAPE_30B, limit, perm=True) == 0 and bridge.count("T") == limit
+    assert bridge.prefill(SHAPE_30B, limit + 1, perm=True) == smoe_amd.SMOE_ERR_SHAPE
+    assert bridge.prefill(SHAPE_30B, limit + 1) == 0 and bridge.count("T") == limit + 1
