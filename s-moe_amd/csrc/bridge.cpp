@@ -1135,8 +1135,7 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
                 if (want_perm)
                     return smoe::launch_permute(ids, w, P, d.K, d.E, offs, s.pairs.p, sorted_tokens, nullptr,
                                                 union_ids, union_size, s.units.p, few, ctx->d_err, st);
-                return smoe::launch_permute_seg(ids, P, d.E, offs, s.pairs.p, s.units.p, few, s.seg_cnt.p, ctx->d_err,
-                                                st);
+                return smoe::launch_permute_seg(ids, P, d.E, s.pairs.p, s.units.p, few, s.seg_cnt.p, ctx->d_err, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_GATE_UP, "grouped_gate_up", [&] {
                 return smoe::launch_grouped_gate_up(d, L, P, few, s.units.p, s.pairs.p, s.x_hi.p, s.x_lo.p, s.x_sc.p,

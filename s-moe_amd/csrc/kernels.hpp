@@ -261,15 +261,15 @@ constexpr size_t permute_lds_bytes(uint32_t P, uint32_t E)
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
                           uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s);
-// The same offsets, sorted pairs and units in segments, one workgroup each, for
-// any P (seg_cnt [perm_segments(P, E) x E]).
+// The same sorted pairs and units in segments, one workgroup each, for any P
+// (seg_cnt [perm_segments(P, E) x E]).
 __host__ __device__ constexpr uint32_t perm_seg_chunks(uint32_t E) { return E <= 256 ? 32u : 16u; }
 constexpr uint32_t perm_segments(uint32_t P, uint32_t E)
 {
     return (P + 64u * perm_seg_chunks(E) - 1) / (64u * perm_seg_chunks(E));
 }
-hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
-                              uint4* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
+hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs, uint4* units,
+                              uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):
 // h [P x I] = silu(x G^T) * (x U^T); y [P x D] = h Dn^T, over the permute's
 // work list.

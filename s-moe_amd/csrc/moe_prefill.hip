@@ -699,8 +699,8 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
 //   k_perm_scatter  every workgroup adds up the counts of the segments before
 //                   its own and of all of them, scans the totals into the
 //                   expert offsets, and places its segment's pairs as
-//                   k_permute does.  Workgroup 0 also writes the offsets and
-//                   the grouped GEMMs' work list.
+//                   k_permute does.  Workgroup 0 also writes the grouped
+//                   GEMMs' work list.
 // A batch of one segment needs no counts from elsewhere: k_perm_scatter counts
 // it itself (ONE) and is the only launch (64 tokens of the 30B shape 115.9 ->
 // 113.5 us a call).
@@ -726,8 +726,8 @@ void k_perm_count(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, uint
 template <bool ONE>
 __global__ __launch_bounds__(PERM_THREADS)
 void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, const uint32_t* __restrict__ seg_cnt,
-                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs, uint4* __restrict__ units,
-                    uint32_t n_slots, uint32_t few_units, uint32_t* __restrict__ err)
+                    uint32_t* __restrict__ sorted_pairs, uint4* __restrict__ units, uint32_t n_slots,
+                    uint32_t few_units, uint32_t* __restrict__ err)
 {
     extern __shared__ uint32_t s_mem[];
     __shared__ uint32_t s_cap;
@@ -814,10 +814,7 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
         const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
         if (ok) sorted_pairs[s_cnt[e * CS + c] + rank] = (seg * CH + c) * 64 + lane;
     }
-    if (seg == 0) {
-        for (uint32_t e = threadIdx.x; e <= E; e += PERM_THREADS) offsets[e] = s_off[e];
-        write_units(s_off, s_unit, E, s_cap, units, n_slots);
-    }
+    if (seg == 0) write_units(s_off, s_unit, E, s_cap, units, n_slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -1616,20 +1613,20 @@ hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint3
     return hipGetLastError();
 }
 
-hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* offsets, uint32_t* sorted_pairs,
-                              uint4* units, uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
+hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs, uint4* units,
+                              uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
 {
     if (P == 0 || E == 0 || E > SMOE_TOPK_MAX_N) return hipErrorInvalidValue;
     const uint32_t nseg = perm_segments(P, E);
     const uint32_t slots = unit_slots(P, E, few_units);
     const uint32_t lds = (E * (perm_seg_chunks(E) | 1u) + 4 * E + 2) * static_cast<uint32_t>(sizeof(uint32_t));
     if (nseg == 1) {
-        launch_kernel_lds(k_perm_scatter<true>, dim3(1), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt, offsets,
+        launch_kernel_lds(k_perm_scatter<true>, dim3(1), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt,
                           sorted_pairs, units, slots, few_units, err);
         return hipGetLastError();
     }
     launch_kernel(k_perm_count, dim3(nseg), dim3(PERM_THREADS), s, ids, P, E, seg_cnt, err);
-    launch_kernel_lds(k_perm_scatter<false>, dim3(nseg), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt, offsets,
+    launch_kernel_lds(k_perm_scatter<false>, dim3(nseg), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt,
                       sorted_pairs, units, slots, few_units, err);
     return hipGetLastError();
 }

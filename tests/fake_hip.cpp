@@ -254,8 +254,8 @@ hipError_t launch_permute(const uint32_t*, const float*, uint32_t, uint32_t, uin
     ++st().permutes;
     return dispatch("permute");
 }
-hipError_t launch_permute_seg(const uint32_t*, uint32_t P, uint32_t E, uint32_t*, uint32_t*, uint4*, uint32_t, uint32_t*,
-                              uint32_t*, hipStream_t)
+hipError_t launch_permute_seg(const uint32_t*, uint32_t P, uint32_t E, uint32_t*, uint4*, uint32_t, uint32_t*, uint32_t*,
+                              hipStream_t)
 {
     ++st().permutes_seg;
     return dispatch("permute_seg", perm_segments(P, E) > 1 ? 2 : 1);
