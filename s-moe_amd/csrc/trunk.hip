@@ -483,9 +483,11 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // layout (134 MB of K and V, 16 query heads a KV head) takes 59 us, 27 of them its two
 // GEMVs, against 80 with k_attn_decode, whose two blocks per KV head and split, on
 // different XCDs, each read every row and whose dot products are the VALU's.
-// Sums run in chains of eight terms that are then added, as there: 3.73e-7 from
-// fp64 over 32768 positions (12 inputs) against 3.69e-7, 3.96e-7 against 3.95e-7
-// over 5000; in chains of 64 it was 4.4e-7.
+// Sums run in chains of eight terms that are then added, also over the splits
+// (k_attn_combine; one chain over them cost most here, with twice as many splits as
+// k_attn_decode takes): the layer is 3.50e-7 from fp64 over 32768 positions (16
+// inputs) against 3.69e-7 for k_attn_decode and one chain over the splits, 3.42e-7
+// against 3.49e-7 over 5000.
 template <int HD>
 __global__ __launch_bounds__(wide_waves(HD) * WAVE, 1)
 void k_attn_wide(AttnArgs p)
@@ -746,10 +748,19 @@ void k_attn_combine(const float* __restrict__ part_ml, const float* __restrict__
     const float M = wave_max(m_s);
     const float f = live ? __expf(m_s - M) : 0.f;
     const float L = wave_sum(f * l_s);
-    float o = 0.f;
+    // chains of eight splits, then pairwise: one chain of up to 64 rounds more than the
+    // sums inside a split do (30B layout, 32768 positions, layer: 3.32e-7 -> 3.08e-7
+    // from fp64; 235B layout 3.73e-7 -> 3.50e-7)
+    constexpr uint32_t C = 8;
+    float o[ATTN_MAX_SPLITS / C];
 #pragma unroll
-    for (uint32_t s = 0; s < ATTN_MAX_SPLITS; ++s) o = fmaf(readlane_f32(f, s), a[s], o);
-    out[static_cast<size_t>(h) * head_dim + d] = o * (1.0f / L);
+    for (uint32_t c = 0; c < ATTN_MAX_SPLITS / C; ++c) {
+        o[c] = readlane_f32(f, c * C) * a[c * C];
+#pragma unroll
+        for (uint32_t s = c * C + 1; s < (c + 1) * C; ++s) o[c] = fmaf(readlane_f32(f, s), a[s], o[c]);
+    }
+    const float t = ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
+    out[static_cast<size_t>(h) * head_dim + d] = t * (1.0f / L);
 }
 
 AttnPlan attn_plan(const AttnDims& a, uint32_t valid)
