@@ -724,11 +724,13 @@ hipError_t launch_moe_up(const MoeDims& d, const LayerDesc& L, const float* hidd
     if (d.group != 64 || d.E > SMOE_TOPK_MAX_N || d.I % UP_RB) return hipErrorInvalidValue;
     const uint32_t row_blocks = d.I / UP_RB;
     // Several row blocks a wave once the waves outnumber what the chip holds at
-    // two a SIMD (2048): the norm, the digits and the top-k, half of a wave's
+    // two a SIMD (2048; one a SIMD with four chunks a lane, D > 4096, where such a
+    // grid takes two rounds): the norm, the digits and the top-k, half of a wave's
     // VALU work with one block, are then done once per wave (11 tokens of the
     // 30B shape 52 -> 33 us, 24 tokens 107 -> 60; with waves for one or three a
-    // SIMD 40 and 36).  Grids between one and two a SIMD fold to one, whose logit
-    // exchange is XCD-local (2 tokens 14.0 -> 12.7).
+    // SIMD 40 and 36).  Grids between one and two a SIMD fold to one (2 tokens 14.0
+    // -> 12.7: every wave then has its SIMD to itself; the logit exchange stays as
+    // it was, 48 waves an XCD being too few for 128 rows).
     const uint32_t waves = row_blocks * d.K * n_tok;
     const uint32_t most = std::max(1u, (n_tok > 1 && waves > 1024 && waves <= 2048 ? 1024u : 2048u) / (d.K * n_tok));
     const uint32_t iters = (row_blocks + most - 1) / most;

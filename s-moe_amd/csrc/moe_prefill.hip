@@ -1135,9 +1135,15 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint4* __restrict__ units, const
 // blocks of a CU pass their barriers independently, so one block's MFMAs
 // overlap the other's conversion.  Needs an even number of groups (a stage's
 // two scales are one dword).
-//   stage    two 64-column groups; gd_depth stages are in flight while one is
-//            computed: their codes in registers, their activation rows in a ring
-//            in LDS, one counted wait and one barrier per stage;
+//   stage    two 64-column groups; gd_depth stages are requested ahead of the one
+//            that is computed: their codes in registers, their activation rows in
+//            a ring in LDS, one counted wait and one barrier per stage.  As
+//            compiled the ring does not stay that full: the loop's exits after
+//            each stage let the registers of the codes meet at its latch, where
+//            the compiler waits for every load in flight, once in gd_depth stages
+//            (not where that is one), and the waits that it adds before the codes'
+//            uses count without the rows' loads, which it does not see, so they
+//            are stricter than the counted ones;
 //   weights  up to two m-tiles a unit (HBM-bound): a load takes 128 bytes of 8
 //            rows, the codes of two stages, marked non-temporal (each weight
 //            line is read once).  Whole lines set the stream's rate: the loads
@@ -1153,8 +1159,8 @@ void k_grouped_mm(MoeDims d, LayerDesc L, const uint4* __restrict__ units, const
 //   acts     [plane][row][16 units of 8 columns], unit x of row r in slot
 //            x ^ (r & 15): conflict-free for the fragment reads (units 4 s + q
 //            of rows 0 .. 15), filled by direct loads (4 rows x 256 bytes each)
-//            issued from inline asm: the compiler does not track them, so it
-//            adds no waits of its own;
+//            issued from inline asm: the compiler does not track them, so it does
+//            not drain them before the reads of another stage's rows;
 //   scales   one load of eight groups of the wave's rows instead of a load per
 //            row and stage, passed across the wave (ds_bpermute).
 //   MFMA     the four products of a group (hi and lo of two steps) accumulate

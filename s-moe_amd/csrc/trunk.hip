@@ -30,9 +30,10 @@
 //                   and weighted V on MFMA.
 //   k_attn_combine  the splits of each head rescaled to their common maximum
 //                   and normalised.  A kernel of its own: the launch boundary
-//                   publishes every partial at once, where an in-kernel
-//                   last-block combine needs an agent-scope release per wave
-//                   (a full L2 write-back each, serialised per XCD).
+//                   publishes every partial at once.  (A combine by the last
+//                   block of a KV head, with partials stored and counted as
+//                   k_route's logits are, would need no L2 write-back either; it
+//                   has not been measured.)
 #include <algorithm>
 
 #include "device_common.hpp"
