@@ -92,7 +92,8 @@ def test_graph_replay_matches_eager(ctx, oracle):
 
 
 @pytest.mark.parametrize("D,E,K,I,Ts", [
-    (2048, 128, 8, 768, (2, 5, 11, 24)),    # one, two, four and ten row blocks a wave
+    (2048, 128, 8, 768, (2, 5, 11, 24)),    # two, two, five and ten row blocks a wave
+    (512, 16, 4, 256, (2, 7)),              # one row block a wave
     (4096, 128, 8, 1536, (5,)),             # two chunks a lane: rows loaded block by block
     (1280, 60, 6, 704, (11, 40)),           # an odd number of row blocks
     (512, 200, 6, 256, (90,)),              # more than 128 experts

@@ -1,9 +1,10 @@
 """The grouped prefill GEMMs and the segmented permute at the edges of their
-passes: pair counts around every 16-row tile and 64-row pass, rows of one to
-several pairs of 64-column groups (with and without a remainder), an odd number of
-groups (the LDS-weight kernel), batches over several permute segments and over
-one pass.  Every result against fp64 (moe_delta_f64_batch) and bit for bit
-against the same tokens in calls of 16."""
+units: work lists of units of up to 32 pairs (short lists: few experts, a narrow
+layer) and of up to 64 (test_units_of_48_and_64_rows), pair counts around every
+16-row tile, rows of one to several pairs of 64-column groups (with and without a
+remainder), an odd number of groups (the LDS-weight kernel), batches over several
+permute segments and over one pass.  Every result against fp64
+(moe_delta_f64_batch) and bit for bit against the same tokens in calls of 16."""
 import numpy as np
 import pytest
 import torch
@@ -36,7 +37,13 @@ def prefill(ctx, layer, h, step):
     (256, 128, 8, 128, (257, 1000, 5000)),   # several segments, several passes
 ])
 def test_passes_and_segments(ctx, D, E, K, I, Ts):
+    check(ctx, D, E, K, I, Ts)
+
+
+def check(ctx, D, E, K, I, Ts):
+    """The ids of every call."""
     layer = Layer(ctx, D, E, K, I, layer_id=500 + D + I)
+    all_ids = []
     hs = hidden_states(ctx, min(max(Ts), 512), D, index0=77)
     hs = hs.repeat((max(Ts) + len(hs) - 1) // len(hs), 1)
     hs[:, 0] += torch.arange(len(hs), device="cuda") * 1e-3      # (repeated rows differ)
@@ -52,3 +59,31 @@ def test_passes_and_segments(ctx, D, E, K, I, Ts):
         got = out.cpu().numpy()[rows]
         err, _ = rel_err(got.astype(np.float64) - x, ref, slack=np.spacing(np.abs(got)))
         assert err <= TOL_F64, f"T={T}: {err:.2e}"
+        all_ids.append(ids.cpu().numpy())
+    return all_ids
+
+
+def unit_rows(ids, E, I):
+    """Rows of the units of the work list that the permute of ids makes: an expert's M pairs in units of up
+    to 64 where that gives as many units as 512 gate/up blocks need, else of up to 32; equal numbers of
+    16-row tiles."""
+    M = np.bincount(ids.ravel(), minlength=E)
+    few = 512 // -(-I // 128)
+    cap = 64 if np.sum(-(-M // 64)) >= few else 32
+    n, tiles = -(-M // cap), -(-M // 16)
+    return {16 * -(-int(t) // int(k)) for t, k in zip(tiles, n) if k}
+
+
+@pytest.mark.parametrize("D,E,K,I,Ts", [
+    (256, 32, 4, 2048, (300, 450, 640)),     # two stages of gate/up, sixteen of down
+    (1152, 36, 4, 1920, (380, 560)),         # odd numbers of stages
+    (128, 64, 4, 1152, (660, 900)),          # one stage of gate/up
+    (320, 32, 4, 2112, (300, 450, 640)),     # odd numbers of groups: the LDS-weight kernel
+])
+def test_units_of_48_and_64_rows(ctx, D, E, K, I, Ts):
+    """Wide layers with enough experts for units of up to 64 pairs: the 48- and the 64-row forms of both
+    kernels give every pair the sums of the 16-row form."""
+    seen = set()
+    for ids in check(ctx, D, E, K, I, Ts):
+        seen |= unit_rows(ids, E, I)
+    assert {48, 64} <= seen, seen

@@ -134,8 +134,8 @@ def check_against_oracle(oracle, layer, h0, got, gids, gw, rows=None, exact=Fals
 
 
 def test_prefill_tiny_shapes(ctx, oracle):
-    # (the E=4 case gives every expert about 100 pairs: two passes of the
-    # grouped GEMM, the second one partial)
+    # (the E=4 case gives every expert about 100 pairs: several units of the
+    # grouped GEMMs' work list, the last one partial)
     for (D, E, K, I, T) in ((128, 16, 4, 128, 70), (256, 64, 8, 192, 33), (512, 200, 6, 256, 9),
                             (256, 4, 2, 128, 200)):
         layer = Layer(ctx, D, E, K, I, layer_id=100 + D)
