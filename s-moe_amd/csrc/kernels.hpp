@@ -213,6 +213,38 @@ struct AttnPlan {
     uint32_t splits;    // context splits
     uint32_t chunk;     // positions per split
 };
+constexpr int AT_MAX_GB = 8;      // k_attn_decode: query heads per block,
+constexpr int AT_MAX_GHD = 1024;  // times head_dim
+constexpr int AW_HEADS = 16;      // k_attn_wide: query heads per block (MFMA columns)
+// query heads per block of k_attn_decode
+constexpr uint32_t attn_group(const AttnDims& a)
+{
+    const uint32_t G = a.num_heads / a.num_kv_heads;
+    uint32_t gb = 1;
+    while (gb < G && gb < static_cast<uint32_t>(AT_MAX_GB) && gb * 2 * a.head_dim <= AT_MAX_GHD) gb *= 2;
+    return gb;
+}
+// The MFMA kernel (k_attn_wide) reads each K and V row once for all query heads of
+// a KV head, k_attn_decode once per block of up to eight.  Long contexts with more
+// than eight: 16 heads of 128 over 32768 positions 80 -> 59 us for the layer, 64
+// heads of 256 over 4 KV heads 195 -> 91.  Over 1000 positions, where the launches'
+// latencies decide, it loses (39.5 against 38.7; ten of 256 over 2048 27.1 against
+// 24.0), at 3000 the two are even, and with eight heads or fewer its columns are
+// half or more empty (8 heads over 32768 positions 39.3 against 41.8, one head 31.5
+// against 30.0).  With up to 64 splits it has 64 blocks for each 16 query heads of a
+// KV head, and half the waves a block at head_dim 256.  One such column of 256:
+// slower at every length (10 heads 20.0 against 23.0 us at 4096 positions, 43.8
+// against 59.8 at 32768).  One or two columns, where k_attn_decode's blocks have no
+// idle heads: from 8192 positions on (16 heads of 128 over one KV head 19.4 / 20.3
+// at 4096, 20.1 / 20.3 at 6000, 21.6 / 20.8 at 8192; 32 of 256 over two 33.5 / 34.6,
+// 37.9 / 38.5, 42.4 / 39.8; with idle heads, 20 of 256 over two, 29.4 / 27.6 at
+// 4096); heads of 64 from 4096 on (17.3 / 16.5).
+constexpr bool attn_wide(const AttnDims& a, uint32_t valid)
+{
+    const uint32_t G = a.num_heads / a.num_kv_heads, columns = a.num_kv_heads * ((G + AW_HEADS - 1) / AW_HEADS);
+    if (G <= static_cast<uint32_t>(AT_MAX_GB) || (a.head_dim > 128 && columns == 1)) return false;
+    return valid >= (a.head_dim > 64 && columns <= 2 && G % attn_group(a) == 0 ? 8192u : 4096u);
+}
 AttnPlan attn_plan(const AttnDims& a, uint32_t valid);
 // scratch of the launch: per-(head, split) partials
 size_t attn_scratch_bytes(const AttnDims& a);

@@ -183,8 +183,6 @@ hipError_t launch_gemv_bf16(const GemvGroup& in, hipStream_t s)
 constexpr int AT_WAVES = 8;
 constexpr int AT_THREADS = AT_WAVES * WAVE;
 constexpr int AT_U = 2;                 // position steps per tile
-constexpr int AT_MAX_GB = 8;            // query heads per block
-constexpr int AT_MAX_GHD = 1024;        // query heads per block x head_dim
 
 struct AttnArgs {
     AttnDims a;
@@ -450,7 +448,6 @@ void k_attn_decode(AttnArgs p)
 // ---------------------------------------------------------------------------
 // k_attn_wide: one block per (KV head, group of up to 16 query heads, context split)
 // ---------------------------------------------------------------------------
-constexpr int AW_HEADS = 16;            // query heads per block (MFMA columns)
 constexpr int AW_TILE = 16;             // positions per wave step (MFMA rows)
 // waves per block: two per SIMD, one where a head's registers leave no room for two
 constexpr int wide_waves(uint32_t head_dim) { return head_dim > 128 ? 4 : 8; }
@@ -768,17 +765,8 @@ AttnPlan attn_plan(const AttnDims& a, uint32_t valid)
 {
     AttnPlan pl{};
     const uint32_t G = a.num_heads / a.num_kv_heads;
-    // The MFMA kernel reads each K and V row once for all query heads of a KV
-    // head, the other one once per block of up to eight.  Long contexts with more than
-    // eight: 16 heads of 128 over 32768 positions 80 -> 59 us for the layer, ten of 256 92
-    // -> 61.  Over 1000 positions, where the launches' latencies decide, it loses (39.5
-    // against 38.7; ten of 256 over 2048 27.1 against 24.0), at 3000 the two are even,
-    // and with eight heads or fewer its columns are half or more empty (8 heads over
-    // 32768 positions 39.3 against 41.8, one head 31.5 against 30.0).
-    pl.wide = G > static_cast<uint32_t>(AT_MAX_GB) && valid >= 4096;
-    uint32_t gb = 1;
-    while (gb < G && gb < static_cast<uint32_t>(AT_MAX_GB) && gb * 2 * a.head_dim <= AT_MAX_GHD) gb *= 2;
-    pl.gb = pl.wide ? AW_HEADS : gb;
+    pl.wide = attn_wide(a, valid);
+    pl.gb = pl.wide ? AW_HEADS : attn_group(a);
     pl.n_sub = (G + pl.gb - 1) / pl.gb;
     const uint32_t bx = a.num_kv_heads * pl.n_sub;
     // at least one tile per wave; about one block per CU (256) in all

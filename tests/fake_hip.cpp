@@ -72,6 +72,10 @@ uint64_t fake_count(const char* what)
     if (w == "permutes_seg") return s.permutes_seg;
     return ~0ull;
 }
+int fake_attn_wide(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t valid)
+{
+    return smoe::attn_wide({head_dim, heads, kv_heads, kv_heads * head_dim, valid, 1.0f}, valid);
+}
 int fake_is_live(uint64_t p) { return st().dev.count(static_cast<uintptr_t>(p)) != 0; }
 
 // ---- the runtime --------------------------------------------------------------

@@ -235,3 +235,26 @@ def test_permute_outputs_take_the_tokens_that_the_header_states(bridge):
     assert bridge.prefill(SHAPE_30B, limit, perm=True) == 0 and bridge.count("T") == limit
     assert bridge.prefill(SHAPE_30B, limit + 1, perm=True) == smoe_amd.SMOE_ERR_SHAPE
     assert bridge.prefill(SHAPE_30B, limit + 1) == 0 and bridge.count("T") == limit + 1
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,wide,plain", [
+    # (positions at which k_attn_wide / k_attn_decode measured faster)
+    (64, 4, 128, (4096, 8192, 32768), (1, 1000, 3000)),
+    (16, 1, 128, (8192, 32768), (4096, 6000)),
+    (24, 1, 128, (8192, 10000), (4096, 6000)),
+    (40, 1, 128, (4096, 10000), (1000,)),
+    (27, 3, 128, (4096, 10000), (1000,)),
+    (32, 2, 64, (4096, 8192), (1000,)),
+    (16, 1, 64, (4096, 8192), (1000,)),
+    (10, 1, 256, (), (2048, 4096, 16384, 32768)),
+    (16, 1, 256, (), (4096, 16384, 32768)),
+    (24, 1, 256, (8192, 32768), (4096,)),
+    (32, 2, 256, (8192, 32768), (4096, 6000)),
+    (20, 2, 256, (4096, 6000, 32768), (2048,)),
+    (64, 4, 256, (4096, 32768), (1000,)),
+    (32, 4, 128, (), (4096, 32768)),
+])
+def test_attention_takes_the_faster_kernel(built, heads, kv_heads, head_dim, wide, plain):
+    f = C.CDLL(built).fake_attn_wide
+    assert all(f(heads, kv_heads, head_dim, n) for n in wide)
+    assert not any(f(heads, kv_heads, head_dim, n) for n in plain)

@@ -98,7 +98,10 @@ def rope(pos, head_dim, theta=1e6):
     (4096, 64, 4, 128, 8192, 3000, 4096, True),  # and the first on MFMA, wrapped
     (1024, 18, 2, 64, 5000, 4999, 5000, False),  # 9 of 16 MFMA columns, uneven splits
     (512, 34, 2, 64, 4200, 7, 4161, True),       # 17 query heads: a second block with one
-    (512, 12, 1, 256, 4300, 100, 4100, True),    # head_dim 256 on MFMA
+    (512, 12, 1, 256, 4300, 100, 4100, True),    # head_dim 256, one KV head: on the VALU at every length
+    (512, 20, 2, 256, 4300, 100, 4100, True),    # head_dim 256 on MFMA
+    (512, 16, 1, 128, 8300, 5000, 8191, True),   # one column of 16 heads: the last VALU context,
+    (512, 16, 1, 128, 8300, 5000, 8192, True),   # and the first on MFMA
 ])
 def test_attention_layer_vs_oracle(ctx, oracle, d_model, nh, nkv, hd, ctx_len, slot, valid, qk):
     run_attention_case(ctx, oracle, d_model, nh, nkv, hd, ctx_len, slot, valid, qk)
