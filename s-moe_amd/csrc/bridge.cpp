@@ -1130,9 +1130,8 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
                                                  s.rt_ctr.p, st);
                    }) ||
             !timed(ctx, SMOE_KERNEL_PERMUTE, "permute", [&] {
-                // one workgroup where its other outputs are wanted, else in segments
-                // (5.2 against 9.4 us at 512 tokens of the 30B shape, 4.4 against 5.3 at 64)
-                if (want_perm)
+                // one workgroup also where its other outputs are wanted
+                if (want_perm || smoe::permute_in_one(P, d.E))
                     return smoe::launch_permute(ids, w, P, d.K, d.E, offs, s.pairs.p, sorted_tokens, nullptr,
                                                 union_ids, union_size, s.units.p, few, ctx->d_err, st);
                 return smoe::launch_permute_seg(ids, P, d.E, s.pairs.p, s.units.p, few, s.seg_cnt.p, ctx->d_err, st);

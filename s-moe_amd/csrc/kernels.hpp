@@ -302,6 +302,17 @@ constexpr uint32_t perm_segments(uint32_t P, uint32_t E)
 }
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs, uint4* units,
                               uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
+// Whether a batch of several segments is permuted in one workgroup all the same (its
+// tables fit, and its threads keep all ids: 8 a thread).  One launch instead of
+// two; kernel times of one workgroup / both segment kernels at 128 experts x top-8:
+// 260 tokens 6.4 / 9.6 us, 512 7.8 / 9.5, 736 9.9 / 10.0; 32 x top-4, 700 tokens
+// 5.7 / 8.8; 8 x top-2, 4000 tokens 7.6 / 8.5; past that 60 x top-6, 1500 tokens
+// 11.5 / 9.9.  One segment is permuted by k_perm_scatter alone (4.1 to 5.0 us
+// against 4.3 to 5.4).
+constexpr bool permute_in_one(uint32_t P, uint32_t E)
+{
+    return perm_segments(P, E) > 1 && P <= 8192 && permute_lds_bytes(P, E) <= PERMUTE_MAX_LDS;
+}
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):
 // h [P x I] = silu(x G^T) * (x U^T); y [P x D] = h Dn^T, over the permute's
 // work list.

@@ -89,12 +89,12 @@ def bridge(built):
     b.close()
 
 
-@pytest.mark.parametrize("T,dispatches", [(256, 1), (257, 2), (4096, 2)])
+@pytest.mark.parametrize("T,dispatches", [(256, 1), (1025, 2), (4096, 2)])
 def test_profile_times_every_dispatch_of_a_launcher(bridge, T, dispatches):
     """The permute of several segments takes two dispatches: both are timed, as one launch."""
     L = bridge.lib
     assert L.smoe_hip_profile_enable(bridge.ctx, 1) == 0
-    calls = 5000 if T == 257 else 3      # (past the ring of event slots)
+    calls = 5000 if T == 1025 else 3     # (past the ring of event slots)
     for _ in range(calls):
         assert bridge.prefill(SHAPE_30B, T) == 0
     n, ms = C.c_uint64(), C.c_double()
@@ -258,3 +258,19 @@ def test_attention_takes_the_faster_kernel(built, heads, kv_heads, head_dim, wid
     f = C.CDLL(built).fake_attn_wide
     assert all(f(heads, kv_heads, head_dim, n) for n in wide)
     assert not any(f(heads, kv_heads, head_dim, n) for n in plain)
+
+
+@pytest.mark.parametrize("E,K,in_one,in_segments", [
+    (128, 8, (257, 300, 512, 736), (64, 256, 737, 4096)),
+    (32, 4, (700, 2000), (512, 2049)),
+    (8, 2, (2000, 4000), (1000,)),
+    (512, 8, (150,), (128, 300)),
+])
+def test_permute_takes_one_workgroup_where_it_is_faster(bridge, E, K, in_one, in_segments):
+    """Batches of several segments that one workgroup holds are permuted by it."""
+    shape = dict(d_model=256, n_experts=E, top_k=K, d_ff=128)
+    for T in in_one + in_segments:
+        one, seg = bridge.count("permutes"), bridge.count("permutes_seg")
+        assert bridge.prefill(shape, T) == 0
+        got = bridge.count("permutes") - one, bridge.count("permutes_seg") - seg
+        assert got == ((1, 0) if T in in_one else (0, 1)), T
