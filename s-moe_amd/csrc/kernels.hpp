@@ -276,10 +276,11 @@ constexpr uint32_t max_units(uint32_t P, uint32_t E, uint32_t few_units)
 {
     return P / (P / 64 >= few_units ? 64 : 32) + (E < P ? E : P);
 }
-// records of the work list: eight XCDs' shares
+// records of the work list: eight XCDs' shares, each of an eighth of the long
+// units and an eighth of the short ones, both rounded up
 constexpr uint32_t unit_slots(uint32_t P, uint32_t E, uint32_t few_units)
 {
-    return (max_units(P, E, few_units) + 7u) / 8u * 8u;
+    return (max_units(P, E, few_units) + 14u) / 8u * 8u;
 }
 // The list length below which units are of up to 32 pairs: 512 gate/up blocks,
 // one round of two per CU.  64 Zipf-routed tokens of the 30B shape (45 experts):
