@@ -62,7 +62,7 @@ struct PrefillScratch {
     Buf<uint32_t> ids;               // [P]
     Buf<float> w;                    // [P]
     Buf<uint32_t> offsets;           // [E + 1]
-    Buf<uint4> units;                // [unit_slots] grouped GEMM work list
+    Buf<uint4> units;                // [unit_records] grouped GEMM work lists
     Buf<uint32_t> seg_cnt;           // [perm_segments x E] pairs per segment
     Buf<uint32_t> pairs;             // [P] sorted pair ids
     Buf<float> h;                    // [P x I]
@@ -80,7 +80,7 @@ bool each_prefill_buf(PrefillScratch& c, const SmoeMoeShape* s, uint32_t T, F&& 
     const size_t E = s->n_experts, x = size_t(T) * s->d_model, P = size_t(T) * s->top_k, h = P * s->d_ff;
     const uint32_t P32 = static_cast<uint32_t>(P), E32 = s->n_experts;
     return f(c.x_hi, x) && f(c.x_lo, x) && f(c.x_sc, size_t(T)) && f(c.logits, T * E) && f(c.rt_ctr, size_t(T)) &&
-           f(c.ids, P) && f(c.w, P) && f(c.offsets, E + 1) && f(c.units, size_t(smoe::unit_slots(P32, E32, ~0u))) &&
+           f(c.ids, P) && f(c.w, P) && f(c.offsets, E + 1) && f(c.units, smoe::unit_records(P32, E32)) &&
            f(c.seg_cnt, smoe::perm_segments(P32, E32) * E) && f(c.pairs, P) && f(c.h, h) && f(c.h_hi, h) &&
            f(c.h_lo, h) && f(c.h_sc, P) && f(c.y, P * s->d_model);
 }
@@ -1113,7 +1113,6 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
         rc = ensure_prefill_scratch(ctx, shape, tb, false);
     }
     if (rc != SMOE_OK) return rc;
-    const uint32_t few = smoe::few_units(d);
     PrefillScratch& s = ctx->ps;
     hipStream_t st = ctx->stream;
     if (stream_capturing(st))
@@ -1124,6 +1123,7 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
         uint32_t* ids = ids_out ? ids_out + size_t(t0) * d.K : s.ids.p;
         float* w = weights_out ? weights_out + size_t(t0) * d.K : s.w.p;
         uint32_t* offs = expert_offsets ? expert_offsets : s.offsets.p;
+        const smoe::UnitLists lists = smoe::unit_lists(d, P, s.units.p);
         if (!timed(ctx, SMOE_KERNEL_ROUTE, "route",
                    [&] {
                        return smoe::launch_route(d, L, hv, T, s.x_hi.p, s.x_lo.p, s.x_sc.p, ids, w, s.logits.p,
@@ -1133,18 +1133,17 @@ extern "C" int smoe_hip_moe_prefill(SmoeMetalCtx* ctx, const SmoeMoeShape* shape
                 // one workgroup also where its other outputs are wanted
                 if (want_perm || smoe::permute_in_one(P, d.E))
                     return smoe::launch_permute(ids, w, P, d.K, d.E, offs, s.pairs.p, sorted_tokens, nullptr,
-                                                union_ids, union_size, s.units.p, few, ctx->d_err, st);
-                return smoe::launch_permute_seg(ids, P, d.E, s.pairs.p, s.units.p, few, s.seg_cnt.p, ctx->d_err, st);
+                                                union_ids, union_size, lists, ctx->d_err, st);
+                return smoe::launch_permute_seg(ids, P, d.E, s.pairs.p, lists, s.seg_cnt.p, ctx->d_err, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_GATE_UP, "grouped_gate_up", [&] {
-                return smoe::launch_grouped_gate_up(d, L, P, few, s.units.p, s.pairs.p, s.x_hi.p, s.x_lo.p, s.x_sc.p,
-                                                    s.h.p, st);
+                return smoe::launch_grouped_gate_up(d, L, P, lists, s.pairs.p, s.x_hi.p, s.x_lo.p, s.x_sc.p, s.h.p,
+                                                    st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SPLIT, "split(h)",
                    [&] { return smoe::launch_split_rows(s.h.p, P, d.I, s.h_hi.p, s.h_lo.p, s.h_sc.p, st); }) ||
             !timed(ctx, SMOE_KERNEL_GROUPED_DOWN, "grouped_down", [&] {
-                return smoe::launch_grouped_down(d, L, P, few, s.units.p, s.pairs.p, s.h_hi.p, s.h_lo.p, s.h_sc.p,
-                                                 s.y.p, st);
+                return smoe::launch_grouped_down(d, L, P, lists, s.pairs.p, s.h_hi.p, s.h_lo.p, s.h_sc.p, s.y.p, st);
             }) ||
             !timed(ctx, SMOE_KERNEL_SCATTER, "combine",
                    [&] { return smoe::launch_combine_pairs(s.y.p, w, T, d.K, d.D, hv, st); }))
@@ -1205,7 +1204,7 @@ extern "C" int smoe_hip_permute(SmoeMetalCtx* ctx, const uint32_t* ids, const fl
                  [&] {
                      return smoe::launch_permute(ids, weights, static_cast<uint32_t>(P), top_k, n_experts,
                                                  expert_offsets, ctx->perm_pairs, sorted_tokens, sorted_weights,
-                                                 union_ids, union_size, nullptr, 0u, ctx->d_err, ctx->stream);
+                                                 union_ids, union_size, smoe::UnitLists{}, ctx->d_err, ctx->stream);
                  })
                ? SMOE_OK
                : SMOE_ERR_HIP;

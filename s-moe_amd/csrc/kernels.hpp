@@ -266,43 +266,75 @@ hipError_t launch_route(const MoeDims& d, const LayerDesc& L, const float* hidde
 // the row) and scale[row] = 2^e.
 hipError_t launch_split_rows(const float* src, uint32_t rows, uint32_t cols, uint16_t* hi, uint16_t* lo,
                              float* scale, hipStream_t s);
+// The grouped GEMMs' work lists, one for gate/up and one for down: units of up to
+// cap (64 or 32) pairs of one expert, u64 or u32 of them, a block for each unit and
+// each of the launch's row tiles.  Units of 32 run a long expert's passes side by
+// side but stream and convert its weights once more each, so they are worth it
+// where they cost no more than the CUs that would otherwise be idle: where the
+// longest XCD's share still gives its 32 CUs at most one block each; and where
+// units of 64 are over that too, up to two blocks a CU if there are few more of
+// 32 (a few long experts) or those of 64 are mostly full.  Kernel times in us with
+// units of 64 / of 32:
+//   one block a CU at most   16 experts, 23 units of 32, 10 tiles  44.5 / 41.2
+//                            8 experts, 23, 6                      36.7 / 26.8
+//                            64, 31, 5 (skewed)                    22.9 / 17.4
+//   more                     16, 32, 10                            55.7 / 63.5
+//                            32, 33, 8                             15.8 / 22.0
+//                            64, 132, 7                            62.4 / 83.4
+//   62 for 57 units, 6 tiles (64 Zipf-routed tokens of 128 experts)  43.3 / 39.2
+//   77 for 45 units of 44 pairs, 6 tiles                           59.1 / 46.0
+__host__ __device__ constexpr uint32_t unit_cap(uint32_t P, uint32_t u64, uint32_t u32, uint32_t tiles)
+{
+    const uint32_t b64 = (u64 + 7u) / 8u * tiles, b32 = (u32 + 7u) / 8u * tiles;   // blocks of an XCD
+    if (b32 <= 32u) return 32u;
+    return b64 > 32u && b32 <= 64u && (8u * u32 <= 9u * u64 || P >= 40u * u64) ? 32u : 64u;
+}
+constexpr uint32_t max_units(uint32_t P, uint32_t E, uint32_t tiles)
+{
+    const uint32_t experts = E < P ? E : P, u64 = P / 64 + experts, u32 = P / 32 + experts;
+    const uint32_t two = 64 / tiles * 8, m32 = u32 < two ? u32 : two;   // (units of 32: two blocks a CU at most)
+    return u64 > m32 ? u64 : m32;
+}
+// records of a work list: eight XCDs' shares, each of an eighth of the long units
+// and an eighth of the short ones, both rounded up
+constexpr uint32_t unit_slots(uint32_t units) { return (units + 14u) / 8u * 8u; }
+struct UnitLists {
+    uint4* units = nullptr;       // [slots[0] + slots[1]], null: none
+    uint32_t tiles[2] = {1, 1};   // row tiles of gate/up and of down
+    uint32_t slots[2] = {0, 0};
+};
+inline UnitLists unit_lists(const MoeDims& d, uint32_t P, uint4* units)
+{
+    UnitLists l;
+    l.units = units;
+    l.tiles[0] = (d.I + 127u) / 128u;
+    l.tiles[1] = (d.D + 255u) / 256u;
+    for (int i = 0; i < 2; ++i) l.slots[i] = unit_slots(max_units(P, d.E, l.tiles[i]));
+    return l;
+}
+// what unit_lists takes at most
+constexpr size_t unit_records(uint32_t P, uint32_t E) { return 2 * size_t(unit_slots(P / 32 + (E < P ? E : P))); }
 // Stable counting sort of the P pairs by expert: offsets [E+1],
 // sorted_pairs [P] (pair = token * K + rank); sorted_tokens, sorted_w,
-// union_ids [E], union_size [1] optional (nullptr).  units [unit_slots(P,
-// E, few_units)] optional: the grouped GEMMs' work list of (expert, pass) units, of up to
-// 64 pairs, or up to 32 where fewer than few_units would result.  Bad ids set err bit 1.
+// union_ids [E], union_size [1] optional (nullptr), and the work lists.  Bad ids
+// set err bit 1.
 constexpr size_t PERMUTE_MAX_LDS = 48 * 1024;
-constexpr uint32_t max_units(uint32_t P, uint32_t E, uint32_t few_units)
-{
-    return P / (P / 64 >= few_units ? 64 : 32) + (E < P ? E : P);
-}
-// records of the work list: eight XCDs' shares, each of an eighth of the long
-// units and an eighth of the short ones, both rounded up
-constexpr uint32_t unit_slots(uint32_t P, uint32_t E, uint32_t few_units)
-{
-    return (max_units(P, E, few_units) + 14u) / 8u * 8u;
-}
-// The list length below which units are of up to 32 pairs: 512 gate/up blocks,
-// one round of two per CU.  64 Zipf-routed tokens of the 30B shape (45 experts):
-// 103 us with units of 64, 89 with 32; 512 even ones (128 experts of 32): 186
-// with 64, 215 with 32, so the shorter units stay below one round.
-constexpr uint32_t few_units(const MoeDims& d) { return 512u / ((d.I + 127u) / 128u); }
 constexpr size_t permute_lds_bytes(uint32_t P, uint32_t E)
 {
     return (size_t((P + 63) / 64) * E + 3 * size_t(E) + 1) * sizeof(uint32_t);
 }
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
-                          uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s);
-// The same sorted pairs and units in segments, one workgroup each, for any P
+                          uint32_t* union_size, const UnitLists& lists, uint32_t* err, hipStream_t s);
+// The same sorted pairs and work lists in segments, one workgroup each, for any P
 // (seg_cnt [perm_segments(P, E) x E]).
 __host__ __device__ constexpr uint32_t perm_seg_chunks(uint32_t E) { return E <= 256 ? 32u : 16u; }
 constexpr uint32_t perm_segments(uint32_t P, uint32_t E)
 {
     return (P + 64u * perm_seg_chunks(E) - 1) / (64u * perm_seg_chunks(E));
 }
-hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs, uint4* units,
-                              uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
+hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs,
+                              const UnitLists& lists, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
 // Whether a batch of several segments is permuted in one workgroup all the same (its
 // tables fit, and its threads keep all ids: 8 a thread).  One launch instead of
 // two; kernel times of one workgroup / both segment kernels at 128 experts x top-8:
@@ -316,11 +348,11 @@ constexpr bool permute_in_one(uint32_t P, uint32_t E)
 }
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):
 // h [P x I] = silu(x G^T) * (x U^T); y [P x D] = h Dn^T, over the permute's
-// work list.
-hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+// work lists.
+hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, const UnitLists& lists,
                                   const uint32_t* sorted_pairs, const uint16_t* x_hi,
                                   const uint16_t* x_lo, const float* x_scale, float* h, hipStream_t s);
-hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, const UnitLists& lists,
                                const uint32_t* sorted_pairs, const uint16_t* h_hi,
                                const uint16_t* h_lo, const float* h_scale, float* y, hipStream_t s);
 // hidden[t] += sum_r w[t][r] * y[t*K + r] (rank order).

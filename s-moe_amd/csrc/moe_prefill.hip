@@ -16,7 +16,7 @@
 //                  columns of every 8 in the order 0 2 4 6 1 3 5 7.
 //   k_perm_count, k_perm_scatter  stable counting sort of the T*k (token,
 //                  rank) pairs by expert, one workgroup per segment of pairs,
-//                  and the GEMMs' work list (k_permute: one workgroup, with the
+//                  and the GEMMs' work lists (k_permute: one workgroup, with the
 //                  union order by first appearance, for callers that ask for
 //                  the permute's outputs).
 //   k_grouped_reg  per unit of up to 64 pairs of an expert: [pairs x K] x [K x
@@ -473,11 +473,11 @@ void k_split_rows(const float* __restrict__ src, uint32_t rows, uint32_t cols, u
 // table put them all in one: 14.2 -> 11.6 us at 512 tokens of the 30B shape).
 // Union order (first appearance, token-major, prefill.cpp:55-68) ranks the
 // touched experts by their first pair.  ids >= E are skipped and flagged in
-// err (bit 1).  units (optional) receives the grouped GEMMs' work list.
+// err (bit 1).  lists (optional) receives the grouped GEMMs' work lists.
 // ---------------------------------------------------------------------------
 constexpr int PERM_THREADS = 1024;
 
-// The grouped GEMMs' work list: units of up to cap (64 or 32) pairs of one
+// The grouped GEMMs' work lists: units of up to cap (unit_cap) pairs of one
 // expert, an expert's M pairs in as few units as cap allows, of equal numbers of
 // 16-row tiles.  First the units of more than 16 rows, then those of 16, experts
 // ascending in either: what is left for the end of a launch is short (in the
@@ -503,12 +503,10 @@ __device__ __forceinline__ uint32_t unit_pair(uint32_t M, uint32_t cap)
     return unit_count(M, cap) << (M > 16u ? 0u : 16u);
 }
 
-// One wave: exclusive scans of the E experts' totals s_tot into s_off [E + 1]
-// (pairs) and s_unit [E + 1] (units), eight experts a lane, and the cap.  Units
-// of 32 rows where 64 would leave the list shorter than few_units: the GEMMs'
-// blocks (units x row tiles) would not fill the chip, and a long expert's
-// passes then run side by side.
-__device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, uint32_t few_units, uint32_t* s_off,
+// One wave, eight experts a lane: exclusive scans of the E experts' totals s_tot
+// into s_off [E + 1] (pairs) and s_unit [2][E + 1] (units of up to 64, of up to 32
+// pairs), and the caps of the two work lists.
+__device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, const UnitLists& lists, uint32_t* s_off,
                                            uint32_t* s_unit, uint32_t* s_cap)
 {
     const uint32_t lane = threadIdx.x & 63;
@@ -530,39 +528,46 @@ __device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, ui
     };
     const uint32_t i_tot = inclusive(sum), i64 = inclusive(u64), i32 = inclusive(u32);
     const uint32_t n64 = readlane_u32(i64, WAVE - 1), n32 = readlane_u32(i32, WAVE - 1);
-    const uint32_t cap = (n64 & 0xFFFFu) + (n64 >> 16) < few_units ? 32u : 64u;
-    uint32_t run = i_tot - sum, urun = (cap == 32u ? i32 - u32 : i64 - u64) + ((cap == 32u ? n32 : n64) << 16);
+    // (the short units' counts start after all the long ones)
+    uint32_t run = i_tot - sum, run64 = i64 - u64 + (n64 << 16), run32 = i32 - u32 + (n32 << 16);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const uint32_t e = 8 * lane + i;
         if (e <= E) {
             s_off[e] = run;
-            s_unit[e] = urun;
+            s_unit[e] = run64;
+            s_unit[E + 1 + e] = run32;
         }
         run += tot[i];
-        urun += unit_pair(tot[i], cap);
+        run64 += unit_pair(tot[i], 64u);
+        run32 += unit_pair(tot[i], 32u);
     }
     if (lane == WAVE - 1) {   // (E = 512 is past the last lane's eight)
         s_off[E] = run;
-        s_unit[E] = urun;
-        *s_cap = cap;
+        s_unit[E] = run64;
+        s_unit[2 * E + 1] = run32;
+        for (int i = 0; i < 2; ++i)
+            s_cap[i] = unit_cap(run, (n64 & 0xFFFFu) + (n64 >> 16), (n32 & 0xFFFFu) + (n32 >> 16), lists.tiles[i]);
     }
 }
 
-// a workgroup writes the n_slots records (s_off, s_unit, cap: scan_units):
+// a workgroup writes the records of both lists (s_off, s_unit, s_cap: scan_units):
 // x = expert | rows of a pass << 16, y = first pair, z = pairs
-__device__ __forceinline__ void write_units(const uint32_t* s_off, const uint32_t* s_unit, uint32_t E, uint32_t cap,
-                                            uint4* units, uint32_t n_slots)
+__device__ __forceinline__ void write_units(const uint32_t* s_off, const uint32_t* s_unit, uint32_t E,
+                                            const uint32_t* s_cap, const UnitLists& lists)
 {
-    const uint32_t n_long = s_unit[E] & 0xFFFFu, n_short = (s_unit[E] >> 16) - n_long;
-    for (uint32_t i = threadIdx.x; i < n_slots; i += blockDim.x) {
+    for (uint32_t k = threadIdx.x; k < lists.slots[0] + lists.slots[1]; k += blockDim.x) {
+        const bool down = k >= lists.slots[0];
+        const uint32_t i = down ? k - lists.slots[0] : k, cap = s_cap[down ? 1 : 0];
+        const uint32_t* tab = s_unit + (cap == 32u ? E + 1u : 0u);
+        const uint32_t n_long = tab[E] & 0xFFFFu, n_short = (tab[E] >> 16) - n_long;
         const uint32_t j = i >> 3, x = i & 7u, xs = 7u - x;
         const uint32_t l0 = x * n_long / 8u, nl = (x + 1u) * n_long / 8u - l0;
         const uint32_t s0 = xs * n_short / 8u, ns = (xs + 1u) * n_short / 8u - s0;
         uint4 rec = make_uint4(0u, 0u, 0u, 0u);
         if (j < nl + ns) {
             const uint32_t sh = j < nl ? 0u : 16u, u = j < nl ? l0 + j : n_long + s0 + (j - nl);
-            auto first = [&](uint32_t e) { return (s_unit[e] >> sh) & 0xFFFFu; };
+            auto first = [&](uint32_t e) { return (tab[e] >> sh) & 0xFFFFu; };
             uint32_t e = 0, hi = E;              // the expert: first(e) <= u < first(e + 1)
             while (hi - e > 1) {
                 const uint32_t mid = (e + hi) >> 1;
@@ -572,7 +577,7 @@ __device__ __forceinline__ void write_units(const uint32_t* s_off, const uint32_
             const uint32_t M = s_off[e + 1] - s_off[e], rows = unit_rows(M, cap), m0 = (u - first(e)) * rows;
             rec = make_uint4(e | (rows << 16), s_off[e] + m0, min(M - m0, rows), 0u);
         }
-        units[i] = rec;
+        lists.units[k] = rec;
     }
 }
 
@@ -580,11 +585,10 @@ __global__ __launch_bounds__(PERM_THREADS)
 void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, uint32_t P, uint32_t K, uint32_t E,
                uint32_t* __restrict__ offsets, uint32_t* __restrict__ sorted_pairs,
                uint32_t* __restrict__ sorted_tokens, float* __restrict__ sorted_w, uint32_t* __restrict__ union_ids,
-               uint32_t* __restrict__ union_size, uint4* __restrict__ units, uint32_t n_slots, uint32_t few_units,
-               uint32_t* __restrict__ err)
+               uint32_t* __restrict__ union_size, UnitLists lists, uint32_t* __restrict__ err)
 {
     extern __shared__ uint32_t s_mem[];
-    __shared__ uint32_t s_cap;
+    __shared__ uint32_t s_cap[2];
     // the count table is [E][C | 1]: the odd row stride puts a chunk's experts,
     // and the chunks one expert's threads read, in different banks
     const uint32_t C = (P + 63) / 64, CS = C | 1u;
@@ -592,7 +596,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
     uint32_t* s_first = s_cnt + CS * E;    // [E]
     uint32_t* s_tot = s_first + E;         // [E]
     uint32_t* s_off = s_tot + E;           // [E + 1]
-    uint32_t* s_unit = s_off + E + 1;      // [E + 1]
+    uint32_t* s_unit = s_off + E + 1;      // [2][E + 1]
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     constexpr int NW = PERM_THREADS / WAVE;
 
@@ -658,7 +662,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
     }
     __syncthreads();
     // expert offsets and units
-    if (wv == 0) scan_units(s_tot, E, few_units, s_off, s_unit, &s_cap);
+    if (wv == 0) scan_units(s_tot, E, lists, s_off, s_unit, s_cap);
     __syncthreads();
     for (uint32_t e = threadIdx.x; e <= E; e += PERM_THREADS) offsets[e] = s_off[e];
     // scatter: rank among equal ids of lower lanes of the same chunk; the
@@ -704,7 +708,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
         for (uint32_t e = 0; e < E; ++e) n += s_tot[e] != 0;
         *union_size = n;
     }
-    if (units) write_units(s_off, s_unit, E, s_cap, units, n_slots);
+    if (lists.units) write_units(s_off, s_unit, E, s_cap, lists);
 }
 
 // ---------------------------------------------------------------------------
@@ -716,7 +720,7 @@ void k_permute(const uint32_t* __restrict__ ids, const float* __restrict__ w, ui
 //                   its own and of all of them, scans the totals into the
 //                   expert offsets, and places its segment's pairs as
 //                   k_permute does.  Workgroup 0 also writes the grouped
-//                   GEMMs' work list.
+//                   GEMMs' work lists.
 // A batch of one segment needs no counts from elsewhere: k_perm_scatter counts
 // it itself (ONE) and is the only launch (64 tokens of the 30B shape 115.9 ->
 // 113.5 us a call).
@@ -742,17 +746,16 @@ void k_perm_count(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, uint
 template <bool ONE>
 __global__ __launch_bounds__(PERM_THREADS)
 void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, const uint32_t* __restrict__ seg_cnt,
-                    uint32_t* __restrict__ sorted_pairs, uint4* __restrict__ units, uint32_t n_slots,
-                    uint32_t few_units, uint32_t* __restrict__ err)
+                    uint32_t* __restrict__ sorted_pairs, UnitLists lists, uint32_t* __restrict__ err)
 {
     extern __shared__ uint32_t s_mem[];
-    __shared__ uint32_t s_cap;
+    __shared__ uint32_t s_cap[2];
     const uint32_t CH = perm_seg_chunks(E), CS = CH | 1u;
     uint32_t* s_cnt = s_mem;               // [E x CS]
     uint32_t* s_base = s_cnt + E * CS;     // [E] pairs of the expert in earlier segments
     uint32_t* s_tot = s_base + E;          // [E]
     uint32_t* s_off = s_tot + E;           // [E + 1]
-    uint32_t* s_unit = s_off + E + 1;      // [E + 1]
+    uint32_t* s_unit = s_off + E + 1;      // [2][E + 1]
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     constexpr uint32_t NW = PERM_THREADS / WAVE;
     const uint32_t seg = blockIdx.x, nseg = gridDim.x;
@@ -788,7 +791,7 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
         }
     }
     if constexpr (ONE) __syncthreads();
-    if (wv == 0) scan_units(s_tot, E, few_units, s_off, s_unit, &s_cap);
+    if (wv == 0) scan_units(s_tot, E, lists, s_off, s_unit, s_cap);
     __syncthreads();
     // counts -> exclusive prefix over the segment's chunks; S threads (a power
     // of two, in one wave) share an expert's chunks
@@ -830,7 +833,7 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
         const uint32_t rank = __popcll(same & ((1ull << lane) - 1ull));
         if (ok) sorted_pairs[s_cnt[e * CS + c] + rank] = (seg * CH + c) * 64 + lane;
     }
-    if (seg == 0) write_units(s_off, s_unit, E, s_cap, units, n_slots);
+    if (seg == 0) write_units(s_off, s_unit, E, s_cap, lists);
 }
 
 // ---------------------------------------------------------------------------
@@ -1617,39 +1620,38 @@ hipError_t launch_split_rows(const float* src, uint32_t rows, uint32_t cols, uin
 }
 
 // what k_permute allocates: the count table's odd row stride and the unit
-// offsets add at most 2 E + 1 words to permute_lds_bytes (which bounds the batch)
+// offsets add at most 3 E + 2 words to permute_lds_bytes (which bounds the batch)
 static size_t permute_lds_alloc(uint32_t P, uint32_t E)
 {
     const size_t CS = ((P + 63) / 64) | 1u;
-    return (CS * E + 4 * size_t(E) + 2) * sizeof(uint32_t);
+    return (CS * E + 5 * size_t(E) + 3) * sizeof(uint32_t);
 }
 
 hipError_t launch_permute(const uint32_t* ids, const float* w, uint32_t P, uint32_t K, uint32_t E, uint32_t* offsets,
                           uint32_t* sorted_pairs, uint32_t* sorted_tokens, float* sorted_w, uint32_t* union_ids,
-                          uint32_t* union_size, uint4* units, uint32_t few_units, uint32_t* err, hipStream_t s)
+                          uint32_t* union_size, const UnitLists& lists, uint32_t* err, hipStream_t s)
 {
     if (P == 0 || E == 0 || permute_lds_bytes(P, E) > PERMUTE_MAX_LDS) return hipErrorInvalidValue;
     const size_t lds = permute_lds_alloc(P, E);
     launch_kernel_lds(k_permute, dim3(1), dim3(PERM_THREADS), static_cast<uint32_t>(lds), s, ids, w, P, K, E,
-                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, units, unit_slots(P, E, few_units), few_units, err);
+                      offsets, sorted_pairs, sorted_tokens, sorted_w, union_ids, union_size, lists, err);
     return hipGetLastError();
 }
 
-hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs, uint4* units,
-                              uint32_t few_units, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
+hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs,
+                              const UnitLists& lists, uint32_t* seg_cnt, uint32_t* err, hipStream_t s)
 {
-    if (P == 0 || E == 0 || E > SMOE_TOPK_MAX_N) return hipErrorInvalidValue;
+    if (P == 0 || E == 0 || E > SMOE_TOPK_MAX_N || !lists.units) return hipErrorInvalidValue;
     const uint32_t nseg = perm_segments(P, E);
-    const uint32_t slots = unit_slots(P, E, few_units);
-    const uint32_t lds = (E * (perm_seg_chunks(E) | 1u) + 4 * E + 2) * static_cast<uint32_t>(sizeof(uint32_t));
+    const uint32_t lds = (E * (perm_seg_chunks(E) | 1u) + 5 * E + 3) * static_cast<uint32_t>(sizeof(uint32_t));
     if (nseg == 1) {
         launch_kernel_lds(k_perm_scatter<true>, dim3(1), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt,
-                          sorted_pairs, units, slots, few_units, err);
+                          sorted_pairs, lists, err);
         return hipGetLastError();
     }
     launch_kernel(k_perm_count, dim3(nseg), dim3(PERM_THREADS), s, ids, P, E, seg_cnt, err);
     launch_kernel_lds(k_perm_scatter<false>, dim3(nseg), dim3(PERM_THREADS), lds, s, ids, P, E, seg_cnt,
-                      sorted_pairs, units, slots, few_units, err);
+                      sorted_pairs, lists, err);
     return hipGetLastError();
 }
 
@@ -1663,37 +1665,37 @@ static bool reg_supported(const LayerDesc& L, uint32_t k_dim)
 }
 
 template <bool GATE_UP>
-static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t P, const UnitLists& lists,
                                  const uint32_t* sorted_pairs, const uint16_t* a_hi,
                                  const uint16_t* a_lo, const float* a_scale, float* out, hipStream_t s)
 {
-    if (d.group != 64 || d.I % 64 || d.D % 64 || P == 0 || !units) return hipErrorInvalidValue;
+    static_assert(GM_ROWS_GU == 128 && GM_ROWS_DN == 256 && GD_ROWS == 256, "the tiles of unit_lists");
+    if (d.group != 64 || d.I % 64 || d.D % 64 || P == 0 || !lists.units) return hipErrorInvalidValue;
     const uint32_t n_dim = GATE_UP ? d.I : d.D, k_dim = GATE_UP ? d.D : d.I, div = GATE_UP ? d.K : 1u;
-    const uint32_t slots = unit_slots(P, d.E, few_units);
-    if (reg_supported(L, k_dim)) {
-        const uint32_t rows = GATE_UP ? GD_ROWS / 2 : GD_ROWS, nt = (n_dim + rows - 1) / rows;
-        launch_kernel(k_grouped_reg<GATE_UP>, dim3(slots * nt), dim3(GD_WAVES * WAVE), s, d, L, units,
-                      sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
-    } else {
-        const uint32_t rows = GATE_UP ? GM_ROWS_GU : GM_ROWS_DN, nt = (n_dim + rows - 1) / rows;
-        launch_kernel(k_grouped_mm<GATE_UP>, dim3(slots * nt), dim3(GM_WAVES * WAVE), s, d, L, units,
-                      sorted_pairs, a_hi, a_lo, a_scale, div, out, n_dim, k_dim, nt);
-    }
+    const uint4* units = lists.units + (GATE_UP ? 0u : lists.slots[0]);
+    const uint32_t nt = lists.tiles[GATE_UP ? 0 : 1];
+    const dim3 grid(lists.slots[GATE_UP ? 0 : 1] * nt);
+    if (reg_supported(L, k_dim))
+        launch_kernel(k_grouped_reg<GATE_UP>, grid, dim3(GD_WAVES * WAVE), s, d, L, units, sorted_pairs, a_hi, a_lo,
+                      a_scale, div, out, n_dim, k_dim, nt);
+    else
+        launch_kernel(k_grouped_mm<GATE_UP>, grid, dim3(GM_WAVES * WAVE), s, d, L, units, sorted_pairs, a_hi, a_lo,
+                      a_scale, div, out, n_dim, k_dim, nt);
     return hipGetLastError();
 }
 
-hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+hipError_t launch_grouped_gate_up(const MoeDims& d, const LayerDesc& L, uint32_t P, const UnitLists& lists,
                                   const uint32_t* sorted_pairs, const uint16_t* x_hi,
                                   const uint16_t* x_lo, const float* x_scale, float* h, hipStream_t s)
 {
-    return launch_grouped<true>(d, L, P, few_units, units, sorted_pairs, x_hi, x_lo, x_scale, h, s);
+    return launch_grouped<true>(d, L, P, lists, sorted_pairs, x_hi, x_lo, x_scale, h, s);
 }
 
-hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, uint32_t few_units, const uint4* units,
+hipError_t launch_grouped_down(const MoeDims& d, const LayerDesc& L, uint32_t P, const UnitLists& lists,
                                const uint32_t* sorted_pairs, const uint16_t* h_hi,
                                const uint16_t* h_lo, const float* h_scale, float* y, hipStream_t s)
 {
-    return launch_grouped<false>(d, L, P, few_units, units, sorted_pairs, h_hi, h_lo, h_scale, y, s);
+    return launch_grouped<false>(d, L, P, lists, sorted_pairs, h_hi, h_lo, h_scale, y, s);
 }
 
 hipError_t launch_combine_pairs(const float* y, const float* w, uint32_t T, uint32_t K, uint32_t D, float* hidden,

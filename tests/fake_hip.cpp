@@ -72,6 +72,12 @@ uint64_t fake_count(const char* what)
     if (w == "permutes_seg") return s.permutes_seg;
     return ~0ull;
 }
+uint32_t fake_unit_cap(uint32_t P, uint32_t u64, uint32_t u32, uint32_t tiles)
+{
+    return smoe::unit_cap(P, u64, u32, tiles);
+}
+uint32_t fake_unit_slots(uint32_t P, uint32_t E, uint32_t tiles) { return smoe::unit_slots(smoe::max_units(P, E, tiles)); }
+uint64_t fake_unit_records(uint32_t P, uint32_t E) { return smoe::unit_records(P, E); }
 int fake_attn_wide(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t valid)
 {
     return smoe::attn_wide({head_dim, heads, kv_heads, kv_heads * head_dim, valid, 1.0f}, valid);
@@ -253,23 +259,23 @@ hipError_t launch_split_rows(const float*, uint32_t, uint32_t, uint16_t*, uint16
     return dispatch("split");
 }
 hipError_t launch_permute(const uint32_t*, const float*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, uint32_t*,
-                          float*, uint32_t*, uint32_t*, uint4*, uint32_t, uint32_t*, hipStream_t)
+                          float*, uint32_t*, uint32_t*, const UnitLists&, uint32_t*, hipStream_t)
 {
     ++st().permutes;
     return dispatch("permute");
 }
-hipError_t launch_permute_seg(const uint32_t*, uint32_t P, uint32_t E, uint32_t*, uint4*, uint32_t, uint32_t*, uint32_t*,
+hipError_t launch_permute_seg(const uint32_t*, uint32_t P, uint32_t E, uint32_t*, const UnitLists&, uint32_t*, uint32_t*,
                               hipStream_t)
 {
     ++st().permutes_seg;
     return dispatch("permute_seg", perm_segments(P, E) > 1 ? 2 : 1);
 }
-hipError_t launch_grouped_gate_up(const MoeDims&, const LayerDesc&, uint32_t, uint32_t, const uint4*, const uint32_t*,
+hipError_t launch_grouped_gate_up(const MoeDims&, const LayerDesc&, uint32_t, const UnitLists&, const uint32_t*,
                                   const uint16_t*, const uint16_t*, const float*, float*, hipStream_t)
 {
     return dispatch("grouped_gate_up");
 }
-hipError_t launch_grouped_down(const MoeDims&, const LayerDesc&, uint32_t, uint32_t, const uint4*, const uint32_t*,
+hipError_t launch_grouped_down(const MoeDims&, const LayerDesc&, uint32_t, const UnitLists&, const uint32_t*,
                                const uint16_t*, const uint16_t*, const float*, float* y, hipStream_t)
 {
     st().y = reinterpret_cast<uintptr_t>(y);

@@ -274,3 +274,69 @@ def test_permute_takes_one_workgroup_where_it_is_faster(bridge, E, K, in_one, in
         assert bridge.prefill(shape, T) == 0
         got = bridge.count("permutes") - one, bridge.count("permutes_seg") - seg
         assert got == ((1, 0) if T in in_one else (0, 1)), T
+
+
+def units_of(M, cap):
+    """Units of up to cap pairs: (number, of more than 16 rows)."""
+    n = -(-M // cap)
+    return int(n.sum()), int(n[M > 16].sum())
+
+
+def test_work_lists_hold_every_unit(built):
+    """Whatever the routing, each XCD's share of the long and of the short units fits the records of the list."""
+    lib, rng = C.CDLL(built), np.random.default_rng(3)
+    lib.fake_unit_records.restype = C.c_uint64
+    for case in range(4000):
+        E = int(rng.choice([1, 2, 7, 8, 16, 60, 128, 300, 512]))
+        P = int(np.exp(rng.uniform(0, np.log(65536))))
+        skew = rng.choice([0.0, 0.5, 1.0, 3.0])
+        p = (np.arange(E) + 1.0) ** -skew
+        M = rng.multinomial(P, rng.permutation(p) / p.sum())
+        if case % 3 == 0:       # as many units as P pairs can make: one pair over a whole number of units
+            M = np.zeros(E, np.int64)
+            e = min(E, P)
+            M[:e] = 1
+            left = (P - e) // 32
+            for k in range(min(left, 400)):
+                M[k % e] += 32
+        tiles = int(rng.choice([1, 2, 3, 5, 6, 8, 12, 16, 33, 64]))
+        P = int(M.sum())
+        u = {cap: units_of(M, cap) for cap in (32, 64)}
+        cap = lib.fake_unit_cap(P, u[64][0], u[32][0], tiles)
+        slots = lib.fake_unit_slots(P, E, tiles)
+        total, long_ = u[cap]
+        short = total - long_
+        share = [(x + 1) * long_ // 8 - x * long_ // 8 + (8 - x) * short // 8 - (7 - x) * short // 8 for x in range(8)]
+        assert sum(share) == total and max(share) <= slots // 8, (E, P, tiles, cap)
+        assert slots % 8 == 0 and 2 * slots <= lib.fake_unit_records(P, E)
+
+
+@pytest.mark.parametrize("cap,pairs,u64,u32,tiles", [
+    # measured points (kernel us with units of 64 / of 32)
+    (32, 514, 16, 23, 10),      # 44.5 / 41.2
+    (32, 600, 15, 23, 6),       # 36.7 / 26.8
+    (32, 400, 26, 31, 5),       # 22.9 / 17.4
+    (32, 600, 15, 23, 4),       # 27.4 / 20.3
+    (32, 300, 8, 14, 16),       # 25.9 / 23.3
+    (32, 800, 32, 33, 6),       # 32.6 / 29.1
+    (32, 512, 57, 62, 6),       # 43.3 / 39.2
+    (32, 512, 57, 62, 8),       # 21.1 / 20.6
+    (32, 2000, 45, 77, 6),      # 59.1 / 46.0
+    (64, 800, 32, 33, 8),       # 15.8 / 22.0
+    (64, 514, 16, 23, 12),      # 22.3 / 35.0
+    (64, 800, 16, 32, 10),      # 55.7 / 63.5
+    (64, 1400, 32, 51, 10),     # 78.7 / 91.8
+    (64, 3200, 68, 132, 7),     # 62.4 / 83.4
+    (64, 2400, 60, 113, 6),     # 37.7 / 45.3
+    (64, 1200, 32, 59, 6),      # 33.4 / 45.0
+    (64, 2000, 45, 77, 8),      # 26.3 / 30.6
+    (64, 1200, 23, 41, 6),      # 37.2 / 42.3
+    (64, 4096, 128, 188, 6),    # 77.0 / 103.5
+    (64, 1024, 77, 91, 6),      # 44.2 / 55.0
+    (64, 512, 79, 81, 12),      # 130.7 / 143.9
+    (64, 2028, 103, 127, 3),    # 22.4 / 25.3
+    (64, 704, 16, 24, 11),      # 21.0 / 28.2
+])
+def test_unit_length_takes_the_faster_cap(built, cap, pairs, u64, u32, tiles):
+    assert C.CDLL(built).fake_unit_cap(pairs, u64, u32, tiles) == cap
+

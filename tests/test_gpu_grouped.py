@@ -1,9 +1,10 @@
 """The grouped prefill GEMMs and the segmented permute at the edges of their
-units: work lists of units of up to 32 pairs (short lists: few experts, a narrow
-layer) and of up to 64 (test_units_of_48_and_64_rows), pair counts around every
-16-row tile, rows of one to several pairs of 64-column groups (with and without a
-remainder), an odd number of groups (the LDS-weight kernel), batches over several
-permute segments and over one pass.  Every result against fp64
+units: work lists of units of up to 32 pairs (few blocks) and of up to 64
+(test_units_of_48_and_64_rows), long units before short ones, pair counts around
+every 16-row tile, rows of one to several pairs of 64-column groups (with and
+without a remainder), small grids and odd numbers of groups (the LDS-weight kernel)
+and larger grids (the register kernel: more than 256 experts with a pair, or
+several row tiles), batches over several permute segments and over one pass.  Every result against fp64
 (moe_delta_f64_batch) and bit for bit against the same tokens in calls of 16."""
 import numpy as np
 import pytest
@@ -35,6 +36,9 @@ def prefill(ctx, layer, h, step):
     (1152, 4, 2, 896, (9, 70)),          # odd numbers of pairs of groups past the first ring of stages
     (256, 512, 8, 128, (300,)),          # segments of 16 chunks
     (256, 128, 8, 128, (257, 1000, 5000)),   # several segments, several passes
+    (128, 300, 4, 128, (290, 1100, 2400)),   # more than a block a CU: the register kernel, one stage
+    (384, 260, 4, 256, (1000, 2600)),        # three stages of gate/up, two of down
+    (640, 260, 2, 640, (3800,)),             # five of both
 ])
 def test_passes_and_segments(ctx, D, E, K, I, Ts):
     check(ctx, D, E, K, I, Ts)
@@ -63,27 +67,31 @@ def check(ctx, D, E, K, I, Ts):
     return all_ids
 
 
-def unit_rows(ids, E, I):
-    """Rows of the units of the work list that the permute of ids makes: an expert's M pairs in units of up
-    to 64 where that gives as many units as 512 gate/up blocks need, else of up to 32; equal numbers of
-    16-row tiles."""
+def unit_rows(ids, E, tiles):
+    """Rows of the units of the work list that the permute of ids makes for a launch of so many row tiles: an
+    expert's M pairs in units of up to 32 or 64 (unit_cap), in equal numbers of 16-row tiles."""
     M = np.bincount(ids.ravel(), minlength=E)
-    few = 512 // -(-I // 128)
-    cap = 64 if np.sum(-(-M // 64)) >= few else 32
-    n, tiles = -(-M // cap), -(-M // 16)
-    return {16 * -(-int(t) // int(k)) for t, k in zip(tiles, n) if k}
+    u64, u32 = np.sum(-(-M // 64)), np.sum(-(-M // 32))
+    b64, b32 = -(-u64 // 8) * tiles, -(-u32 // 8) * tiles
+    small = b32 <= 32 or (b64 > 32 and b32 <= 64 and (8 * u32 <= 9 * u64 or M.sum() >= 40 * u64))
+    cap = 32 if small else 64
+    n, m16 = -(-M // cap), -(-M // 16)
+    return {16 * -(-int(t) // int(k)) for t, k in zip(m16, n) if k}
 
 
 @pytest.mark.parametrize("D,E,K,I,Ts", [
-    (256, 32, 4, 2048, (300, 450, 640)),     # two stages of gate/up, sixteen of down
-    (1152, 36, 4, 1920, (380, 560)),         # odd numbers of stages
+    (256, 32, 4, 2048, (300, 450, 640)),     # two stages of gate/up
+    (1152, 36, 4, 1920, (380, 560)),         # odd numbers of stages, also of down
     (128, 64, 4, 1152, (660, 900)),          # one stage of gate/up
-    (320, 32, 4, 2112, (300, 450, 640)),     # odd numbers of groups: the LDS-weight kernel
+    (128, 300, 4, 128, (2900, 3900)),        # one stage of both
+    (1600, 32, 4, 2112, (300, 450, 640)),    # odd numbers of groups: the LDS-weight kernel
 ])
 def test_units_of_48_and_64_rows(ctx, D, E, K, I, Ts):
     """Wide layers with enough experts for units of up to 64 pairs: the 48- and the 64-row forms of both
     kernels give every pair the sums of the 16-row form."""
-    seen = set()
+    seen = [set(), set()]
     for ids in check(ctx, D, E, K, I, Ts):
-        seen |= unit_rows(ids, E, I)
-    assert {48, 64} <= seen, seen
+        for s, tiles in zip(seen, (-(-I // 128), -(-D // 256))):
+            s |= unit_rows(ids, E, tiles)
+    assert {48, 64} <= seen[0], seen
+    assert {48, 64} <= seen[1] or -(-D // 256) == 1 and E < 300, seen
