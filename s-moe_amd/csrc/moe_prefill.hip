@@ -24,7 +24,7 @@
 //                  block) on MFMA v_mfma_f32_16x16x32_f16, weights streamed into
 //                  registers, activation rows through LDS (k_grouped_mm, with
 //                  the weights through LDS too, where a row has an odd number
-//                  of groups).  Weights enter exactly as
+//                  of groups or the grid is small).  Weights enter exactly as
 //                  (2c - 15)/8 (f16), activations as hi and lo planes (two
 //                  MFMAs into one fp32 accumulator); each 64-column group adds
 //                  s_g * sum, the row scale 8 * 2^e / 15 closes the dot
@@ -863,8 +863,9 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
 // v_mfma_f32_16x16x32_f16 operand layout: lane l holds A[l % 16][8 (l/16) + j]
 // and B[8 (l/16) + j][l % 16] (j < 8) and receives D[4 (l/16) + i][l % 16].
 // Inside a 64-column group, lane quarter q = l/16 of MFMA step s uses the
-// physical columns 16 q + 8 s + j (both operands hold a lane's 8 columns in
-// the order 0 2 4 6 1 3 5 7).  Weights enter as f16 (2c - 15)/8 (exact), so
+// physical columns 32 s + 8 q + j (both operands hold a lane's 8 columns in
+// the order 0 2 4 6 1 3 5 7), as k_grouped_reg does: a pair's sums are the same
+// bits in either kernel.  Weights enter as f16 (2c - 15)/8 (exact), so
 // a group's MFMA sum times s_g is 15/60 of its dequantised dot product
 // (kernels.metal:90-105, 140-145) and the epilogue is one FMA per output.
 // LDS layouts (16-byte slots; XOR swizzles keep the fragment reads free of
@@ -982,16 +983,19 @@ __device__ __forceinline__ void grouped_mm_expert(
                                              16, 0, 0);
         __builtin_amdgcn_global_load_lds(s_src + min(gs, G - 1), SMOE_LDS_AS(&S.sc[wv * 64]), 2, 0, 0);
     };
-    // B fragment of this lane for group g of a stage: row m16, bytes 8 q .. 8 q + 7 of the group
-    uint32_t boff[2];
+    // B fragment of this lane for group g of a stage, step stp: row m16, unit 4 stp + q (4 bytes) of the group
+    uint32_t boff[2][2];
 #pragma unroll
-    for (int g = 0; g < 2; ++g) boff[g] = wv * 2048 + m16 * 64 + 16 * ((2 * g + (q >> 1)) ^ ((m16 >> 2) & 3)) + 8 * (q & 1);
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int stp = 0; stp < 2; ++stp)
+            boff[g][stp] = wv * 2048 + m16 * 64 + 16 * ((2 * g + stp) ^ ((m16 >> 2) & 3)) + 4 * q;
     // A fragment offsets of this lane inside an activation stage (m-tile ms adds 4096 bytes)
     uint32_t aoff[2][2];
 #pragma unroll
     for (int stp = 0; stp < 2; ++stp)
 #pragma unroll
-        for (int pl = 0; pl < 2; ++pl) aoff[stp][pl] = m16 * 256 + 16 * ((8 * pl + 2 * q + stp) ^ m16);
+        for (int pl = 0; pl < 2; ++pl) aoff[stp][pl] = m16 * 256 + 16 * ((8 * pl + 4 * stp + q) ^ m16);
 
     if (threadIdx.x < PASS) {
         const uint32_t p = sorted_pairs[base + min(threadIdx.x, M - 1)];
@@ -1051,9 +1055,9 @@ __device__ __forceinline__ void grouped_mm_expert(
         float sc[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const uint2 v = *reinterpret_cast<const uint2*>(&W.w[boff[g] + 1024 * j]);
-            b[j][0] = q4_codes_to_f16(v.x);
-            b[j][1] = q4_codes_to_f16(v.y);
+#pragma unroll
+            for (int stp = 0; stp < 2; ++stp)
+                b[j][stp] = q4_codes_to_f16(*reinterpret_cast<const uint32_t*>(&W.w[boff[g][stp] + 1024 * j]));
             sc[j] = f16_bits_to_f32(static_cast<uint16_t>(W.sc[wv * 64 + 32 * g + 16 * j + m16]));
         }
 #pragma unroll
@@ -1675,7 +1679,7 @@ static hipError_t launch_grouped(const MoeDims& d, const LayerDesc& L, uint32_t 
     const uint4* units = lists.units + (GATE_UP ? 0u : lists.slots[0]);
     const uint32_t nt = lists.tiles[GATE_UP ? 0 : 1];
     const dim3 grid(lists.slots[GATE_UP ? 0 : 1] * nt);
-    if (reg_supported(L, k_dim))
+    if (reg_supported(L, k_dim) && !lds_weights(P, d.E, nt))
         launch_kernel(k_grouped_reg<GATE_UP>, grid, dim3(GD_WAVES * WAVE), s, d, L, units, sorted_pairs, a_hi, a_lo,
                       a_scale, div, out, n_dim, k_dim, nt);
     else

@@ -78,6 +78,7 @@ uint32_t fake_unit_cap(uint32_t P, uint32_t u64, uint32_t u32, uint32_t tiles)
 }
 uint32_t fake_unit_slots(uint32_t P, uint32_t E, uint32_t tiles) { return smoe::unit_slots(smoe::max_units(P, E, tiles)); }
 uint64_t fake_unit_records(uint32_t P, uint32_t E) { return smoe::unit_records(P, E); }
+int fake_lds_weights(uint32_t P, uint32_t E, uint32_t tiles) { return smoe::lds_weights(P, E, tiles); }
 int fake_attn_wide(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t valid)
 {
     return smoe::attn_wide({head_dim, heads, kv_heads, kv_heads * head_dim, valid, 1.0f}, valid);
