@@ -347,16 +347,18 @@ constexpr uint32_t perm_segments(uint32_t P, uint32_t E)
 }
 hipError_t launch_permute_seg(const uint32_t* ids, uint32_t P, uint32_t E, uint32_t* sorted_pairs,
                               const UnitLists& lists, uint32_t* seg_cnt, uint32_t* err, hipStream_t s);
-// Whether a batch of several segments is permuted in one workgroup all the same (its
-// tables fit, and its threads keep all ids: 8 a thread).  One launch instead of
-// two; kernel times of one workgroup / both segment kernels at 128 experts x top-8:
-// 260 tokens 6.4 / 9.6 us, 512 7.8 / 9.5, 736 9.9 / 10.0; 32 x top-4, 700 tokens
-// 5.7 / 8.8; 8 x top-2, 4000 tokens 7.6 / 8.5; past that 60 x top-6, 1500 tokens
-// 11.5 / 9.9.  One segment is permuted by k_perm_scatter alone (4.1 to 5.0 us
-// against 4.3 to 5.4).
+// Whether a batch of several segments is permuted in one workgroup all the same:
+// one launch instead of two, but one CU's time for all the pairs.  Call times in
+// us of one workgroup / both segment kernels at 128 experts x top-8: 260 tokens
+// 134.7 / 135.8, 400 151.1 / 151.8, 512 160.2 / 160.2, 640 188.3 / 187.4, 736 215.1
+// / 213.2; 32 x top-4: 700 tokens 116.7 / 117.5, 1500 192.1 / 191.3; 8 x top-2:
+// 1500 52.0 / 53.1, 4000 86.8 / 85.6; 512 x top-8, 150 tokens 118.0 / 119.5.  (The
+// kernels' own times say more, 7.7 against 9.5 us at 512 tokens: the second of two
+// short launches hides part of the first one's.)  One segment is permuted by
+// k_perm_scatter alone.
 constexpr bool permute_in_one(uint32_t P, uint32_t E)
 {
-    return perm_segments(P, E) > 1 && P <= 8192 && permute_lds_bytes(P, E) <= PERMUTE_MAX_LDS;
+    return perm_segments(P, E) > 1 && P <= 4096 && permute_lds_bytes(P, E) <= PERMUTE_MAX_LDS;
 }
 // Grouped expert GEMMs over the permuted pairs (MFMA f16, hi/lo activations):
 // h [P x I] = silu(x G^T) * (x U^T); y [P x D] = h Dn^T, over the permute's

@@ -503,17 +503,18 @@ __device__ __forceinline__ uint32_t unit_pair(uint32_t M, uint32_t cap)
     return unit_count(M, cap) << (M > 16u ? 0u : 16u);
 }
 
-// One wave, eight experts a lane: exclusive scans of the E experts' totals s_tot
-// into s_off [E + 1] (pairs) and s_unit [2][E + 1] (units of up to 64, of up to 32
+// One wave, EPL experts a lane: exclusive scans of the E experts' totals s_tot into
+// s_off [E + 1] (pairs) and s_unit [2][E + 1] (units of up to 64, of up to 32
 // pairs), and the caps of the two work lists.
-__device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, const UnitLists& lists, uint32_t* s_off,
-                                           uint32_t* s_unit, uint32_t* s_cap)
+template <int EPL>
+__device__ __forceinline__ void scan_units_n(const uint32_t* s_tot, uint32_t E, const UnitLists& lists, uint32_t* s_off,
+                                             uint32_t* s_unit, uint32_t* s_cap)
 {
     const uint32_t lane = threadIdx.x & 63;
-    uint32_t tot[8], u64 = 0, u32 = 0, sum = 0;
+    uint32_t tot[EPL], u64 = 0, u32 = 0, sum = 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t e = 8 * lane + i;
+    for (int i = 0; i < EPL; ++i) {
+        const uint32_t e = EPL * lane + i;
         tot[i] = e < E ? s_tot[e] : 0u;
         sum += tot[i];
         u64 += unit_pair(tot[i], 64u);
@@ -528,12 +529,13 @@ __device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, co
     };
     const uint32_t i_tot = inclusive(sum), i64 = inclusive(u64), i32 = inclusive(u32);
     const uint32_t n64 = readlane_u32(i64, WAVE - 1), n32 = readlane_u32(i32, WAVE - 1);
+    const uint32_t P = readlane_u32(i_tot, WAVE - 1);
     // (the short units' counts start after all the long ones)
     uint32_t run = i_tot - sum, run64 = i64 - u64 + (n64 << 16), run32 = i32 - u32 + (n32 << 16);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t e = 8 * lane + i;
-        if (e <= E) {
+    for (int i = 0; i < EPL; ++i) {
+        const uint32_t e = EPL * lane + i;
+        if (e < E) {
             s_off[e] = run;
             s_unit[e] = run64;
             s_unit[E + 1 + e] = run32;
@@ -542,13 +544,21 @@ __device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, co
         run64 += unit_pair(tot[i], 64u);
         run32 += unit_pair(tot[i], 32u);
     }
-    if (lane == WAVE - 1) {   // (E = 512 is past the last lane's eight)
+    if (lane == WAVE - 1) {
         s_off[E] = run;
         s_unit[E] = run64;
         s_unit[2 * E + 1] = run32;
-        for (int i = 0; i < 2; ++i)
-            s_cap[i] = unit_cap(run, (n64 & 0xFFFFu) + (n64 >> 16), (n32 & 0xFFFFu) + (n32 >> 16), lists.tiles[i]);
     }
+    if (lane < 2)
+        s_cap[lane] = unit_cap(P, (n64 & 0xFFFFu) + (n64 >> 16), (n32 & 0xFFFFu) + (n32 >> 16),
+                               lane == 0 ? lists.tiles[0] : lists.tiles[1]);
+}
+__device__ __forceinline__ void scan_units(const uint32_t* s_tot, uint32_t E, const UnitLists& lists, uint32_t* s_off,
+                                           uint32_t* s_unit, uint32_t* s_cap)
+{
+    if (E <= 64) scan_units_n<1>(s_tot, E, lists, s_off, s_unit, s_cap);
+    else if (E <= 128) scan_units_n<2>(s_tot, E, lists, s_off, s_unit, s_cap);
+    else scan_units_n<8>(s_tot, E, lists, s_off, s_unit, s_cap);
 }
 
 // a workgroup writes the records of both lists (s_off, s_unit, s_cap: scan_units):

@@ -261,9 +261,9 @@ def test_attention_takes_the_faster_kernel(built, heads, kv_heads, head_dim, wid
 
 
 @pytest.mark.parametrize("E,K,in_one,in_segments", [
-    (128, 8, (257, 300, 512, 736), (64, 256, 737, 4096)),
-    (32, 4, (700, 2000), (512, 2049)),
-    (8, 2, (2000, 4000), (1000,)),
+    (128, 8, (257, 300, 512), (64, 256, 640, 736, 4096)),
+    (32, 4, (700, 1000), (512, 1500)),
+    (8, 2, (1500, 2000), (1000, 4000)),
     (512, 8, (150,), (128, 300)),
 ])
 def test_permute_takes_one_workgroup_where_it_is_faster(bridge, E, K, in_one, in_segments):
