@@ -423,10 +423,12 @@ bool timed(SmoeMetalCtx* ctx, uint32_t kind, const char* what, F&& launch)
 // when the queued copy has read the entry, so that is waited for here.
 void* end_dispatch(SmoeMetalCtx* ctx, SmoeMetalCtx::HostIn* in, bool launched)
 {
-    const uint64_t h = ++ctx->seq;
-    if (launched && hip_ok(ctx, hipEventRecord(ctx->ev[h % kEvents], ctx->stream), "hipEventRecord")) {
-        in->handle = h;
-        return reinterpret_cast<void*>(static_cast<uintptr_t>(h));
+    if (launched) {
+        const uint64_t h = ++ctx->seq;
+        if (hip_ok(ctx, hipEventRecord(ctx->ev[h % kEvents], ctx->stream), "hipEventRecord")) {
+            in->handle = h;
+            return reinterpret_cast<void*>(static_cast<uintptr_t>(h));
+        }
     }
     (void)hipStreamSynchronize(ctx->stream);
     return nullptr;

@@ -313,16 +313,16 @@ inline UnitLists unit_lists(const MoeDims& d, uint32_t P, uint4* units)
     return l;
 }
 // Whether a launch of the grouped GEMMs takes k_grouped_mm though k_grouped_reg could
-// run it: where its blocks are at most about one a CU, half of the waves that a CU
-// holds of k_grouped_reg would be missing.  The host knows the units only as
-// between the experts with a pair and one more for every 64 pairs.  Kernel times in
-// us, k_grouped_reg / k_grouped_mm: 16 experts, 10 tiles of 3072 columns, 64 tokens
-// 32.1 / 29.0; 8 experts, 4 and 16 tiles, 60 tokens (down) 21.9 / 20.8; one expert,
-// 6 tiles, 16 tokens 21.4 / 18.7; over one a CU 60 experts, 6 tiles 26.0 / 28.0.
+// run it: where its blocks are at most one a CU, half of the waves that a CU holds
+// of k_grouped_reg would be missing.  The host knows of the units that there is at
+// most one for every expert with a pair and one more for every 64 pairs.  Kernel
+// times in us, k_grouped_reg / k_grouped_mm: 16 experts, 10 tiles of 3072 columns, 64
+// tokens 32.1 / 29.0; 8 experts, 4 and 16 tiles, 60 tokens (down) 21.9 / 20.8; one
+// expert, 6 tiles, 16 tokens 21.4 / 18.7; over one a CU 60 experts, 6 tiles 26.0 /
+// 28.0, and 68 units of 64 pairs, 4 tiles 34.3 / 42.6.
 constexpr bool lds_weights(uint32_t P, uint32_t E, uint32_t tiles)
 {
-    const uint32_t experts = E < P ? E : P;
-    return experts * tiles <= 256 && (experts + P / 64) * tiles <= 320;
+    return ((E < P ? E : P) + P / 64) * tiles <= 256;
 }
 // what unit_lists takes at most
 constexpr size_t unit_records(uint32_t P, uint32_t E) { return 2 * size_t(unit_slots(P / 32 + (E < P ? E : P))); }

@@ -342,9 +342,9 @@ def test_unit_length_takes_the_faster_cap(built, cap, pairs, u64, u32, tiles):
 
 
 @pytest.mark.parametrize("pairs,experts,tiles,lds", [
-    (128, 16, 10, True), (300, 16, 10, True), (120, 8, 16, True), (16, 1, 6, True), (320, 32, 8, True), (128, 8, 2, True),
+    (128, 16, 10, True), (300, 16, 10, True), (120, 8, 16, True), (16, 1, 6, True), (400, 32, 6, True), (128, 8, 2, True),
     (222, 60, 6, False), (128, 128, 6, False), (900, 60, 5, False), (514, 16, 20, False), (1400, 32, 8, False),
-    (4000, 8, 6, False),
+    (4000, 8, 6, False), (4000, 16, 4, False), (8000, 8, 2, False), (1200, 8, 12, False),
 ])
 def test_grouped_launches_of_one_block_a_cu_take_the_lds_kernel(built, pairs, experts, tiles, lds):
     assert bool(C.CDLL(built).fake_lds_weights(pairs, experts, tiles)) == lds
