@@ -18,7 +18,7 @@
 //                  rank) pairs by expert, one workgroup per segment of pairs,
 //                  and the GEMMs' work lists (k_permute: one workgroup, with the
 //                  union order by first appearance, for callers that ask for
-//                  the permute's outputs).
+//                  the permute's outputs and for batches of a few segments).
 //   k_grouped_reg  per unit of up to 64 pairs of an expert: [pairs x K] x [K x
 //                  rows] tiles (128 gate + 128 up rows, or 256 down rows, per
 //                  block) on MFMA v_mfma_f32_16x16x32_f16, weights streamed into
@@ -852,7 +852,8 @@ void k_perm_scatter(const uint32_t* __restrict__ ids, uint32_t P, uint32_t E, co
 // (gate+up, SiLU fused) or 256 rows of down.  Block = 8 waves; wave w owns two
 // 16-row MFMA subtiles (gate and up rows 16w.., or down rows 32w.. and
 // 32w + 16..) and all m-tiles of the pass.  Serves rows with an odd number of
-// groups and weights that are not 16-byte aligned; others take k_grouped_reg.
+// groups, weights that are not 16-byte aligned, and grids of at most one block a
+// CU (lds_weights); others take k_grouped_reg.
 //
 // The k dimension streams through two rings in LDS, filled by direct
 // global->LDS loads (global_load_lds_dwordx4) so that nothing in flight holds
