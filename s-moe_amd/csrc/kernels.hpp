@@ -295,9 +295,22 @@ constexpr uint32_t max_units(uint32_t P, uint32_t E, uint32_t tiles)
     const uint32_t two = 64 / tiles * 8, m32 = u32 < two ? u32 : two;   // (units of 32: two blocks a CU at most)
     return u64 > m32 ? u64 : m32;
 }
-// records of a work list: eight XCDs' shares, each of an eighth of the long units
-// and an eighth of the short ones, both rounded up
-constexpr uint32_t unit_slots(uint32_t units) { return (units + 14u) / 8u * 8u; }
+// XCD x's share of a work list: consecutive long units, then consecutive short ones.
+// The XCDs with one short unit more follow those with one long unit more, so that no
+// share is over an eighth of the units rounded up.  A share one unit over that cost
+// 62 units of 12 tiles 86 us for 76.
+struct UnitShare {
+    uint32_t l0, nl;   // first long unit, number
+    uint32_t s0, ns;   // first short unit, number
+};
+__host__ __device__ constexpr UnitShare unit_share(uint32_t x, uint32_t n_long, uint32_t n_short)
+{
+    const uint32_t a = n_long & 7u, b = n_short & 7u, y = (x - a) & 7u;
+    return {x * (n_long >> 3) + (x < a ? x : a), (n_long >> 3) + (x < a ? 1u : 0u),
+            y * (n_short >> 3) + (y < b ? y : b), (n_short >> 3) + (y < b ? 1u : 0u)};
+}
+// records of a work list: the eight shares, each as long as the longest can be
+constexpr uint32_t unit_slots(uint32_t units) { return (units + 7u) / 8u * 8u; }
 struct UnitLists {
     uint4* units = nullptr;       // [slots[0] + slots[1]], null: none
     uint32_t tiles[2] = {1, 1};   // row tiles of gate/up and of down

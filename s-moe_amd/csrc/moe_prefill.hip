@@ -483,12 +483,12 @@ constexpr int PERM_THREADS = 1024;
 // ascending in either: what is left for the end of a launch is short (in the
 // order of the experts alone 32 Zipf-routed tokens of the 30B shape took 89 us
 // against 81, 200 of them 141 against 117, 150 tokens of 60 experts 80 against
-// 73).  XCD x takes the x-th eighth of the long ones and the (7 - x)-th of the
-// short ones (block id mod 8 is a block's XCD), so an expert's blocks run
-// together on one XCD and share its activation rows and, between its units, its
-// weights in the L2.  The record of the j-th unit of XCD x stands at 8 j + x, all
-// 8 slots of every j the grid covers are written (no pairs: no unit), and a record
-// holds all that a block needs: one scalar load, then the pairs and the weights.
+// 73).  An XCD takes consecutive long units and consecutive short ones (unit_share;
+// block id mod 8 is a block's XCD), so an expert's blocks run together on one XCD
+// and share its activation rows and, between its units, its weights in the L2.
+// The record of the j-th unit of XCD x stands at 8 j + x, all 8 slots of every j
+// the grid covers are written (no pairs: no unit), and a record holds all that a
+// block needs: one scalar load, then the pairs and the weights.
 //
 // The tables over the experts hold two counts a word: long units before the
 // expert's in the low half, short ones (after all the long ones) in the high half.
@@ -571,12 +571,11 @@ __device__ __forceinline__ void write_units(const uint32_t* s_off, const uint32_
         const uint32_t i = down ? k - lists.slots[0] : k, cap = s_cap[down ? 1 : 0];
         const uint32_t* tab = s_unit + (cap == 32u ? E + 1u : 0u);
         const uint32_t n_long = tab[E] & 0xFFFFu, n_short = (tab[E] >> 16) - n_long;
-        const uint32_t j = i >> 3, x = i & 7u, xs = 7u - x;
-        const uint32_t l0 = x * n_long / 8u, nl = (x + 1u) * n_long / 8u - l0;
-        const uint32_t s0 = xs * n_short / 8u, ns = (xs + 1u) * n_short / 8u - s0;
+        const uint32_t j = i >> 3;
+        const UnitShare xcd = unit_share(i & 7u, n_long, n_short);
         uint4 rec = make_uint4(0u, 0u, 0u, 0u);
-        if (j < nl + ns) {
-            const uint32_t sh = j < nl ? 0u : 16u, u = j < nl ? l0 + j : n_long + s0 + (j - nl);
+        if (j < xcd.nl + xcd.ns) {
+            const uint32_t sh = j < xcd.nl ? 0u : 16u, u = j < xcd.nl ? xcd.l0 + j : n_long + xcd.s0 + (j - xcd.nl);
             auto first = [&](uint32_t e) { return (tab[e] >> sh) & 0xFFFFu; };
             uint32_t e = 0, hi = E;              // the expert: first(e) <= u < first(e + 1)
             while (hi - e > 1) {

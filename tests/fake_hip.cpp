@@ -77,6 +77,11 @@ uint32_t fake_unit_cap(uint32_t P, uint32_t u64, uint32_t u32, uint32_t tiles)
     return smoe::unit_cap(P, u64, u32, tiles);
 }
 uint32_t fake_unit_slots(uint32_t P, uint32_t E, uint32_t tiles) { return smoe::unit_slots(smoe::max_units(P, E, tiles)); }
+void fake_unit_share(uint32_t x, uint32_t n_long, uint32_t n_short, uint32_t* out)
+{
+    const smoe::UnitShare u = smoe::unit_share(x, n_long, n_short);
+    out[0] = u.l0, out[1] = u.nl, out[2] = u.s0, out[3] = u.ns;
+}
 uint64_t fake_unit_records(uint32_t P, uint32_t E) { return smoe::unit_records(P, E); }
 int fake_lds_weights(uint32_t P, uint32_t E, uint32_t tiles) { return smoe::lds_weights(P, E, tiles); }
 int fake_attn_wide(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t valid)

@@ -282,6 +282,22 @@ def units_of(M, cap):
     return int(n.sum()), int(n[M > 16].sum())
 
 
+def shares(lib, n_long, n_short):
+    out = (C.c_uint32 * 4)()
+    return [(lib.fake_unit_share(x, n_long, n_short, out), tuple(out))[1] for x in range(8)]
+
+
+def test_work_list_shares(built):
+    """Every unit on one XCD, and no XCD with more than an eighth of them rounded up."""
+    lib = C.CDLL(built)
+    for n_long in range(35):
+        for n_short in range(35):
+            share = shares(lib, n_long, n_short)
+            assert sorted(u for l0, nl, _, _ in share for u in range(l0, l0 + nl)) == list(range(n_long))
+            assert sorted(u for _, _, s0, ns in share for u in range(s0, s0 + ns)) == list(range(n_short))
+            assert max(nl + ns for _, nl, _, ns in share) == -(-(n_long + n_short) // 8), (n_long, n_short)
+
+
 def test_work_lists_hold_every_unit(built):
     """Whatever the routing, each XCD's share of the long and of the short units fits the records of the list."""
     lib, rng = C.CDLL(built), np.random.default_rng(3)
@@ -306,8 +322,8 @@ def test_work_lists_hold_every_unit(built):
         slots = lib.fake_unit_slots(P, E, tiles)
         total, long_ = u[cap]
         short = total - long_
-        share = [(x + 1) * long_ // 8 - x * long_ // 8 + (8 - x) * short // 8 - (7 - x) * short // 8 for x in range(8)]
-        assert sum(share) == total and max(share) <= slots // 8, (E, P, tiles, cap)
+        share = shares(lib, long_, short)
+        assert max(nl + ns for _, nl, _, ns in share) <= slots // 8, (E, P, tiles, cap)
         assert slots % 8 == 0 and 2 * slots <= lib.fake_unit_records(P, E)
 
 
